@@ -304,6 +304,12 @@ double launch_bytes(const Launch& L, double es) {
         b += es * ((double)d.M * d.K + (double)d.K * d.N + (double)d.M * d.N * (d.beta != 0.0 ? 2 : 1));
       return b;
     }
+    case LK_THIN: {
+      double b = 0;
+      for (const FmThinDesc& d : L.tdescs)
+        b += es * ((double)d.M * d.K + (double)d.K * d.N + (double)d.M * d.N * (d.beta != 0.0 ? 2 : 1));
+      return b;
+    }
     case LK_SPLIT: {
       double b = 0;
       for (const FmSplitDesc& d : L.sdescs)

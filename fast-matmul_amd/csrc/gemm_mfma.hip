@@ -2,8 +2,7 @@
 //
 // One launch runs every product of a recursion level (the BFS form of the
 // reference's leaf dgemm calls, linalg/linalg.hpp:261-269 reached from
-// algorithms/strassen.hpp:385-388) plus any peeling products
-// (linalg/linalg.hpp:213-243).  Work-group w takes output tile w of the
+// algorithms/strassen.hpp:385-388).  Work-group w takes output tile w of the
 // concatenated tile list; products are found by division (uniform shapes) or
 // by binary search over tile_begin.
 //

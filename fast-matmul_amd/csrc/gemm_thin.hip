@@ -1,0 +1,224 @@
+// gemm_thin.hip -- dynamic-peeling products (linalg/linalg.hpp:201-244): the
+// rows, columns and K slices left over by a floor split into blocks.
+//
+// Each product is bound by memory: it reads the one large operand once (the
+// right strip of C reads A, the bottom strip B) or updates C once, at 2 to 14
+// flops an element, while its thin dimension (1 to FM_THIN_MAX) fills a
+// sixteenth of a matrix instruction.  On 64 x 64 matrix-core tiles a strip
+// had one work group per 64 rows walking all of K through LDS, 16 deep at a
+// time: a serial chain of loads and barriers, 0.25 us per unit of K whatever
+// the machine could stream.  Here K is spread over the lanes of a work group
+// (16 or 8 K segments in the right strip, 64 lanes in the bottom strip) with 8
+// (4) loads in flight per lane, and the segments' sums meet once at the end,
+// in a fixed order that depends on the product alone.
+// Measured on MI355X (peeling per multiply, before -> after):
+// smirnov333 one level 4799^3 FP64 1190 -> 250 us; grey333_23_152 two levels
+// 4009 x 2800 x 2489 FP64 630 -> 234 us; strassen 257 x 500 x 55 FP64
+// 41 -> 7 us.
+#include <hip/hip_runtime.h>
+
+#include <type_traits>
+
+#include "gemm_thin.hpp"
+#include "gmem.hpp"
+
+namespace {
+
+// Tiles.  Update of C: one row per lane, 16 columns.  Right strip: 128-byte
+// runs of rows (16 FP64, 32 FP32), the rest of the work group on K segments.
+// Bottom strip: 4 columns per wave, K over the wave's lanes, so each A value
+// a lane fetches (a cache line of its own) serves 4 columns.
+constexpr int UPD_COLS = 16;
+constexpr int BOT_COLS = 4, BOT_WAVES = FM_THIN_THREADS / 64;
+template <typename T>
+constexpr int strip_rows() {
+  return 128 / (int)sizeof(T);
+}
+
+template <typename T>
+__device__ __forceinline__ void put(fm_gptr<T> p, T alpha, T beta, T sum) {
+  T r = alpha * sum;
+  if (beta != T(0)) r += beta * *p;
+  *p = r;
+}
+
+template <typename T, int KT>
+__device__ __forceinline__ void thin_k(const FmThinDesc& d, int tm, int tn, fm_gptr<const T> A,
+                                       fm_gptr<const T> B, fm_gptr<T> C) {
+  const int i = tm * FM_THIN_THREADS + (int)threadIdx.x, j0 = tn * UPD_COLS;
+  if (i >= d.M) return;
+  const T alpha = (T)d.alpha, beta = (T)d.beta;
+  const int64_t ldb = d.b.ld, ldc = d.c.ld;
+  T a[KT];
+#pragma unroll
+  for (int q = 0; q < KT; ++q) a[q] = A[i + q * d.a.ld];
+  C += i;
+  // columns past N read column N - 1 again and are not stored: every load of
+  // the tile is in flight at once
+  T c[UPD_COLS];
+  if (beta != T(0)) {
+#pragma unroll
+    for (int u = 0; u < UPD_COLS; ++u) c[u] = C[(int64_t)min(j0 + u, d.N - 1) * ldc];
+  }
+#pragma unroll
+  for (int u = 0; u < UPD_COLS; ++u) {
+    const int j = j0 + u;
+    if (j >= d.N) break;
+    T s = T(0);
+#pragma unroll
+    for (int q = 0; q < KT; ++q) s += a[q] * B[q + (int64_t)j * ldb];
+    T r = alpha * s;
+    if (beta != T(0)) r += beta * c[u];
+    C[(int64_t)j * ldc] = r;
+  }
+}
+
+template <typename T, int NT>
+__device__ __forceinline__ void thin_n(const FmThinDesc& d, int tm, fm_gptr<const T> A,
+                                       fm_gptr<const T> B, fm_gptr<T> C, T* red) {
+  constexpr int TR = strip_rows<T>(), SEG = FM_THIN_THREADS / TR, U = 8;
+  const int r = threadIdx.x % TR, seg = threadIdx.x / TR;
+  const int i = tm * TR + r;
+  const int64_t lda = d.a.ld, ldb = d.b.ld;
+  const int K = d.K;
+  const fm_gptr<const T> Ai = A + min(i, d.M - 1);  // rows past M: row M - 1, not stored
+  T acc[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j) acc[j] = T(0);
+  for (int k0 = seg; k0 < K; k0 += U * SEG) {
+    T a[U], b[U][NT];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = min(k0 + u * SEG, K - 1);
+      a[u] = Ai[k * lda];
+#pragma unroll
+      for (int j = 0; j < NT; ++j) b[u][j] = B[k + j * ldb];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+        acc[j] = k0 + u * SEG < K ? fma(a[u], b[u][j], acc[j]) : acc[j];
+  }
+#pragma unroll
+  for (int j = 0; j < NT; ++j) red[(j * SEG + seg) * TR + r] = acc[j];
+  __syncthreads();
+  for (int e = threadIdx.x; e < NT * TR; e += FM_THIN_THREADS) {
+    const int j = e / TR, rr = e - j * TR;
+    if (tm * TR + rr >= d.M) continue;
+    T s = T(0);
+#pragma unroll
+    for (int q = 0; q < SEG; ++q) s += red[(j * SEG + q) * TR + rr];
+    put<T>(C + tm * TR + rr + j * d.c.ld, (T)d.alpha, (T)d.beta, s);
+  }
+}
+
+template <typename T, int MT>
+__device__ __forceinline__ void thin_m(const FmThinDesc& d, int tn, fm_gptr<const T> A,
+                                       fm_gptr<const T> B, fm_gptr<T> C) {
+  constexpr int U = 4;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int j0 = (tn * BOT_WAVES + wave) * BOT_COLS;
+  if (j0 >= d.N) return;
+  const int64_t lda = d.a.ld, ldb = d.b.ld;
+  const int K = d.K;
+  fm_gptr<const T> Bj[BOT_COLS];
+#pragma unroll
+  for (int c = 0; c < BOT_COLS; ++c) Bj[c] = B + (int64_t)min(j0 + c, d.N - 1) * ldb;
+  T acc[BOT_COLS][MT];
+#pragma unroll
+  for (int c = 0; c < BOT_COLS; ++c)
+#pragma unroll
+    for (int i = 0; i < MT; ++i) acc[c][i] = T(0);
+  for (int k0 = lane; k0 < K; k0 += U * 64) {
+    T a[U][MT], b[U][BOT_COLS];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = min(k0 + u * 64, K - 1);
+#pragma unroll
+      for (int c = 0; c < BOT_COLS; ++c) b[u][c] = Bj[c][k];
+#pragma unroll
+      for (int i = 0; i < MT; ++i) a[u][i] = A[i + k * lda];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int c = 0; c < BOT_COLS; ++c)
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+          acc[c][i] = k0 + u * 64 < K ? fma(a[u][i], b[u][c], acc[c][i]) : acc[c][i];
+  }
+  T mine = T(0);
+#pragma unroll
+  for (int c = 0; c < BOT_COLS; ++c)
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      T s = acc[c][i];
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+      if (lane == c * MT + i) mine = s;
+    }
+  const int c = lane / MT, i = lane - c * MT;
+  if (c < BOT_COLS && j0 + c < d.N)
+    put<T>(C + i + (int64_t)(j0 + c) * d.c.ld, (T)d.alpha, (T)d.beta, mine);
+}
+
+// f(std::integral_constant) for the thin dimension's value 1 .. FM_THIN_MAX
+template <int V, class F>
+__device__ __forceinline__ void thin_dispatch(int v, F&& f) {
+  if (v == V)
+    f(std::integral_constant<int, V>());
+  else if constexpr (V < FM_THIN_MAX)
+    thin_dispatch<V + 1>(v, f);
+}
+
+template <typename T>
+__global__ void __launch_bounds__(FM_THIN_THREADS) fm_thin_kernel(FmThinArgs args) {
+  __shared__ T red[FM_THIN_MAX * FM_THIN_THREADS];
+  const int t = blockIdx.x;
+  int g;
+  if (args.uniform) {
+    const int q = t >= args.t0[2] ? 2 : t >= args.t0[1] ? 1 : 0;
+    g = args.d0[q] + (t - args.t0[q]) / args.per[q];
+  } else {
+    int lo = 0, hi = args.ndesc - 1;
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (args.descs[mid].tile_begin <= t)
+        lo = mid;
+      else
+        hi = mid - 1;
+    }
+    g = lo;
+  }
+  const FmThinDesc d = args.descs[g];
+  const int local = t - d.tile_begin;
+  const int tn = local / d.tiles_m, tm = local - tn * d.tiles_m;
+  const fm_gptr<const T> A = fm_global(reinterpret_cast<const T*>(fm_base(args.bases, d.a.role)) + d.a.off);
+  const fm_gptr<const T> B = fm_global(reinterpret_cast<const T*>(fm_base(args.bases, d.b.role)) + d.b.off);
+  const fm_gptr<T> C = fm_global(reinterpret_cast<T*>(fm_base(args.bases, d.c.role)) + d.c.off);
+  if (d.kind == FM_THIN_K)
+    thin_dispatch<1>(d.K, [&](auto v) { thin_k<T, decltype(v)::value>(d, tm, tn, A, B, C); });
+  else if (d.kind == FM_THIN_N)
+    thin_dispatch<1>(d.N, [&](auto v) { thin_n<T, decltype(v)::value>(d, tm, A, B, C, red); });
+  else
+    thin_dispatch<1>(d.M, [&](auto v) { thin_m<T, decltype(v)::value>(d, tn, A, B, C); });
+}
+
+}  // namespace
+
+void fm_thin_tile(int dtype_f64, int kind, int* rows, int* cols) {
+  *rows = kind == FM_THIN_K   ? FM_THIN_THREADS
+          : kind == FM_THIN_N ? (dtype_f64 ? strip_rows<double>() : strip_rows<float>())
+                              : FM_THIN_MAX;
+  *cols = kind == FM_THIN_K ? UPD_COLS : kind == FM_THIN_N ? FM_THIN_MAX : BOT_COLS * BOT_WAVES;
+}
+
+hipError_t fm_thin_launch(int dtype_f64, const FmThinArgs& a, hipStream_t s) {
+  if (a.total_tiles <= 0) return hipSuccess;
+  if (dtype_f64)
+    hipLaunchKernelGGL(fm_thin_kernel<double>, dim3(a.total_tiles), dim3(FM_THIN_THREADS), 0, s, a);
+  else
+    hipLaunchKernelGGL(fm_thin_kernel<float>, dim3(a.total_tiles), dim3(FM_THIN_THREADS), 0, s, a);
+  return hipGetLastError();
+}

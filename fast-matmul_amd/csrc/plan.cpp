@@ -118,23 +118,70 @@ Launch stage_launch(fm_dtype dt, LaunchKind kind, const FmAlgDesc* alg, std::vec
 
 // Peeling products of one node (linalg/linalg.hpp:201-244).
 void peel_descs(const Node& nd, const Dims& D, int am, int ak, int an, double beta,
-                std::vector<FmGemmDesc>& out) {
+                std::vector<FmThinDesc>& out) {
   const int64_t erA = D.m % am, ecA = D.k % ak, ecB = D.n % an;
-  auto mk = [&](FmOp a, FmOp b, FmOp c, int64_t M, int64_t N, int64_t K, double bta) {
-    if (M > 0 && N > 0) out.push_back(gdesc(a, b, c, M, N, K, nd.mu, bta));
+  auto mk = [&](FmThinKind kind, FmOp a, FmOp b, FmOp c, int64_t M, int64_t N, int64_t K, double bta) {
+    if (M <= 0 || N <= 0) return;
+    FmThinDesc d;
+    memset(&d, 0, sizeof(d));
+    d.a = a;
+    d.b = b;
+    d.c = c;
+    d.M = (int32_t)M;
+    d.N = (int32_t)N;
+    d.K = (int32_t)K;
+    d.kind = kind;
+    d.alpha = nd.mu;
+    d.beta = bta;
+    out.push_back(d);
   };
   if (ecA > 0) {
     const int64_t row_dim = D.m - erA, col_dim = D.n - ecB, kk = D.k - ecA;
-    mk(op_sub(nd.a, 0, kk), op_sub(nd.b, kk, 0), nd.c, row_dim, col_dim, ecA, 1.0);
+    mk(FM_THIN_K, op_sub(nd.a, 0, kk), op_sub(nd.b, kk, 0), nd.c, row_dim, col_dim, ecA, 1.0);
   }
   if (ecB > 0) {
     const int64_t s = D.n - ecB;
-    mk(nd.a, op_sub(nd.b, 0, s), op_sub(nd.c, 0, s), D.m, ecB, D.k, beta);
+    mk(FM_THIN_N, nd.a, op_sub(nd.b, 0, s), op_sub(nd.c, 0, s), D.m, ecB, D.k, beta);
   }
   if (erA > 0) {
     const int64_t s = D.m - erA, nc = D.n - ecB;
-    mk(op_sub(nd.a, s, 0), nd.b, op_sub(nd.c, s, 0), erA, nc, D.k, beta);
+    mk(FM_THIN_M, op_sub(nd.a, s, 0), nd.b, op_sub(nd.c, s, 0), erA, nc, D.k, beta);
   }
+}
+
+// One launch of peeling products, ordered by kind.  The products of one
+// problem's level have one shape per kind, so a tile finds its product by
+// division; a batch's are found by a search over tile_begin.
+Launch thin_launch(std::vector<FmThinDesc> descs, fm_dtype dt) {
+  std::stable_sort(descs.begin(), descs.end(),
+                   [](const FmThinDesc& x, const FmThinDesc& y) { return x.kind < y.kind; });
+  Launch L;
+  L.kind = LK_THIN;
+  L.stage = FM_STAGE_PEEL;
+  L.th.uniform = 1;
+  int32_t t = 0;
+  size_t i = 0;
+  for (int kind = 0; kind < 3; ++kind) {
+    L.th.t0[kind] = t;
+    L.th.d0[kind] = (int32_t)i;
+    L.th.per[kind] = 1;
+    const size_t first = i;
+    for (; i < descs.size() && descs[i].kind == kind; ++i) {
+      FmThinDesc& d = descs[i];
+      int bm, bn;
+      fm_thin_tile(dt == FM_F64, kind, &bm, &bn);
+      d.tiles_m = (d.M + bm - 1) / bm;
+      d.tile_begin = t;
+      const int32_t per = d.tiles_m * ((d.N + bn - 1) / bn);
+      t += per;
+      L.th.per[kind] = per;
+      if (d.M != descs[first].M || d.N != descs[first].N) L.th.uniform = 0;
+    }
+  }
+  L.th.ndesc = (int32_t)descs.size();
+  L.th.total_tiles = t;
+  L.tdescs = std::move(descs);
+  return L;
 }
 
 Launch gemm_launch(std::vector<FmGemmDesc> descs, int cfg, int stage, fm_dtype dt) {
@@ -685,6 +732,8 @@ fm_status build_subplan(fm_dtype dt, const Problem& p, int64_t ws_base, SubPlan&
     return FM_OK;
   }
   const FmAlgDesc* alg = p.alg;
+  if (std::max(alg->m, std::max(alg->k, alg->n)) > FM_THIN_MAX + 1)
+    return set_err(FM_ERR_UNSUPPORTED, "block split finer than the peeling kernels take");
   const int L = p.steps;
   std::vector<Dims> dims(L + 1);
   dims[0] = {p.m, p.k, p.n};
@@ -868,7 +917,9 @@ namespace {
 // grid-stride loop; blocks of 2^31 elements or more are refused (only
 // reachable with matrices near the device's memory size).
 fm_status check_stage_size(const Launch& L) {
-  if (L.kind == LK_GEMM || L.kind == LK_OZAKI || L.kind == LK_SPLIT || L.kind == LK_NONE) return FM_OK;
+  if (L.kind == LK_GEMM || L.kind == LK_OZAKI || L.kind == LK_SPLIT || L.kind == LK_THIN ||
+      L.kind == LK_NONE)
+    return FM_OK;
   const bool two = L.kind == LK_S2 || L.kind == LK_T2 || L.kind == LK_W2;
   const int64_t elems = two ? (int64_t)L.st.rows2 * L.st.cols2 : (int64_t)L.st.rows * L.st.cols;
   if (elems >= (int64_t(1) << 31))
@@ -1042,7 +1093,7 @@ fm_status assemble(Plan& P, std::vector<SubPlan>& subs, int64_t ws_elems, int pe
   int maxd = 0;
   for (const SubPlan& s : subs) maxd = std::max(maxd, s.depth);
   for (int l = maxd - 1; l >= 0; --l) {
-    std::vector<FmGemmDesc> peel;
+    std::vector<FmThinDesc> peel;
     std::vector<Launch> wl;
     for (SubPlan& s : subs) {
       if (s.depth <= l) continue;
@@ -1061,9 +1112,8 @@ fm_status assemble(Plan& P, std::vector<SubPlan>& subs, int64_t ws_elems, int pe
     } else {
       for (Launch& L : wl) P.launches.push_back(std::move(L));
     }
-    // peeling products stay on the plain kernel in OZAKI mode (FP64) and
-    // take the split kernel in SPLIT_BF16 mode
-    if (!peel.empty()) P.launches.push_back(gemm_launch(std::move(peel), FM_TILE_64x64, FM_STAGE_PEEL, P.dtype));
+    // peeling products are sums in the data type in every leaf mode
+    if (!peel.empty()) P.launches.push_back(thin_launch(std::move(peel), P.dtype));
   }
   P.ws_bytes = wsb;
   return FM_OK;
@@ -1088,6 +1138,8 @@ void Plan::pack(std::vector<char>& buf) {
       L.dev_off = put(L.gdescs.data(), L.gdescs.size() * sizeof(FmGemmDesc));
     else if (L.kind == LK_OZAKI)
       L.dev_off = put(L.odescs.data(), L.odescs.size() * sizeof(FmOzakiDesc));
+    else if (L.kind == LK_THIN)
+      L.dev_off = put(L.tdescs.data(), L.tdescs.size() * sizeof(FmThinDesc));
     else if (L.kind == LK_SPLIT) {
       L.dev_off = put(L.sdescs.data(), L.sdescs.size() * sizeof(FmSplitDesc));
       L.dev_off2 = put(L.spreps.data(), L.spreps.size() * sizeof(FmSplitPrep));
@@ -1108,6 +1160,8 @@ void Plan::bind(void* dev) {
       L.gm.descs = reinterpret_cast<const FmGemmDesc*>(p);
     else if (L.kind == LK_OZAKI)
       L.oz.descs = reinterpret_cast<const FmOzakiDesc*>(p);
+    else if (L.kind == LK_THIN)
+      L.th.descs = reinterpret_cast<const FmThinDesc*>(p);
     else if (L.kind == LK_SPLIT) {
       L.sp.descs = reinterpret_cast<const FmSplitDesc*>(p);
       L.sp.preps = reinterpret_cast<const FmSplitPrep*>((char*)dev + L.dev_off2);
@@ -1222,6 +1276,10 @@ fm_status Plan::run(const void* A, const void* B, void* C, void* ws, hipStream_t
       } else {
         e = go(FM_PHASE_ALL);
       }
+    } else if (L.kind == LK_THIN) {
+      FmThinArgs t = L.th;
+      t.bases = bases;
+      e = fm_thin_launch(dtype == FM_F64, t, s);
     } else if (L.kind == LK_GEMM) {
       FmGemmArgs g = L.gm;
       g.bases = bases;

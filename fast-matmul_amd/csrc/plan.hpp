@@ -11,6 +11,7 @@
 #include "alg_desc.hpp"
 #include "gemm_mfma.hpp"
 #include "gemm_ozaki.hpp"
+#include "gemm_thin.hpp"
 
 namespace fmplan {
 
@@ -19,7 +20,7 @@ fm_status hip_err(hipError_t e, const char* what);
 const std::string& last_error();
 void clear_error();
 
-enum LaunchKind { LK_S, LK_T, LK_W, LK_GEMM, LK_OZAKI, LK_S2, LK_T2, LK_W2, LK_SPLIT, LK_NONE };
+enum LaunchKind { LK_S, LK_T, LK_W, LK_GEMM, LK_OZAKI, LK_S2, LK_T2, LK_W2, LK_SPLIT, LK_THIN, LK_NONE };
 
 // One kernel launch.  Descriptors stay on the host until Plan::upload packs
 // them into the plan's device buffer.
@@ -31,6 +32,7 @@ struct Launch {
   FmGemmArgs gm{};
   FmOzakiArgs oz{};
   FmSplitArgs sp{};
+  FmThinArgs th{};
   int cfg = 0;
   int vec_ok = 1;
   int planes = 0;  // LK_S2 / LK_T2 writing split-bf16 slice planes (byte offsets in st)
@@ -41,6 +43,7 @@ struct Launch {
   std::vector<FmOzakiDesc> odescs;
   std::vector<FmSplitDesc> sdescs;
   std::vector<FmSplitPrep> spreps;
+  std::vector<FmThinDesc> tdescs;
   size_t dev_off = 0, dev_off2 = 0;
 };
 
@@ -94,7 +97,7 @@ struct SubPlan {
   std::vector<Launch> pre;                          // S/T stages, level order
   std::vector<FmGemmDesc> leaves;                   // base-case products
   std::vector<Launch> w;                            // W stage of level l at w[l]
-  std::vector<std::vector<FmGemmDesc>> peels;       // peeling products of level l
+  std::vector<std::vector<FmThinDesc>> peels;       // peeling products of level l
   int depth = 0;
   int64_t ws_elems = 0;
   Dims leaf{0, 0, 0};

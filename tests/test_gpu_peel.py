@@ -1,0 +1,74 @@
+"""Dynamic-peeling products at the edges of their kernels' tiles: every
+remainder of every block split the algorithms have, in each dimension.
+
+A's rows and columns inside the block split are zero except where a peeling
+product reads them, so the recursion contributes exact zeros and, on integer
+data, every element of C is an exact integer: the comparison is bit for bit,
+whatever the order of the sums."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+SPLITS = {"strassen": (2, 2, 2), "classical333_27_81": (3, 3, 3), "grey424_26_206": (4, 2, 4),
+          "grey522_18_99": (5, 2, 2), "smirnov633_40_960": (6, 3, 3), "smirnov363_40_960": (3, 6, 3),
+          "smirnov336_40_960": (3, 3, 6)}
+
+
+def _check(fm, alg, m, k, n, dtype, alpha, beta, seed):
+    sm, sk, sn = SPLITS[alg]
+    rng = np.random.default_rng(seed)
+    A = rng.integers(-8, 9, (m, k)).astype(dtype)
+    B = rng.integers(-8, 9, (k, n)).astype(dtype)
+    C0 = rng.integers(-8, 9, (m, n)).astype(dtype)
+    A[:m - m % sm, :k - k % sk] = 0  # the core's products vanish
+    if n % sn:  # the right strip reads these columns of A: keep its product
+        want_r = alpha * (A.astype(np.float64) @ B[:, n - n % sn:].astype(np.float64))
+    want = alpha * (A.astype(np.float64) @ B.astype(np.float64)) + beta * C0.astype(np.float64)
+    dev = lambda x: fm.col_major(torch.from_numpy(np.asfortranarray(x)).to(DEV))  # noqa: E731
+    C = fm.fastmatmul(alg, dev(A), dev(B), dev(C0), 1, alpha=alpha, beta=beta).double().cpu().numpy()
+    assert np.array_equal(C, want), (alg, m, k, n, np.argwhere(C != want)[:4])
+    if n % sn:
+        got = C[:, n - n % sn:] - beta * C0[:, n - n % sn:]
+        assert np.array_equal(got, want_r)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("alg", sorted(SPLITS))
+def test_every_remainder(fm, alg, dtype):
+    sm, sk, sn = SPLITS[alg]
+    for r in range(1, max(SPLITS[alg])):
+        m, k, n = 48 * sm + r % sm, 40 * sk + r % sk, 24 * sn + r % sn
+        _check(fm, alg, m, k, n, dtype, 2.0, -3.0, r)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("shape", [
+    (3, 3, 3),            # single rows, columns and K
+    (17, 255, 31),        # one past a strip's row tile, one short of a segment round
+    (257, 1027, 65),      # one past the update's rows, a wave's K round and columns
+    (33, 129, 1031),      # many bottom-strip tiles
+    (1031, 65, 19),
+])
+def test_tile_edges(fm, shape, dtype):
+    for alpha, beta in [(1.0, 0.0), (-1.0, 2.0)]:
+        _check(fm, "strassen", *shape, dtype, alpha, beta, sum(shape))
+
+
+def test_peeling_in_a_batch_of_unequal_problems(fm):
+    """Products of several shapes in one launch (found by the search, not by
+    division), each equal to its own call bit for bit."""
+    rng = np.random.default_rng(9)
+    dev = lambda x: fm.col_major(torch.from_numpy(np.asfortranarray(x)).to(DEV))  # noqa: E731
+    probs, single = [], []
+    for alg, (m, k, n) in [("strassen", (131, 77, 95)), ("grey522_18_99", (204, 301, 65)),
+                           ("strassen", (64, 65, 64)), ("strassen", (66, 64, 131))]:
+        A, B, C0 = (dev(rng.random(s) * 2 - 1) for s in ((m, k), (k, n), (m, n)))
+        probs.append({"A": A, "B": B, "C": C0.clone(), "alg": alg, "num_steps": 1, "alpha": 1.5, "beta": 0.5})
+        single.append(fm.fastmatmul(alg, A, B, C0.clone(), 1, alpha=1.5, beta=0.5))
+    fm.Batch(probs, graph=False).run()
+    torch.cuda.synchronize()
+    for p, s in zip(probs, single):
+        assert torch.equal(p["C"], s)
