@@ -715,7 +715,7 @@ fm_status fm_set_ozaki_slices(int slices) {
 
 fm_status fm_set_gemm_tile(int cfg) {
   std::lock_guard<std::mutex> lock(fm_api_mutex());
-  if (cfg < -1 || cfg >= FM_TILE_NUM) return set_err(FM_ERR_INVALID_ARG, "unknown tile config");
+  if (cfg < -1 || cfg >= FM_TILE_OPTIONS) return set_err(FM_ERR_INVALID_ARG, "unknown tile config");
   g_defaults.gemm_tile = cfg;
   return FM_OK;
 }

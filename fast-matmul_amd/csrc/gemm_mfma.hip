@@ -17,6 +17,8 @@
 // columns, i.e. contiguous 128-byte runs of column-major C.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "gemm_mfma.hpp"
 #include "gmem.hpp"
 
@@ -63,15 +65,15 @@ __device__ __forceinline__ int fm_xcd_remap(int wg, int nwg) {
 // interleaves the next step's LDS reads with the current step's MFMAs
 // (one read, then two MFMAs) through scheduling-group barriers; PIPE == 3
 // is PIPE == 2 with the next slice's LDS stores and the slice after's
-// global loads spread over the K steps of the current slice (FULL and EVEN
+// global loads spread over the K steps of the current slice (FULL and ANY
 // launches; others run as PIPE == 2).  FULL: every product is a whole
 // number of tiles and K slices with 16-byte aligned columns (the launch
-// checks), so only the unpredicated 16-byte load path is compiled.  EVEN:
-// every product has M and K multiples of the vector width and aligned
-// columns, so every tile, edge tiles and a partial last K slice included,
-// takes 16-byte loads.
+// checks), so only the unpredicated 16-byte load path is compiled.  ANY:
+// products of any size, offset and leading dimension (M >= the vector
+// width, K >= BK, 32-bit tile spans: the launch checks) on the same
+// unconditional 16-byte loads; see the loop.
 template <typename T, int BM, int BN, int BK, int WM, int WN, int MINW = 1, int UNR = BK / 4,
-          int PIPE = 0, bool FULL = false, bool EVEN = false>
+          int PIPE = 0, bool FULL = false, bool ANY = false>
 __global__ void __launch_bounds__(64 * WM * WN, MINW) fm_gemm_kernel(FmGemmArgs args) {
   using Op = FmMfma<T>;
   using acc_t = typename Op::acc_t;
@@ -93,10 +95,11 @@ __global__ void __launch_bounds__(64 * WM * WN, MINW) fm_gemm_kernel(FmGemmArgs 
   static_assert(NT % BM == 0 && NT % BK == 0, "tile/thread mismatch");
   static_assert(A_PER * NT == BM * BK && B_PER * NT == BK * BN, "tile/thread mismatch");
   static_assert(TM >= 1 && TN >= 1 && BK % 4 == 0, "bad tile");
+  constexpr int MR = TM * TN >= TM + TN ? TM * TN / (TM + TN) : 1;  // MFMAs per LDS fragment read
   typedef T vec_t __attribute__((ext_vector_type(VL)));
-  // the spread loop (PIPE == 3 on FULL and EVEN launches); other PIPE == 3
+  // the spread loop (PIPE == 3 on FULL and ANY launches); other PIPE == 3
   // launches run the PIPE == 2 loop
-  constexpr bool SPREAD = PIPE == 3 && (FULL || EVEN);
+  constexpr bool SPREAD = PIPE == 3 && (FULL || ANY);
   constexpr int PIPE_EFF = PIPE == 3 ? 2 : PIPE;
   // Operand pointers: global address space (global loads, which the LDS
   // wait counter does not track) for FP32 and for the spread loop, which
@@ -167,7 +170,7 @@ __global__ void __launch_bounds__(64 * WM * WN, MINW) fm_gemm_kernel(FmGemmArgs 
   const bool d_aligned = d.a.off % VL == 0 && d.a.ld % VL == 0 && d.b.off % VL == 0 && d.b.ld % VL == 0;
   const bool edge_free = FULL || ((m0 + BM <= M) && (n0 + BN <= N));
   const bool interior =
-      FULL || EVEN || (CAN_VEC && args.vec && d_aligned && (m0 + BM <= M || M % VL == 0));
+      FULL || ANY || (CAN_VEC && args.vec && d_aligned && (m0 + BM <= M || M % VL == 0));
 
   // element-load coordinates
   const int a_row = tid % BM, a_k = tid / BM;
@@ -263,7 +266,7 @@ __global__ void __launch_bounds__(64 * WM * WN, MINW) fm_gemm_kernel(FmGemmArgs 
   // (FULL: K is a positive multiple of BK; the constant keeps a tile's
   // epilogue stores out of the next tile's main loop, where the compiler
   // would otherwise have to wait for every load and store in flight)
-  bool vec_stage = FULL || EVEN || (interior && BK <= K);
+  bool vec_stage = FULL || ANY || (interior && BK <= K);
   if constexpr (!SPREAD) {  // the spread loop stages its first slice by parts
     if (vec_stage) {
       gload_vec(0);
@@ -296,65 +299,119 @@ __global__ void __launch_bounds__(64 * WM * WN, MINW) fm_gemm_kernel(FmGemmArgs 
 #pragma unroll
         for (int j = 0; j < TN; ++j) acc[i][j] = Op::mma(bf[set][j], af[set][i], acc[i][j]);
     };
-    // Edge tiles and a partial last K slice (EVEN launches: K a multiple
-    // of the vector width, so a B vector's VL k lie wholly inside or
-    // outside): a vector outside the product loads from the product's first
-    // row, column or k instead, in bounds, so every lane loads
-    // unconditionally (no branch for the compiler's wait counts to merge
-    // over), and is zeroed when stored to LDS (zeroing it at the load would
-    // make the compiler wait for the load right there).
-    const bool a_ok = edge_free || av_in;
-    const fm_ptr<GM, const T> av_src = a_ok ? av_ptr : A + (int64_t)av_k * lda;
-    auto b_ok = [&](int i) { return edge_free || n0 + bv_col + i * BV_NSTEP < N; };
-    auto ak_ok = [&](int k0, int i) { return FULL || k0 + av_k + i * AV_KSTEP < K; };
-    auto bk_ok = [&](int k0) { return FULL || k0 + bv_k < K; };
-    // store part q of the slice at k0 (loaded by load_part(k0, q))
-    auto store_part = [&](int buf, int q, int k0) {
+    // ANY launches: every lane loads unconditionally and in bounds (no
+    // branch for the compiler's wait counts to merge over).
+    //  - Loads are 16 bytes at the alignment of an element, from a base that
+    //    is uniform over the work group and a 32-bit lane offset.
+    //  - Rows past M: a vector starts at row M - VL at the latest; the
+    //    epilogue knows which row a shifted LDS row is.  Columns past N
+    //    repeat column N - 1, and are not stored.
+    //  - The partial last K slice (kr deep; TAIL below): k past K read the
+    //    slice before, or, in B's vector that straddles K, the VL values
+    //    that end at K - 1 (elements move down by b_sh), and are zeroed in
+    //    both operands when stored to LDS.  The MFMA sequence is that of a
+    //    zero-padded slice.  Only the last three iterations, which load or
+    //    store it, carry this: with it in every iteration the 128 x 128
+    //    FP64 tile ran 8190 x 8190 x 4090 at 64.4 TFLOP/s, 70.0 without.
+    const int kr = K - (nk - 1) * BK;  // depth of the last slice
+    typedef T uvec_t __attribute__((ext_vector_type(VL))) __attribute__((aligned(sizeof(T))));
+    const int mb = min(m0, M - VL), a_row0 = min(m0 + av_row, M - VL);
+    const fm_ptr<GM, const T> a_base = A + mb, b_base = B + (int64_t)n0 * ldb;
+    const uint32_t a_off = (uint32_t)((a_row0 - mb) + (int64_t)av_k * lda) * (uint32_t)sizeof(T);
+    uint32_t b_off[BV_PER];
+#pragma unroll
+    for (int i = 0; i < BV_PER; ++i)
+      b_off[i] = (uint32_t)(bv_k + (int64_t)min(bv_col + i * BV_NSTEP, N - 1 - n0) * ldb) * (uint32_t)sizeof(T);
+    auto gld = [&](fm_ptr<GM, const T> p, uint32_t off) {
+      return *(fm_ptr<GM, const uvec_t>)((fm_ptr<GM, const char>)p + off);
+    };
+    // store part q of slice ks (loaded by load_part(ks, q))
+    auto store_part = [&](auto tail_c, int buf, int q, int ks) {
+      constexpr bool TAIL = decltype(tail_c)::value;
+      const bool tail = TAIL && ks >= nk - 1;
+      const int b_sh = bv_k < kr ? max(bv_k + VL - kr, 0) : 0;
 #pragma unroll
       for (int i = 0; i < AV_PER; ++i)
         if (i % NS4 == q) {
           vec_t v;
 #pragma unroll
           for (int e = 0; e < VL; ++e) v[e] = ra[i * VL + e];
-          if constexpr (!FULL) v = a_ok && ak_ok(k0, i) ? v : vec_t{};
+          if constexpr (TAIL)
+            if (tail && av_k + i * AV_KSTEP >= kr) v = vec_t{};
           *reinterpret_cast<vec_t*>(&As[buf][av_k + i * AV_KSTEP][av_row]) = v;
         }
 #pragma unroll
       for (int i = 0; i < BV_PER; ++i)
         if (i % NS4 == q) {
-          const bool ok = FULL || (b_ok(i) && bk_ok(k0));
+          if constexpr (TAIL) {
+            vec_t v;
 #pragma unroll
-          for (int e = 0; e < VL; ++e)
-            Bs[buf][bv_col + i * BV_NSTEP][bv_k + e] = ok ? rb[i * VL + e] : T(0);
+            for (int e = 0; e < VL; ++e) v[e] = rb[i * VL + e];
+#pragma unroll
+            for (int e = 0; e < VL; ++e) {
+              T t = v[e];
+#pragma unroll
+              for (int j = e + 1; j < VL; ++j) t = tail && b_sh == j - e ? (T)v[j] : t;
+              Bs[buf][bv_col + i * BV_NSTEP][bv_k + e] = tail && bv_k + e >= kr ? T(0) : t;
+            }
+          } else {
+#pragma unroll
+            for (int e = 0; e < VL; ++e) Bs[buf][bv_col + i * BV_NSTEP][bv_k + e] = rb[i * VL + e];
+          }
         }
     };
-    auto load_part = [&](int k0, int q) {
+    auto load_part = [&](auto tail_c, int ks, int q) {
+      constexpr bool TAIL = decltype(tail_c)::value;
+      if constexpr (FULL) {
+        const int k0 = ks * BK;
 #pragma unroll
-      for (int i = 0; i < AV_PER; ++i)
-        if (i % NS4 == q) {
-          const int64_t kc = ak_ok(k0, i) ? (int64_t)(k0 + i * AV_KSTEP) : -(int64_t)av_k;
-          const vec_t v = *(const fm_ptr<GM, const vec_t>)(av_src + kc * lda);
+        for (int i = 0; i < AV_PER; ++i)
+          if (i % NS4 == q) {
+            const vec_t v = *(const fm_ptr<GM, const vec_t>)(av_ptr + (int64_t)(k0 + i * AV_KSTEP) * lda);
 #pragma unroll
-          for (int e = 0; e < VL; ++e) ra[i * VL + e] = v[e];
-        }
+            for (int e = 0; e < VL; ++e) ra[i * VL + e] = v[e];
+          }
 #pragma unroll
-      for (int i = 0; i < BV_PER; ++i)
-        if (i % NS4 == q) {
-          const int64_t col = FULL || b_ok(i) ? (int64_t)(i * BV_NSTEP) : -(int64_t)(n0 + bv_col);
-          const int kr = bk_ok(k0) ? k0 : -bv_k;
-          const vec_t v = *(const fm_ptr<GM, const vec_t>)(bv_ptr + kr + col * ldb);
+        for (int i = 0; i < BV_PER; ++i)
+          if (i % NS4 == q) {
+            const vec_t v = *(const fm_ptr<GM, const vec_t>)(bv_ptr + k0 + (int64_t)(i * BV_NSTEP) * ldb);
 #pragma unroll
-          for (int e = 0; e < VL; ++e) rb[i * VL + e] = v[e];
-        }
+            for (int e = 0; e < VL; ++e) rb[i * VL + e] = v[e];
+          }
+      } else {
+        // the partial slice is addressed from one slice earlier
+        const bool tail = TAIL && ks == nk - 1;
+        const int k0 = (tail ? ks - 1 : ks) * BK;
+        const uint32_t bk_lda = (uint32_t)(BK * lda) * (uint32_t)sizeof(T);
+        const int b_sh = max(bv_k + VL - kr, 0);
+        const uint32_t b_tail = tail && bv_k < kr ? (uint32_t)(BK - b_sh) * (uint32_t)sizeof(T) : 0u;
+#pragma unroll
+        for (int i = 0; i < AV_PER; ++i)
+          if (i % NS4 == q) {
+            const uint32_t t = tail && av_k + i * AV_KSTEP < kr ? bk_lda : 0u;
+            const uvec_t v = gld(a_base + (int64_t)(k0 + i * AV_KSTEP) * lda, a_off + t);
+#pragma unroll
+            for (int e = 0; e < VL; ++e) ra[i * VL + e] = v[e];
+          }
+#pragma unroll
+        for (int i = 0; i < BV_PER; ++i)
+          if (i % NS4 == q) {
+            const uvec_t v = gld(b_base + k0, b_off[i] + b_tail);
+#pragma unroll
+            for (int e = 0; e < VL; ++e) rb[i * VL + e] = v[e];
+          }
+      }
     };
+    const std::integral_constant<bool, false> body;
+    const std::integral_constant<bool, !FULL> last;  // iterations that may meet the partial slice
     // first slice
 #pragma unroll
     for (int q = 0; q < NS4; ++q) {
-      load_part(0, q);
+      load_part(body, 0, q);
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
-    for (int q = 0; q < NS4; ++q) store_part(0, q, 0);
+    for (int q = 0; q < NS4; ++q) store_part(body, 0, q, 0);
     __syncthreads();
     // The stores and loads run unconditionally (the last slices store into
     // a buffer no one reads again and reload slice nk - 1, in bounds):
@@ -365,34 +422,44 @@ __global__ void __launch_bounds__(64 * WM * WN, MINW) fm_gemm_kernel(FmGemmArgs 
     // alike)
 #pragma unroll
     for (int q = 0; q < NS4; ++q) {
-      load_part(min(1, nk - 1) * BK, q);
+      load_part(last, min(1, nk - 1), q);
       __builtin_amdgcn_sched_barrier(0);
     }
     frag(0, 0, 0);
-    for (int kt = 0; kt < nk; ++kt) {
-      const int cur = kt & 1;
-      const int kl = min(kt + 2, nk - 1) * BK;
-#pragma unroll
-      for (int q = 0; q < NS4; ++q) {
-        store_part(cur ^ 1, q, (kt + 1) * BK);
-        load_part(kl, q);
-        __builtin_amdgcn_sched_barrier(0);
-        if (q < NS4 - 1) {
-          frag(cur, q + 1, (q + 1) & 1);
-          mma_step(q & 1);
-#pragma unroll
-          for (int r = 0; r < TM + TN; ++r) {
-            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one LDS read
-            __builtin_amdgcn_sched_group_barrier(0x008, (TM * TN) / (TM + TN), 0);  // MFMAs
-          }
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      }
-      __syncthreads();
-      frag(cur ^ 1, 0, NS4 & 1);
-      __builtin_amdgcn_sched_barrier(0);
-      mma_step((NS4 - 1) & 1);
+// One iteration of the spread loop.  A macro: written as a lambda (inlined all
+// the same) the compiler allots the registers differently and the 128 x 128
+// FP64 tile loses 2.5% (72.1 -> 70.2 TFLOP/s at 8192 x 8192 x 4096).
+#define FM_SPREAD_ITERATION(TAIL_C, KT)                                                    \
+  {                                                                                        \
+    const int cur = (KT) & 1;                                                              \
+    const int kl = min((KT) + 2, nk - 1);                                                  \
+    _Pragma("unroll") for (int q = 0; q < NS4; ++q) {                                      \
+      store_part(TAIL_C, cur ^ 1, q, (KT) + 1);                                            \
+      load_part(TAIL_C, kl, q);                                                            \
+      __builtin_amdgcn_sched_barrier(0);                                                   \
+      if (q < NS4 - 1) {                                                                   \
+        frag(cur, q + 1, (q + 1) & 1);                                                     \
+        mma_step(q & 1);                                                                   \
+        _Pragma("unroll") for (int r = 0; r < TM + TN; ++r) {                              \
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  /* one LDS read */           \
+          __builtin_amdgcn_sched_group_barrier(0x008, MR, 0); /* MFMAs */                  \
+        }                                                                                  \
+        __builtin_amdgcn_sched_barrier(0);                                                 \
+      }                                                                                    \
+    }                                                                                      \
+    __syncthreads();                                                                       \
+    frag(cur ^ 1, 0, NS4 & 1);                                                             \
+    __builtin_amdgcn_sched_barrier(0);                                                     \
+    mma_step((NS4 - 1) & 1);                                                               \
+  }
+    if constexpr (FULL) {
+      for (int kt = 0; kt < nk; ++kt) FM_SPREAD_ITERATION(body, kt)
+    } else {
+      const int kb = kr < BK ? max(nk - 3, 0) : nk;
+      for (int kt = 0; kt < kb; ++kt) FM_SPREAD_ITERATION(body, kt)
+      for (int kt = kb; kt < nk; ++kt) FM_SPREAD_ITERATION(last, kt)
     }
+#undef FM_SPREAD_ITERATION
   } else if constexpr (PIPE_EFF) {
     // Fragments of K step s + 1 are read from LDS before the MFMAs of step s
     // (two register sets), and the MFMAs of a slice's last step are issued
@@ -431,7 +498,7 @@ __global__ void __launch_bounds__(64 * WM * WN, MINW) fm_gemm_kernel(FmGemmArgs 
 #pragma unroll
           for (int r = 0; r < TM + TN; ++r) {
             __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one LDS read
-            __builtin_amdgcn_sched_group_barrier(0x008, (TM * TN) / (TM + TN), 0);  // MFMAs
+            __builtin_amdgcn_sched_group_barrier(0x008, MR, 0);  // MFMAs
           }
           __builtin_amdgcn_sched_barrier(0);
         }
@@ -490,7 +557,14 @@ __global__ void __launch_bounds__(64 * WM * WN, MINW) fm_gemm_kernel(FmGemmArgs 
   const T alpha = (T)d.alpha, beta = (T)d.beta;
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
-    const int row = m0 + wm * WTM + i * 16 + (lane & 15);
+    int row = m0 + wm * WTM + i * 16 + (lane & 15);
+    if constexpr (SPREAD && !FULL) {
+      // rows of the vector that straddles M were loaded sh rows earlier: the
+      // first sh of them are also the vector before's, and not stored here
+      const int v0 = row & ~(VL - 1), sh = max(v0 + VL - M, 0);
+      row -= sh;
+      if (row < v0) continue;
+    }
     if (row >= M) continue;
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
@@ -524,7 +598,7 @@ static void fm_gemm_go(const FmGemmArgs& a, hipStream_t s) {
       return;
     }
     if constexpr (PIPE == 3) {
-      if (a.even && a.vec) {
+      if (a.any) {
         hipLaunchKernelGGL((fm_gemm_kernel<T, BM, BN, BK, WM, WN, MINW, UNR, PIPE, false, true>),
                            dim3(grid), dim3(NT), 0, s, a);
         return;
@@ -540,9 +614,9 @@ static hipError_t fm_gemm_launch(int cfg, const FmGemmArgs& a, hipStream_t s) {
   if (a.total_tiles <= 0) return hipSuccess;
   switch (cfg) {
     case FM_TILE_128x128: fm_gemm_go<T, 128, 128, 16, 2, 2>(a, s); break;
-    case FM_TILE_64x64: fm_gemm_go<T, 64, 64, 16, 2, 2>(a, s); break;
-    case FM_TILE_128x64: fm_gemm_go<T, 128, 64, 16, 2, 2>(a, s); break;
-    case FM_TILE_64x128: fm_gemm_go<T, 64, 128, 16, 2, 2>(a, s); break;
+    case FM_TILE_64x64: fm_gemm_go<T, 64, 64, 16, 2, 2, 4, 4, 3>(a, s); break;
+    case FM_TILE_128x64: fm_gemm_go<T, 128, 64, 16, 2, 2, 3, 4, 3>(a, s); break;
+    case FM_TILE_64x128: fm_gemm_go<T, 64, 128, 16, 2, 2, 3, 4, 3>(a, s); break;
     case FM_TILE_128x128_K32: fm_gemm_go<T, 128, 128, 32, 2, 2>(a, s); break;
     case FM_TILE_128x128_W8: fm_gemm_go<T, 128, 128, 16, 2, 4>(a, s); break;
     case FM_TILE_128x128_K32_W8: fm_gemm_go<T, 128, 128, 32, 2, 4>(a, s); break;
@@ -565,8 +639,9 @@ static hipError_t fm_gemm_launch(int cfg, const FmGemmArgs& a, hipStream_t s) {
     case FM_TILE_PI_128x256_W8: fm_gemm_go<T, 128, 256, 16, 2, 4, 1, 4, 2>(a, s); break;
     case FM_TILE_PI_128x96_O2: fm_gemm_go<T, 128, 96, 16, 2, 2, 2, 4, 2>(a, s); break;
     case FM_TILE_PS_128x128_O2: fm_gemm_go<T, 128, 128, 16, 2, 2, 2, 4, 3>(a, s); break;
-    case FM_TILE_PS_128x256_W8: fm_gemm_go<T, 128, 256, 16, 2, 4, 1, 4, 3>(a, s); break;
+    case FM_TILE_PS_128x256_W8: fm_gemm_go<T, 128, 256, 16, 2, 4, sizeof(T) == 4 ? 4 : 1, 4, 3>(a, s); break;
     case FM_TILE_PS_128x96_O2: fm_gemm_go<T, 128, 96, 16, 2, 2, 2, 4, 3>(a, s); break;
+    case FM_TILE_PS_32x32_K32: fm_gemm_go<T, 32, 32, 32, 2, 2, 4, 8, 3>(a, s); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();

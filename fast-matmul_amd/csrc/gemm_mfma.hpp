@@ -27,17 +27,18 @@ struct FmGemmArgs {
                     // products whose own offsets and leading dimensions keep columns aligned
   int32_t grid;     // > 0: persistent launch with this many work groups
   int32_t full;     // every product is a whole number of tiles and K slices
-  int32_t even;     // every product has M and K multiples of the vector width and
-                    // 16-byte aligned columns (edge tiles and a partial last K slice)
+  int32_t any;      // every product fits the spread kernels' ANY variant: M at least the
+                    // vector width, K at least the slice depth, and a tile's columns
+                    // within 32-bit byte offsets
 };
 
 // Tile configurations of the leaf kernel: BM x BN output tile, BK-deep K
 // slices, WM x WN waves (64 * WM * WN threads).
 enum FmTileCfg : int {
   FM_TILE_128x128 = 0,         // BK 16, 2x2 waves
-  FM_TILE_64x64 = 1,           // BK 16, 2x2 waves
-  FM_TILE_128x64 = 2,          // BK 16, 2x2 waves
-  FM_TILE_64x128 = 3,          // BK 16, 2x2 waves
+  FM_TILE_64x64 = 1,           // BK 16, 2x2 waves, spread (see 32)
+  FM_TILE_128x64 = 2,          // BK 16, 2x2 waves, spread
+  FM_TILE_64x128 = 3,          // BK 16, 2x2 waves, spread
   FM_TILE_128x128_K32 = 4,     // BK 32, 2x2 waves
   FM_TILE_128x128_W8 = 5,      // BK 16, 2x4 waves
   FM_TILE_128x128_K32_W8 = 6,  // BK 32, 2x4 waves
@@ -74,13 +75,21 @@ enum FmTileCfg : int {
   // split-bf16 on slice planes, B fragments loaded straight into registers
   FM_TILE_SP_128x256_BD = 31,  // 2x4 waves, A through double-buffered LDS
   // as 22 and 23, with the next slice's LDS stores and global loads spread
-  // over the K steps (edge launches too, on products whose M and K are
-  // multiples of the vector width and whose columns are 16-byte aligned)
+  // over the K steps
   FM_TILE_PS_128x128_O2 = 32,
   FM_TILE_PS_128x256_W8 = 33,
   FM_TILE_PS_128x96_O2 = 34,   // as 30, spread
-  FM_TILE_NUM = 35
+  FM_TILE_OPTIONS = 35,        // configurations the tile option names: 0 .. 34
+  // chosen by the plan only: launches too small for a larger tile to fill the chip
+  FM_TILE_PS_32x32_K32 = 35,   // BK 32, 2x2 waves of 16 x 16, spread
+  FM_TILE_NUM = 36
 };
+
+// configurations on the spread loop, which also takes ragged products (ANY)
+inline bool fm_tile_spread(int cfg) {
+  return (cfg >= FM_TILE_64x64 && cfg <= FM_TILE_64x128) ||
+         (cfg >= FM_TILE_PS_128x128_O2 && cfg <= FM_TILE_PS_32x32_K32);
+}
 
 // configurations that run on prepared slice planes
 inline bool fm_tile_planes(int cfg) {
@@ -90,7 +99,7 @@ inline bool fm_tile_planes(int cfg) {
 // K slice depth of each configuration
 inline int fm_tile_bk(int cfg) {
   return (cfg == FM_TILE_128x128_K32 || cfg == FM_TILE_128x128_K32_W8 || cfg == FM_TILE_64x64_K32 ||
-          fm_tile_planes(cfg))
+          cfg == FM_TILE_PS_32x32_K32 || fm_tile_planes(cfg))
              ? 32
              : 16;
 }
@@ -105,7 +114,7 @@ inline void fm_tile_dims(int cfg, int* bm, int* bn) {
                                         {128, 128}, {128, 128}, {128, 128}, {128, 256},
                                         {128, 128}, {256, 128}, {128, 256}, {128, 128},
                                         {256, 128}, {128, 256}, {128, 96},  {128, 256},
-                                        {128, 128}, {128, 256}, {128, 96}};
+                                        {128, 128}, {128, 256}, {128, 96}, {32, 32}};
   *bm = d[cfg][0];
   *bn = d[cfg][1];
 }

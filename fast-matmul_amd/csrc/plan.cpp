@@ -184,6 +184,34 @@ Launch thin_launch(std::vector<FmThinDesc> descs, fm_dtype dt) {
   return L;
 }
 
+// Every product a whole number of tiles and K slices, columns 16-byte aligned.
+bool whole_tiles(fm_dtype dt, int cfg, const std::vector<FmGemmDesc>& prods) {
+  if (fm_tile_planes(cfg)) return true;
+  int bm, bn;
+  fm_tile_dims(cfg, &bm, &bn);
+  const int bk = fm_tile_bk(cfg), vl = dt == FM_F64 ? 2 : 4;
+  for (const FmGemmDesc& d : prods)
+    if (d.M % bm || d.N % bn || d.K % bk || d.K == 0 || d.a.off % vl || d.a.ld % vl ||
+        d.b.off % vl || d.b.ld % vl)
+      return false;
+  return true;
+}
+
+// Every product fits the spread kernels' ANY variant: a 16-byte vector of
+// rows and a whole K slice exist to load from, and the byte offsets of a
+// tile's columns (two slices of A, the tile's columns of B) stay within 32
+// bits.
+bool any_tiles(fm_dtype dt, int cfg, const std::vector<FmGemmDesc>& prods) {
+  if (!fm_tile_spread(cfg)) return false;
+  int bm, bn;
+  fm_tile_dims(cfg, &bm, &bn);
+  const int64_t bk = fm_tile_bk(cfg), vl = dt == FM_F64 ? 2 : 4;
+  const int64_t span = (int64_t(1) << 32) / elem_size(dt);
+  for (const FmGemmDesc& d : prods)
+    if (d.M < vl || d.K < bk || bm + 2 * bk * d.a.ld >= span || 2 * bk + bn * d.b.ld >= span) return false;
+  return true;
+}
+
 Launch gemm_launch(std::vector<FmGemmDesc> descs, int cfg, int stage, fm_dtype dt) {
   int bm, bn;
   fm_tile_dims(cfg, &bm, &bn);
@@ -202,21 +230,12 @@ Launch gemm_launch(std::vector<FmGemmDesc> descs, int cfg, int stage, fm_dtype d
   L.gm.ndesc = (int32_t)descs.size();
   L.gm.total_tiles = t;
   L.gm.uniform = uniform ? 1 : 0;
-  // 16-byte loads need A/B column starts aligned: even (FP64) or
-  // multiple-of-4 (FP32) offsets and leading dimensions.  The kernels check
-  // each product's own; the base pointers are checked at launch.  The
-  // unpredicated whole-tile kernel needs every product whole and aligned.
-  const int vl = dt == FM_F64 ? 2 : 4;
-  const int bk = fm_tile_bk(cfg);
-  bool vec = true, full = true, even = true;
-  for (const FmGemmDesc& d : descs) {
-    vec = vec && d.a.off % vl == 0 && d.a.ld % vl == 0 && d.b.off % vl == 0 && d.b.ld % vl == 0;
-    full = full && d.M % bm == 0 && d.N % bn == 0 && d.K % bk == 0 && d.K > 0;
-    even = even && d.M % vl == 0 && d.K % vl == 0 && d.K > 0;
-  }
+  // The unpredicated whole-tile kernel needs every product whole and its
+  // A/B column starts 16-byte aligned (the base pointers are checked at
+  // launch); the spread kernels' ANY variant takes the others.
   L.vec_ok = 1;
-  L.gm.full = (full && vec) ? 1 : 0;
-  L.gm.even = (even && vec) ? 1 : 0;
+  L.gm.full = whole_tiles(dt, cfg, descs) ? 1 : 0;
+  L.gm.any = any_tiles(dt, cfg, descs) ? 1 : 0;
   L.cfg = cfg;
   L.gdescs = std::move(descs);
   return L;
@@ -350,7 +369,7 @@ Launch split_launch(std::vector<FmGemmDesc> prods, int cfg, size_t* ws_bytes) {
 fm_options g_defaults = {-1, 0, 0, 1, 1, 8};
 
 fm_status check_options(const fm_options& o) {
-  if (o.gemm_tile < -1 || o.gemm_tile >= FM_TILE_NUM) return set_err(FM_ERR_INVALID_ARG, "unknown tile config");
+  if (o.gemm_tile < -1 || o.gemm_tile >= FM_TILE_OPTIONS) return set_err(FM_ERR_INVALID_ARG, "unknown tile config");
   if (o.dfs_levels < -1) return set_err(FM_ERR_INVALID_ARG, "dfs_levels must be >= -1");
   if (o.stage_fusion < 0 || o.stage_fusion > 2)
     return set_err(FM_ERR_INVALID_ARG, "stage_fusion must be 0, 1 or 2");
@@ -373,228 +392,205 @@ int64_t align_up(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
 double round_scalar(double v, fm_dtype dt) { return dt == FM_F32 ? (double)(float)v : v; }
 int elem_size(fm_dtype dt) { return dt == FM_F64 ? 8 : 4; }
 
-// Tile of a grouped launch: smallest estimated time over the configurations,
-// where a configuration's throughput per tile (eff, measured on MI355X at
-// 8192^3) and its resident work groups per CU set how many rounds of tiles
-// the launch takes.
+// Tile of a grouped launch: smallest estimated time over the configurations.
 namespace {
-// A tile shape with the kernel used when every product of the launch is a
-// whole number of tiles and K slices with 16-byte aligned columns
-// (cfg_full), and the kernel for launches with edges (cfg_edge; -1: the
-// shape is not offered, its edge kernel spills registers).
+// Plain leaves: what one tile of a configuration costs a CU, in us on MI355X,
+// measured on launches of 1 to 16 tiles per CU at K = 256 and 1024: us_k per
+// unit of K and k0 units of K for its start and end, whether the CU holds one
+// work group or several; and lat_k, the same for a tile that has its CU to
+// itself and waits for its own loads (the small tiles).  Whole-tile and ragged
+// products cost the same on these kernels (FP64 128 x 128: 8192 x 8192 x 4096
+// 71.7 TFLOP/s, 8190 x 8190 x 4090 70.0, 8191 x 8191 x 4091 69.7).
 struct TileCand {
-  int cfg_full, cfg_edge;
-  double eff;           // throughput per tile area, relative
-  int per_cu;           // resident work groups per CU
-  bool spread = false;  // cfg_full also takes edge tiles when every product has whole K
-                        // slices and aligned columns (its EVEN variant)
+  int cfg;
+  double us_k, k0, lat_k;
 };
-// Relative throughput: whole-tile rates on MI355X (8192^3 and the 676-leaf
-// product of 512 x 2048 x 512), best = 1.  Work groups per CU: the lesser of
-// what the register allocation (waves per SIMD x 4 / waves per group) and
-// the 160 KB of LDS allow.
-// (8192^3: FP64 72.6 TFLOP/s with the spread 128 x 128 tile, 69.0 with
-// the same tile loading each slice at once; FP32 141.9 with the spread
-// 128 x 256 tile, 136 with the 256 x 256 one)
 const TileCand kF64Tiles[] = {
-    {FM_TILE_PS_128x128_O2, FM_TILE_128x128_O2_U1, 1.00, 2},
-    {FM_TILE_PS_128x256_W8, FM_TILE_128x256_W8_U1, 0.97, 1},
-    {FM_TILE_128x256_W8, FM_TILE_128x256_W8_U1, 0.93, 1},
-    {FM_TILE_256x128_W8, FM_TILE_256x128_W8_U1, 0.92, 1},
-    {FM_TILE_128x128_W16, FM_TILE_128x128_W16, 0.86, 1},
-    {FM_TILE_128x64_W8, FM_TILE_128x64_W8, 0.84, 2},
-    {FM_TILE_PS_128x96_O2, FM_TILE_PI_128x96_O2, 0.87, 2, true},
-    {FM_TILE_64x64, FM_TILE_64x64, 0.75, 3}};
+    {FM_TILE_PS_128x128_O2, 0.1257, 30, 0},  {FM_TILE_PS_128x256_W8, 0.2560, 30, 0},
+    {FM_TILE_PS_128x96_O2, 0.0960, 30, 0},   {FM_TILE_128x64, 0.0650, 34, 0},
+    {FM_TILE_64x128, 0.0655, 34, 0},         {FM_TILE_64x64, 0.0340, 32, 0.037},
+    {FM_TILE_PS_32x32_K32, 0.0103, 50, 0.0129}};
 const TileCand kF32Tiles[] = {
-    {FM_TILE_PS_128x256_W8, FM_TILE_PP_128x256_W8, 1.00, 2},
-    {FM_TILE_PS_128x128_O2, FM_TILE_128x128_W8, 0.985, 3},
-    {FM_TILE_256x256_W16, -1, 0.96, 1},
-    {FM_TILE_256x128_W8, FM_TILE_256x128_W8, 0.89, 1},
-    {FM_TILE_128x128_W8, FM_TILE_128x128_W8, 0.76, 2},
-    {FM_TILE_64x128, FM_TILE_64x128, 0.71, 3},
-    {FM_TILE_128x64, FM_TILE_128x64, 0.68, 3},
-    {FM_TILE_64x64, FM_TILE_64x64, 0.63, 4}};
+    {FM_TILE_PS_128x256_W8, 0.1383, 44, 0}, {FM_TILE_PS_128x128_O2, 0.0695, 40, 0},
+    {FM_TILE_128x64, 0.0368, 43, 0},        {FM_TILE_64x128, 0.0368, 43, 0},
+    {FM_TILE_64x64, 0.0192, 43, 0.0227},    {FM_TILE_PS_32x32_K32, 0.0057, 60, 0.0099}};
+// a launch's own cost beside its tiles
+const double kLaunchUs = 3.0;
+const double kCopyBytesPerUs = 4.9e6;
+// one work group to a CU: nothing covers its wait for operands that are not in
+// L2 (strassen one level 2048^3 FP64: 4 of 7 leaves as 256 128 x 128 tiles and
+// 3 as 64 x 64 ones 294 us, all on 64 x 64 tiles 266)
+const double kAlonePenalty = 1.15;
+// What the spread kernels cannot take (M below a vector, K below a slice,
+// columns past 32-bit offsets) runs on the 64 x 64 tile's predicated loop.
+const double kEdgePenalty = 1.3;
 // split-bf16: kernels on prepared slice planes (any shape: the planes are
-// padded to whole tiles)
+// padded to whole tiles), throughput per tile area and resident work groups
+// per CU
 // (Strassen, two levels, 16384^3 FP32, i.e. 49 products of 4096^3, whole
 // multiply: 251 TFLOP/s with B straight to registers, 232 and 229 with the
 // LDS-staged 128 x 256 and 256 x 128 kernels)
-const TileCand kSplitTiles[] = {{FM_TILE_SP_128x256_BD, FM_TILE_SP_128x256_BD, 1.00, 1},
-                                {FM_TILE_SP_256x128_IL, FM_TILE_SP_256x128_IL, 0.92, 1},
-                                {FM_TILE_SP_128x256_IL, FM_TILE_SP_128x256_IL, 0.92, 1},
-                                {FM_TILE_SP_128x128, FM_TILE_SP_128x128, 0.88, 2},
-                                {FM_TILE_SP_128x128_DB, FM_TILE_SP_128x128_DB, 0.83, 1}};
-// edge kernels run slower than whole-tile ones (predicated loads).  The
-// spread kernels' edge variant is offered for the 128 x 96 tile only: on
-// 128 x 128 and 128 x 256 tiles it measured 6% slower per tile than the
-// whole-tile kernel (classical 131072 x 2400 x 2400 FP64 66.8 TFLOP/s as
-// one launch, 71.8 cut into a whole-tile core and a strip; the C3 FP32
-// batch 119.2 against 124.4), while as the tall-skinny leaves' 88-column
-// strip kernel it took the one-level multiply from 68.7 to 71.0
-const double kEdgePenalty = 0.93;
-const double kSpreadEdgePenalty = 0.93;
+struct SplitCand {
+  int cfg;
+  double eff;
+  int per_cu;
+};
+const SplitCand kSplitTiles[] = {{FM_TILE_SP_128x256_BD, 1.00, 1},
+                                 {FM_TILE_SP_256x128_IL, 0.92, 1},
+                                 {FM_TILE_SP_128x256_IL, 0.92, 1},
+                                 {FM_TILE_SP_128x128, 0.88, 2},
+                                 {FM_TILE_SP_128x128_DB, 0.83, 1}};
+const int kCUs = 256;
 
-const TileCand* tile_cands(fm_dtype dt, fm_mode mode, int* n) {
-  if (mode == FM_MODE_SPLIT_BF16) {
-    *n = (int)(sizeof(kSplitTiles) / sizeof(kSplitTiles[0]));
-    return kSplitTiles;
-  }
-  if (dt == FM_F64) {
-    *n = (int)(sizeof(kF64Tiles) / sizeof(kF64Tiles[0]));
-    return kF64Tiles;
-  }
-  *n = (int)(sizeof(kF32Tiles) / sizeof(kF32Tiles[0]));
-  return kF32Tiles;
-}
-
-int64_t count_tiles(int cfg, const std::vector<FmGemmDesc>& prods, size_t from = 0) {
+int64_t count_tiles(int cfg, const std::vector<FmGemmDesc>& prods) {
   int bm, bn;
   fm_tile_dims(cfg, &bm, &bn);
   int64_t tiles = 0;
-  for (size_t i = from; i < prods.size(); ++i)
-    tiles += ((prods[i].M + bm - 1) / bm) * ((prods[i].N + bn - 1) / bn);
+  for (const FmGemmDesc& d : prods) tiles += (int64_t)((d.M + bm - 1) / bm) * ((d.N + bn - 1) / bn);
   return tiles;
 }
 
-// Every product a whole number of tiles and K slices, columns 16-byte aligned.
-bool whole_tiles(fm_dtype dt, int cfg, const std::vector<FmGemmDesc>& prods) {
-  if (fm_tile_planes(cfg)) return true;
+// Estimated time of one launch of `prods` on candidate c (us).  Equal depths:
+// the busiest CU's tiles.  Unequal depths: the CUs' mean, and half of the
+// deepest tile for the end of the launch.  At least the time of the products'
+// bytes (a strip reads a whole operand again), a fifth of which is not hidden
+// behind the products of a compute-bound launch.
+double cand_us(fm_dtype dt, const TileCand& c, const std::vector<FmGemmDesc>& prods) {
   int bm, bn;
-  fm_tile_dims(cfg, &bm, &bn);
-  const int bk = fm_tile_bk(cfg), vl = dt == FM_F64 ? 2 : 4;
-  for (const FmGemmDesc& d : prods)
-    if (d.M % bm || d.N % bn || d.K % bk || d.K == 0 || d.a.off % vl || d.a.ld % vl ||
-        d.b.off % vl || d.b.ld % vl)
-      return false;
-  return true;
-}
-
-// Every product has M and K multiples of the vector width and 16-byte
-// aligned columns (the spread kernels' EVEN launch).
-bool even_slices(fm_dtype dt, int cfg, const std::vector<FmGemmDesc>& prods) {
-  (void)cfg;
-  const int vl = dt == FM_F64 ? 2 : 4;
-  for (const FmGemmDesc& d : prods)
-    if (d.M % vl || d.K % vl || d.K == 0 || d.a.off % vl || d.a.ld % vl || d.b.off % vl ||
-        d.b.ld % vl)
-      return false;
-  return true;
-}
-
-// How a candidate takes a product list: the kernel (-1: not offered) and
-// its form, 2 whole tiles, 1 the spread kernel's edge variant, 0 the
-// predicated edge kernel.
-int cand_kernel(fm_dtype dt, const TileCand& c, const std::vector<FmGemmDesc>& prods, int* form) {
-  if (whole_tiles(dt, c.cfg_full, prods)) {
-    *form = 2;
-    return c.cfg_full;
+  fm_tile_dims(c.cfg, &bm, &bn);
+  double work = 0, kmax = 0, kmin = 1e30, elems = 0;
+  int64_t tiles = 0;
+  for (const FmGemmDesc& d : prods) {
+    const int64_t t = (int64_t)((d.M + bm - 1) / bm) * ((d.N + bn - 1) / bn);
+    tiles += t;
+    work += (double)t * (d.K + c.k0);
+    kmax = std::max(kmax, (double)d.K);
+    kmin = std::min(kmin, (double)d.K);
+    elems += ((double)d.M + d.N) * d.K + (double)d.M * d.N;
   }
-  if (c.spread && even_slices(dt, c.cfg_full, prods)) {
-    *form = 1;
-    return c.cfg_full;
-  }
-  *form = 0;
-  return c.cfg_edge;
+  const double mem = elems * elem_size(dt) / kCopyBytesPerUs;
+  const double tile = c.us_k * (kmax + c.k0);
+  const double busy = kmin < kmax      ? c.us_k * work / kCUs + 0.5 * tile
+                      : tiles > kCUs ? tile * (double)((tiles + kCUs - 1) / kCUs)
+                                     : tile * kAlonePenalty;
+  const double t = std::max(busy, std::max(c.lat_k * kmax, mem)) + 0.2 * mem;
+  const bool fits = any_tiles(dt, c.cfg, prods) || whole_tiles(dt, c.cfg, prods);
+  return kLaunchUs + t * (fits ? 1.0 : kEdgePenalty);
 }
 
-// Estimated time of one launch of `tiles` tiles: rounds of per_cu work
-// groups on each of the 256 CUs.
-double tile_time(const TileCand& c, int64_t tiles, int form) {
+// Split-bf16: rounds of per_cu work groups on each CU, in relative units.
+double split_time(const SplitCand& c, int64_t tiles) {
   int bm, bn;
-  fm_tile_dims(c.cfg_full, &bm, &bn);
-  const int64_t slots = 256LL * c.per_cu;
-  const double rounds = (double)((tiles + slots - 1) / slots);
-  const double pen = form == 2 ? 1.0 : form == 1 ? kSpreadEdgePenalty : kEdgePenalty;
-  return rounds * bm * bn * c.per_cu / (c.eff * pen);
+  fm_tile_dims(c.cfg, &bm, &bn);
+  const int64_t slots = (int64_t)kCUs * c.per_cu;
+  return (double)((tiles + slots - 1) / slots) * bm * bn * c.per_cu / c.eff;
 }
 
-const TileCand* find_cand(fm_dtype dt, fm_mode mode, int cfg) {
-  int n;
-  const TileCand* c = tile_cands(dt, mode, &n);
-  for (int i = 0; i < n; ++i)
-    if (c[i].cfg_full == cfg || c[i].cfg_edge == cfg) return &c[i];
-  return nullptr;
-}
-
-// Best candidate for a product list: its kernel and estimated time.
-int best_tile(fm_dtype dt, fm_mode mode, const std::vector<FmGemmDesc>& prods, double* t_out) {
-  int nc;
-  const TileCand* cands = tile_cands(dt, mode, &nc);
-  int best = FM_TILE_64x64;
-  double best_t = 1e300;
-  for (int i = 0; i < nc; ++i) {
-    int form;
-    const int cfg = cand_kernel(dt, cands[i], prods, &form);
-    if (cfg < 0) continue;
-    const double t = tile_time(cands[i], count_tiles(cfg, prods), form);
-    if (t < best_t * 0.999) {
-      best_t = t;
+// Best candidate for a product list and its estimated time.  The lists run
+// from large tiles to small: a smaller one has to be estimated faster by
+// `margin`, about what the estimates are good for.
+int best_tile(fm_dtype dt, fm_mode mode, const std::vector<FmGemmDesc>& prods, double* t_out,
+              double margin = 0.97) {
+  int best = -1;
+  double best_t = 0;
+  auto offer = [&](int cfg, double t, double margin) {
+    if (best < 0 || t < best_t * margin) {
       best = cfg;
+      best_t = t;
     }
+  };
+  if (mode == FM_MODE_SPLIT_BF16) {
+    for (const SplitCand& c : kSplitTiles) offer(c.cfg, split_time(c, count_tiles(c.cfg, prods)), 0.999);
+  } else {
+    auto fits = [&](int cfg) { return whole_tiles(dt, cfg, prods) || any_tiles(dt, cfg, prods); };
+    auto each = [&](const TileCand* c, size_t n) {
+      for (size_t i = 0; i < n; ++i)
+        if (fits(c[i].cfg) || c[i].cfg == FM_TILE_64x64) offer(c[i].cfg, cand_us(dt, c[i], prods), margin);
+    };
+    if (dt == FM_F64)
+      each(kF64Tiles, sizeof(kF64Tiles) / sizeof(kF64Tiles[0]));
+    else
+      each(kF32Tiles, sizeof(kF32Tiles) / sizeof(kF32Tiles[0]));
   }
   if (t_out) *t_out = best_t;
   return best;
 }
-}  // namespace
 
-namespace {
-// Whole-tile carve-out: a launch whose products are not all whole tiles runs
-// every tile on the predicated edge kernel.  Cutting each ragged product
-// into its whole-tile core (the unpredicated kernel) and the row / column
-// strips left over (a second launch, its own tile) is worth it when the
-// strips are a small share; every output element is still computed by the
-// same K-ordered MFMA sequence.  Returns false (prods unchanged) when it
-// does not pay or does not apply.
+// Estimated time of `prods` on configuration cfg (negative: not a candidate)
+// and the tiles one round of the launch holds.
+double list_time(fm_dtype dt, fm_mode mode, int cfg, const std::vector<FmGemmDesc>& prods, int64_t* round) {
+  *round = kCUs;
+  if (mode == FM_MODE_SPLIT_BF16) {
+    for (const SplitCand& c : kSplitTiles)
+      if (c.cfg == cfg) {
+        *round = (int64_t)kCUs * c.per_cu;
+        return split_time(c, count_tiles(cfg, prods));
+      }
+    return -1;
+  }
+  const TileCand* c = dt == FM_F64 ? kF64Tiles : kF32Tiles;
+  const size_t n = dt == FM_F64 ? sizeof(kF64Tiles) / sizeof(kF64Tiles[0]) : sizeof(kF32Tiles) / sizeof(kF32Tiles[0]);
+  for (size_t i = 0; i < n; ++i)
+    if (c[i].cfg == cfg) return cand_us(dt, c[i], prods);
+  return -1;
+}
+
 FmGemmDesc gsub(const FmGemmDesc& d, int64_t i0, int64_t j0, int64_t m, int64_t n) {
   return gdesc(op_sub(d.a, i0, 0), op_sub(d.b, 0, j0), op_sub(d.c, i0, j0), m, n, d.K, d.alpha,
                d.beta);
 }
 
+// Whole-tile carve-out: a ragged product's last tile row and column are
+// partly empty.  Cutting each product into its whole-tile core and the row and
+// column strips left over (a second launch, with the tile that fits them) is
+// worth it when the emptiness is a large share; every output element is
+// computed by the same K-ordered MFMA sequence either way.  Returns false
+// (prods unchanged) when it does not pay or does not apply.
 bool carve_full(const Plan& P, int cfg, std::vector<FmGemmDesc>& prods, std::vector<FmGemmDesc>& strips,
-                std::vector<FmGemmDesc>& odd, int* cfg_core, int* cfg_strips, int* cfg_odd) {
+                int* cfg_core, int* cfg_strips) {
   if (P.tile >= 0 || P.mode != FM_MODE_PLAIN) return false;
-  const TileCand* c = find_cand(P.dtype, P.mode, cfg);
-  if (!c || whole_tiles(P.dtype, c->cfg_full, prods)) return false;
-  int bm, bn;
-  fm_tile_dims(c->cfg_full, &bm, &bn);
-  const int bk = fm_tile_bk(c->cfg_full), vl = P.dtype == FM_F64 ? 2 : 4;
-  std::vector<FmGemmDesc> core, st, od;
-  for (const FmGemmDesc& d : prods) {
-    if (d.K % bk || d.K == 0 || d.a.off % vl || d.a.ld % vl || d.b.off % vl || d.b.ld % vl) {
-      // a product the whole-tile kernel cannot take (ragged K, unaligned
-      // columns) runs whole in a launch of its own, with its own tile, so
-      // that it neither sends every other product of a grouped launch to
-      // the edge kernel nor takes the thin strips' small tile
-      od.push_back(d);
-      continue;
+  int64_t round;
+  const double t_all = list_time(P.dtype, P.mode, cfg, prods, &round);
+  const TileCand* cands = P.dtype == FM_F64 ? kF64Tiles : kF32Tiles;
+  const size_t n = P.dtype == FM_F64 ? sizeof(kF64Tiles) / sizeof(kF64Tiles[0])
+                                     : sizeof(kF32Tiles) / sizeof(kF32Tiles[0]);
+  double best_t = 0.995 * t_all;
+  std::vector<FmGemmDesc> core, st, best_core, best_st;
+  for (size_t i = 0; i < n; ++i) {
+    int bm, bn;
+    fm_tile_dims(cands[i].cfg, &bm, &bn);
+    core.clear();
+    st.clear();
+    for (const FmGemmDesc& d : prods) {
+      const int64_t Mf = d.M / bm * bm, Nf = d.N / bn * bn;
+      if (Mf > 0 && Nf > 0) core.push_back(gsub(d, 0, 0, Mf, Nf));
+      if (d.N > Nf) st.push_back(gsub(d, 0, Nf, d.M, d.N - Nf));           // right strip, all rows
+      if (d.M > Mf && Nf > 0) st.push_back(gsub(d, Mf, 0, d.M - Mf, Nf));  // bottom strip
     }
-    const int64_t Mf = d.M / bm * bm, Nf = d.N / bn * bn;
-    if (Mf > 0 && Nf > 0) core.push_back(gsub(d, 0, 0, Mf, Nf));
-    if (d.N > Nf) st.push_back(gsub(d, 0, Nf, d.M, d.N - Nf));          // right strip, all rows
-    if (d.M > Mf && Nf > 0) st.push_back(gsub(d, Mf, 0, d.M - Mf, Nf));  // bottom strip
+    if (core.empty() || st.empty()) continue;
+    if (!whole_tiles(P.dtype, cands[i].cfg, core) && !any_tiles(P.dtype, cands[i].cfg, core)) continue;
+    double t_strips = 0;
+    const int cs = best_tile(P.dtype, P.mode, st, &t_strips);
+    const double t = cand_us(P.dtype, cands[i], core) + t_strips;
+    if (t >= best_t) continue;
+    best_t = t;
+    best_core = core;
+    best_st = st;
+    *cfg_core = cands[i].cfg;
+    *cfg_strips = cs;
   }
-  if (core.empty() || (st.empty() && od.empty())) return false;
-  double t_strips = 0, t_odd = 0;
-  const int cs = st.empty() ? cfg : best_tile(P.dtype, P.mode, st, &t_strips);
-  const int co = od.empty() ? cfg : best_tile(P.dtype, P.mode, od, &t_odd);
-  int form_all;
-  (void)cand_kernel(P.dtype, *c, prods, &form_all);
-  const double t_core = tile_time(*c, count_tiles(c->cfg_full, core), 2);
-  const double t_all = tile_time(*c, count_tiles(cfg, prods), form_all);
-  if (t_core + t_strips + t_odd >= 0.97 * t_all) return false;
-  prods = std::move(core);
-  strips = std::move(st);
-  odd = std::move(od);
-  *cfg_core = c->cfg_full;
-  *cfg_strips = cs;
-  *cfg_odd = co;
+  if (best_core.empty()) return false;
+  prods = std::move(best_core);
+  strips = std::move(best_st);
   return true;
 }
 }  // namespace
 
-int pick_tile(fm_dtype dt, fm_mode mode, int tile, const std::vector<FmGemmDesc>& prods) {
-  if (tile >= 0) return tile;
-  return best_tile(dt, mode, prods, nullptr);
+// (a depth-first child changes its one launch to a smaller tile only for a
+// tenth: its siblings' stages and leaves follow, and fill the machine again)
+int pick_tile(const Plan& P, const std::vector<FmGemmDesc>& prods) {
+  if (P.tile >= 0) return P.tile;
+  return best_tile(P.dtype, P.mode, prods, nullptr, P.child ? 0.90 : 0.97);
 }
 
 // The GPU form of the reference's HYBRID remainder rule (util/par_util.hpp:
@@ -604,21 +600,24 @@ int pick_tile(fm_dtype dt, fm_mode mode, int tile, const std::vector<FmGemmDesc>
 // launch with the tile that finishes them soonest.  Products stay whole, so
 // every output element is computed by the same instructions either way.
 void split_remainder(const Plan& P, int cfg, std::vector<FmGemmDesc>& prods,
-                     std::vector<FmGemmDesc>& rest, int* cfg_rest, int* cfg_head) {
+                     std::vector<FmGemmDesc>& rest, int* cfg_rest) {
   if (P.tile >= 0 || P.mode == FM_MODE_OZAKI_INT8) return;
-  const TileCand* c = find_cand(P.dtype, P.mode, cfg);
-  if (!c) return;
-  const int64_t slots = 256LL * c->per_cu;
+  int64_t round;
+  const double t_one = list_time(P.dtype, P.mode, cfg, prods, &round);
+  if (t_one < 0) return;
   const int64_t total = count_tiles(cfg, prods);
-  const int64_t full = total / slots * slots;
+  const int64_t full = total / round * round;
   if (full == 0 || full == total) return;
+  // a depth-first child whose tiles are all resident at once keeps the one
+  // leaf launch its schedule is documented with
+  if (P.child && P.mode == FM_MODE_PLAIN && total < 2 * round) return;
   // the longest prefix of products whose tiles fill whole rounds
   int bm, bn;
   fm_tile_dims(cfg, &bm, &bn);
   int64_t acc = 0;
   size_t cut = 0;
   while (cut < prods.size()) {
-    const int64_t t = ((prods[cut].M + bm - 1) / bm) * ((prods[cut].N + bn - 1) / bn);
+    const int64_t t = (int64_t)((prods[cut].M + bm - 1) / bm) * ((prods[cut].N + bn - 1) / bn);
     if (acc + t > full) break;
     acc += t;
     ++cut;
@@ -628,17 +627,11 @@ void split_remainder(const Plan& P, int cfg, std::vector<FmGemmDesc>& prods,
   std::vector<FmGemmDesc> head(prods.begin(), prods.begin() + (std::ptrdiff_t)cut);
   double t_tail = 0;
   const int cr = best_tile(P.dtype, P.mode, tail, &t_tail);
-  int form_one, form_head;
-  (void)cand_kernel(P.dtype, *c, prods, &form_one);
-  const int ch = cand_kernel(P.dtype, *c, head, &form_head);
-  const double t_one = tile_time(*c, total, form_one);
-  const double t_two = tile_time(*c, full, form_head) + t_tail;
+  const double t_two = list_time(P.dtype, P.mode, cfg, head, &round) + t_tail;
   if (t_two >= t_one * 0.99) return;
   prods.resize(cut);
   rest = std::move(tail);
   *cfg_rest = cr;
-  // the full rounds may be whole tiles even where the remainder was not
-  if (ch >= 0) *cfg_head = ch;
 }
 
 // Depth-first top level (the reference's DFS order, algorithms/strassen.hpp:
@@ -706,6 +699,7 @@ fm_status build_dfs(fm_dtype dt, const Problem& p, const std::vector<Dims>& dims
     seq.slices = p.slices;
     seq.tile = p.tile;
     seq.split_rem = p.split_rem;
+    seq.child = true;
     st = assemble(seq, child, child_base + child[0].ws_elems);
     if (st != FM_OK) return st;
     for (Launch& L : seq.launches) out.pre.push_back(std::move(L));
@@ -1054,7 +1048,7 @@ fm_status assemble(Plan& P, std::vector<SubPlan>& subs, int64_t ws_elems, int pe
       if (st != FM_OK) return st;
       P.launches.push_back(std::move(L));
     } else {
-      const int cfg = pick_tile(P.dtype, P.mode, P.tile, leaves);
+      const int cfg = pick_tile(P, leaves);
       if (fm_tile_planes(cfg) && P.mode != FM_MODE_SPLIT_BF16)
         return set_err(FM_ERR_INVALID_ARG, "tile config " + std::to_string(cfg) + " is for split_bf16 leaves");
       // split_bf16 leaves off the slice planes run the in-loop kernel, which
@@ -1064,13 +1058,12 @@ fm_status assemble(Plan& P, std::vector<SubPlan>& subs, int64_t ws_elems, int pe
           cfg != FM_TILE_128x128_W8)
         return set_err(FM_ERR_INVALID_ARG, "tile config " + std::to_string(cfg) +
                                                " has no split_bf16 kernel");
-      std::vector<FmGemmDesc> rest, strips, odd;
-      int cfg_rest = cfg, cfg_head = cfg, cfg_main = cfg, cfg_strips = cfg, cfg_odd = cfg;
-      if (persistent_grid == 0 && P.split_rem &&
-          carve_full(P, cfg, leaves, strips, odd, &cfg_main, &cfg_strips, &cfg_odd))
-        cfg_rest = cfg_head = cfg_main;
-      if (persistent_grid == 0 && P.split_rem)
-        split_remainder(P, cfg_main, leaves, rest, &cfg_rest, &cfg_head);
+      std::vector<FmGemmDesc> rest, strips;
+      int cfg_rest = cfg, cfg_main = cfg, cfg_strips = cfg;
+      if (persistent_grid == 0 && P.split_rem) {
+        (void)carve_full(P, cfg, leaves, strips, &cfg_main, &cfg_strips);
+        split_remainder(P, cfg_main, leaves, rest, &cfg_rest);
+      }
       auto leaf = [&](std::vector<FmGemmDesc> prods, int c) {
         // the preparation launch is one flat grid of at most 2^31 - 1 work
         // groups (64 rows x 4 K slices each, per operand; an upper bound
@@ -1082,12 +1075,11 @@ fm_status assemble(Plan& P, std::vector<SubPlan>& subs, int64_t ws_elems, int pe
         if (fm_tile_planes(c)) return split_launch(std::move(prods), c, &wsb);
         return gemm_launch(std::move(prods), c, FM_STAGE_LEAF, P.dtype);
       };
-      P.launches.push_back(leaf(std::move(leaves), cfg_head));
+      P.launches.push_back(leaf(std::move(leaves), cfg_main));
       P.launches.back().gm.grid = persistent_grid;
       P.launches.back().sp.grid = persistent_grid;
       if (!rest.empty()) P.launches.push_back(leaf(std::move(rest), cfg_rest));
       if (!strips.empty()) P.launches.push_back(leaf(std::move(strips), cfg_strips));
-      if (!odd.empty()) P.launches.push_back(leaf(std::move(odd), cfg_odd));
     }
   }
   int maxd = 0;

@@ -54,6 +54,7 @@ struct Plan {
   int tile = -1;       // forced leaf tile configuration (-1: cost model)
   int split_rem = 1;   // whole-tile carve-out and remainder launch
   int dfs_levels = 0;  // depth-first top levels the plan runs
+  bool child = false;  // the sub-plan of a depth-first child
   std::vector<Launch> launches;
   std::vector<void*> ext;          // role table (roles >= 4) of batched plans
   void* dbuf = nullptr;            // descriptors + role table on the device (owned)
@@ -116,10 +117,10 @@ fm_status build_dfs(fm_dtype dt, const Problem& p, const std::vector<Dims>& dims
 // 0 launches one work group per tile.
 fm_status assemble(Plan& P, std::vector<SubPlan>& subs, int64_t ws_elems, int persistent_grid = 0);
 
-int pick_tile(fm_dtype dt, fm_mode mode, int tile, const std::vector<FmGemmDesc>& prods);
+int pick_tile(const Plan& P, const std::vector<FmGemmDesc>& prods);
 // move the products of a part-empty last round of tiles to `rest`
 void split_remainder(const Plan& P, int cfg, std::vector<FmGemmDesc>& prods,
-                     std::vector<FmGemmDesc>& rest, int* cfg_rest, int* cfg_head);
+                     std::vector<FmGemmDesc>& rest, int* cfg_rest);
 // process defaults of the per-call options (fm_set_* change them)
 extern fm_options g_defaults;
 fm_status check_options(const fm_options& o);
