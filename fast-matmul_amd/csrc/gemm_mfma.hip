@@ -45,16 +45,7 @@ struct FmMfma<float> {
   __device__ __forceinline__ static int out_row(int g, int v) { return 4 * g + v; }
 };
 
-// Map a work-group id to a tile id so that each of the 8 XCDs (which receive
-// work groups round-robin) walks a contiguous range of tiles: neighbouring
-// tiles share A/B panels in that XCD's L2.
 constexpr int FM_TILE_GROUP = 8;
-
-__device__ __forceinline__ int fm_xcd_remap(int wg, int nwg) {
-  const int full = nwg & ~7;
-  if (wg < full) return (wg & 7) * (full >> 3) + (wg >> 3);
-  return wg;
-}
 
 // MINW: minimum waves per SIMD the register allocation must allow (2 with
 // four-wave work groups lets two work groups share a CU, so one group's
@@ -115,7 +106,7 @@ __global__ void __launch_bounds__(64 * WM * WN, MINW) fm_gemm_kernel(FmGemmArgs 
   // Persistent when the grid is smaller than the tile count: work group b
   // takes tiles b, b + grid, b + 2 grid, ...
   for (int tile = blockIdx.x; tile < args.total_tiles; tile += gridDim.x) {
-  const int wg = fm_xcd_remap(tile, args.total_tiles);
+  const int wg = fm_xcd_tile(tile, args.total_tiles, args.chunk);
   int g;
   if (args.uniform) {
     const int per = args.descs[0].tiles_m * args.descs[0].tiles_n;

@@ -17,6 +17,8 @@ struct FmGemmDesc {
   double alpha, beta;
 };
 
+constexpr int FM_XCD_CHUNK = 64;  // tiles per XCD run of launches of unequal depth (fm_xcd_tile)
+
 struct FmGemmArgs {
   FmBases bases;
   const FmGemmDesc* descs;
@@ -25,6 +27,7 @@ struct FmGemmArgs {
   int32_t uniform;  // all products have one shape: tile -> product by division
   int32_t vec;      // the base pointers are 16-byte aligned: vector loads allowed for the
                     // products whose own offsets and leading dimensions keep columns aligned
+  int32_t chunk;    // tiles per XCD run (fm_xcd_tile); 0: one eighth each
   int32_t grid;     // > 0: persistent launch with this many work groups
   int32_t full;     // every product is a whole number of tiles and K slices
   int32_t any;      // every product fits the spread kernels' ANY variant: M at least the
@@ -162,6 +165,7 @@ struct FmSplitArgs {
   const FmSplitPrep* preps;
   int32_t ndesc, total_tiles;
   int32_t uniform, grid;        // as in FmGemmArgs
+  int32_t chunk;                // as in FmGemmArgs
   int32_t nprep;
   int32_t prep_wgs;             // work groups of the preparation launch (all operands)
   int32_t even_k;               // 1: every product has an even number of K slices

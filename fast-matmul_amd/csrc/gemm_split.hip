@@ -37,12 +37,6 @@ __device__ __forceinline__ void fm_split3(const float (&x)[8], uint4 (&out)[3]) 
   out[2] = make_uint4(l[0] | l[1] << 16, l[2] | l[3] << 16, l[4] | l[5] << 16, l[6] | l[7] << 16);
 }
 
-__device__ __forceinline__ int fm_xcd_remap2(int wg, int nwg) {
-  const int full = nwg & ~7;
-  if (wg < full) return (wg & 7) * (full >> 3) + (wg >> 3);
-  return wg;
-}
-
 template <int BM, int BN, int WM, int WN>
 __global__ void __launch_bounds__(64 * WM * WN) fm_gemm_bf16x3_kernel(FmGemmArgs args) {
   constexpr int NT = 64 * WM * WN;
@@ -59,7 +53,7 @@ __global__ void __launch_bounds__(64 * WM * WN) fm_gemm_bf16x3_kernel(FmGemmArgs
 
   // persistent when the grid is smaller than the tile count
   for (int tile = blockIdx.x; tile < args.total_tiles; tile += gridDim.x) {
-  const int wg = fm_xcd_remap2(tile, args.total_tiles);
+  const int wg = fm_xcd_tile(tile, args.total_tiles, args.chunk);
   int g;
   if (args.uniform) {
     g = wg / (args.descs[0].tiles_m * args.descs[0].tiles_n);
@@ -330,7 +324,7 @@ __global__ void __launch_bounds__(64 * WM * WN) fm_split_gemm(FmSplitArgs args) 
   __shared__ __align__(16) fm_u32x4 Bs[NBUF][3][BN][4];
 
   for (int tile = blockIdx.x; tile < args.total_tiles; tile += gridDim.x) {
-  const int wg = fm_xcd_remap2(tile, args.total_tiles);
+  const int wg = fm_xcd_tile(tile, args.total_tiles, args.chunk);
   int g;
   if (args.uniform) {
     g = wg / (args.descs[0].tiles_m * args.descs[0].tiles_n);
@@ -509,7 +503,7 @@ __global__ void __launch_bounds__(64 * WM * WN) fm_split_gemm_bd(FmSplitArgs arg
   static_assert(TM >= 1 && TN >= 1, "bad tile");
   __shared__ __align__(16) fm_u32x4 As[2][KS][3][BM][4];
 
-  const int wg = fm_xcd_remap2(blockIdx.x, args.total_tiles);
+  const int wg = fm_xcd_tile(blockIdx.x, args.total_tiles, args.chunk);
   int g;
   if (args.uniform) {
     g = wg / (args.descs[0].tiles_m * args.descs[0].tiles_n);

@@ -212,6 +212,12 @@ bool any_tiles(fm_dtype dt, int cfg, const std::vector<FmGemmDesc>& prods) {
   return true;
 }
 
+bool depths_differ(const std::vector<FmGemmDesc>& prods) {
+  for (const FmGemmDesc& d : prods)
+    if (d.K != prods[0].K) return true;
+  return false;
+}
+
 Launch gemm_launch(std::vector<FmGemmDesc> descs, int cfg, int stage, fm_dtype dt) {
   int bm, bn;
   fm_tile_dims(cfg, &bm, &bn);
@@ -234,6 +240,7 @@ Launch gemm_launch(std::vector<FmGemmDesc> descs, int cfg, int stage, fm_dtype d
   // A/B column starts 16-byte aligned (the base pointers are checked at
   // launch); the spread kernels' ANY variant takes the others.
   L.vec_ok = 1;
+  L.gm.chunk = depths_differ(descs) ? FM_XCD_CHUNK : 0;
   L.gm.full = whole_tiles(dt, cfg, descs) ? 1 : 0;
   L.gm.any = any_tiles(dt, cfg, descs) ? 1 : 0;
   L.cfg = cfg;
@@ -355,6 +362,7 @@ Launch split_launch(std::vector<FmGemmDesc> prods, int cfg, size_t* ws_bytes) {
   L.sp.ndesc = (int32_t)L.sdescs.size();
   L.sp.total_tiles = t;
   L.sp.uniform = uniform ? 1 : 0;
+  L.sp.chunk = depths_differ(prods) ? FM_XCD_CHUNK : 0;
   L.sp.nprep = (int32_t)L.spreps.size();
   L.sp.prep_wgs = prep_wgs;
   L.sp.even_k = 1;
@@ -1040,6 +1048,10 @@ fm_status assemble(Plan& P, std::vector<SubPlan>& subs, int64_t ws_elems, int pe
   }
   std::vector<FmGemmDesc> leaves;
   for (SubPlan& s : subs) leaves.insert(leaves.end(), s.leaves.begin(), s.leaves.end());
+  // products of unequal depth: deepest first (fm_xcd_tile)
+  if (depths_differ(leaves))
+    std::stable_sort(leaves.begin(), leaves.end(),
+                     [](const FmGemmDesc& x, const FmGemmDesc& y) { return x.K > y.K; });
   size_t wsb = (size_t)ws_elems * elem_size(P.dtype);
   if (!leaves.empty()) {
     if (P.mode == FM_MODE_OZAKI_INT8) {
