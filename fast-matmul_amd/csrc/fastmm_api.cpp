@@ -536,10 +536,11 @@ fm_status fm_fastmatmul_scaled(const char* alg_name, fm_dtype dtype, fm_mode mod
   hipStream_t s = (hipStream_t)stream;
   const int f64 = dtype == FM_F64;
   return timed(s, ms_out, lock, [&]() -> fm_status {
-    hipError_t e = fm_scaling_copy(f64, A, lda, w + lay.o_a, m, m, k, s);
-    if (e == hipSuccess) e = fm_scaling_copy(f64, B, ldb, w + lay.o_b, k, k, n, s);
-    if (e != hipSuccess) return hip_err(e, "scaling copy");
     FmScaleArgs sa;
+    sa.srcA = A;
+    sa.srcB = B;
+    sa.ld_srcA = lda;
+    sa.ld_srcB = ldb;
     sa.A = w + lay.o_a;
     sa.B = w + lay.o_b;
     sa.lda = m;
@@ -555,7 +556,7 @@ fm_status fm_fastmatmul_scaled(const char* alg_name, fm_dtype dtype, fm_mode mod
     sa.f2 = w + lay.o_f2;
     sa.u1 = w + lay.o_u1;
     sa.u2 = w + lay.o_u2;
-    e = fm_scaling_run(f64, sa, s);
+    hipError_t e = fm_scaling_run(f64, sa, s);
     if (e != hipSuccess) return hip_err(e, "scaling");
     void* prod = temp ? (void*)(w + lay.o_t) : C;
     const int64_t ldp = temp ? m : ldc;

@@ -5,11 +5,14 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-// A (m x k) and B (k x n) are scaled in place (they are the caller's
-// operands copied into the workspace); r (m) and s (n) receive the row and
-// column factors of the product; f, f2 hold per-pass factors and u1, u2 the
-// per-pass maxima (max(m, k, n) entries each).
+// srcA (m x k) and srcB (k x n), the caller's operands, are scaled into A and
+// B (in the workspace); r (m) and s (n) receive the row and column factors of
+// the product.  f, f2 and u1, u2 hold a step's maxima and then its factors,
+// outer and inner (max(m, k, n) entries each).
 struct FmScaleArgs {
+  const void* srcA;
+  const void* srcB;
+  int64_t ld_srcA, ld_srcB;
   void* A;
   void* B;
   int64_t lda, ldb;
@@ -25,8 +28,6 @@ struct FmScaleArgs {
 };
 
 hipError_t fm_scaling_run(int dtype_f64, const FmScaleArgs& a, hipStream_t s);
-hipError_t fm_scaling_copy(int dtype_f64, const void* X, int64_t ldx, void* Y, int64_t ldy,
-                           int rows, int cols, hipStream_t s);
 hipError_t fm_scaling_post(int dtype_f64, const void* P, int64_t ldp, void* C, int64_t ldc,
                            int rows, int cols, const void* r, const void* sv, double alpha,
                            double beta, hipStream_t s);
