@@ -75,6 +75,9 @@ struct FmStageNode {
   double x, beta;
 };
 
+struct FmThinDesc;  // gemm_thin.hpp
+struct FmThinArgs;
+
 struct FmStageArgs {
   FmBases bases;
   const FmOp* ops;
@@ -85,6 +88,9 @@ struct FmStageArgs {
   int32_t rows2, cols2;
   int64_t view_off;
   const FmStageNode* node;  // grouped launch: per-node descriptors (nullptr otherwise)
+  // one-level W stage of one problem: node q also adds the product upd[q] of
+  // its peeled K columns (nullptr: none)
+  const FmThinDesc* upd;
 };
 
 // The placement of node q of a stage launch, uniform or grouped.  nout: output
@@ -130,6 +136,9 @@ __host__ __device__ __forceinline__ FmNodeView fm_node_view(const FmStageArgs& a
 }
 
 typedef hipError_t (*FmStageLaunch)(const FmStageArgs& a, hipStream_t s);
+// launches that share a grid: S and T; W and the peeled strips of C
+typedef hipError_t (*FmStagePairLaunch)(const FmStageArgs& a, const FmStageArgs& b, hipStream_t s);
+typedef hipError_t (*FmStageStripLaunch)(const FmStageArgs& a, const FmThinArgs& t, hipStream_t s);
 
 struct FmAlgDesc {
   const char* name;
@@ -157,6 +166,9 @@ struct FmAlgDesc {
   // two-level S/T stages of FP32 data writing the leaves' split-bf16 slice
   // planes (nullptr where s2_f / t2_f are)
   FmStageLaunch s2p_f, t2p_f;
+  // small problems: S and T in one launch, W and the peeled strips in one
+  FmStagePairLaunch st_d, st_f;
+  FmStageStripLaunch ws_d, ws_f;
 };
 
 // generated registry (csrc/gen/registry.cpp): one accessor per algorithm

@@ -270,11 +270,22 @@ fm_status timed(hipStream_t s, float* ms_out, std::unique_lock<std::mutex>& lock
 // Workspace for a plan: the caller's buffer if given, else the arena.
 // Algorithmic HBM bytes of one launch: every source element read once,
 // every output written once (the minimum any schedule of that launch needs).
-double launch_bytes(const Launch& L, double es) {
+// A shared launch (S and T, W and strips) counts under both its kinds.
+double launch_bytes(const Launch& L, double es, int stage) {
   const FmAlgDesc* g = L.alg;
+  if (stage != L.stage) {  // the second kind of a shared launch
+    if (L.kind == LK_ST) return es * L.st2.nodes * L.st2.rows * L.st2.cols * (g->k * g->n + g->nt);
+    double b = 0;
+    for (size_t i = (size_t)L.nupd; i < L.tdescs.size(); ++i) {
+      const FmThinDesc& d = L.tdescs[i];
+      b += es * ((double)d.M * d.K + (double)d.K * d.N + (double)d.M * d.N * (d.beta != 0.0 ? 2 : 1));
+    }
+    return b;
+  }
   const double nodes = L.st.nodes;
   switch (L.kind) {
     case LK_S:
+    case LK_ST:
       return es * nodes * L.st.rows * L.st.cols * (g->m * g->k + g->ns);
     case LK_T:
       return es * nodes * L.st.rows * L.st.cols * (g->k * g->n + g->nt);
@@ -289,6 +300,7 @@ double launch_bytes(const Launch& L, double es) {
       return (double)nodes * L.st.rows2 * L.st.cols2 * (es * nb * nb + (L.planes ? 6.0 : es) * outs);
     }
     case LK_W:
+    case LK_WS:
       return es * nodes * L.st.rows * L.st.cols *
              (g->R + g->m * g->n * (L.st.beta != 0.0 ? 2.0 : 1.0));
     case LK_W2: {
@@ -626,7 +638,12 @@ fm_status fm_plan_query(const char* alg_name, fm_dtype dtype, fm_mode mode, int 
   const double es = elem_size(dtype);
   for (const Launch& L : P.launches) {
     info->launches[L.stage] += 1;
-    info->stage_bytes[L.stage] += launch_bytes(L, es);
+    info->stage_bytes[L.stage] += launch_bytes(L, es, L.stage);
+    if (L.kind == LK_ST || L.kind == LK_WS) {
+      const int second = L.kind == LK_ST ? FM_STAGE_T : FM_STAGE_PEEL;
+      info->launches[second] += 1;
+      info->stage_bytes[second] += launch_bytes(L, es, second);
+    }
     if (L.kind == LK_S2 || L.kind == LK_T2 || L.kind == LK_W2) info->two_level_stages += 1;
     if (L.kind == LK_SPLIT)
       for (const FmSplitPrep& r : L.spreps)

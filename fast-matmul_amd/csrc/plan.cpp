@@ -922,6 +922,8 @@ fm_status check_stage_size(const Launch& L) {
   if (L.kind == LK_GEMM || L.kind == LK_OZAKI || L.kind == LK_SPLIT || L.kind == LK_THIN ||
       L.kind == LK_NONE)
     return FM_OK;
+  if (L.kind == LK_ST && (int64_t)L.st2.rows * L.st2.cols >= (int64_t(1) << 31))
+    return set_err(FM_ERR_SHAPE, "a recursion block exceeds the stage kernels' 2^31 element limit; use more steps");
   const bool two = L.kind == LK_S2 || L.kind == LK_T2 || L.kind == LK_W2;
   const int64_t elems = two ? (int64_t)L.st.rows2 * L.st.cols2 : (int64_t)L.st.rows * L.st.cols;
   if (elems >= (int64_t(1) << 31))
@@ -1026,6 +1028,71 @@ void group_sequence(std::vector<std::vector<Launch>*> seqs, std::vector<Launch>&
 }
 }  // namespace
 
+namespace {
+// Stages that move less than this run two to a launch (fm_st_stage, fm_w_strips,
+// one element a lane): a launch of its own costs about 3 us, which these bytes
+// no longer hide.  Measured, one level, whole call, apart -> together in us:
+// strassen FP64 257^3 (2.4 MB of S and T) 22.6 -> 18.0, 801^3 (23 MB) 49.9 ->
+// 43.6, 1201^3 (52 MB; W 32 MB) 96.7 -> 95.0, 1501^3 (81 MB; W 50 MB) 144.3 ->
+// 145.3; grey522 FP64 1201^3 (63 MB; W 32 MB) 99.8 -> 92.0; smirnov333 FP32
+// 1501^3 (52 MB; W 32 MB) 97.8 -> 91.0.
+const double kSmallPairBytes = 64e6;  // S and T
+const double kSmallWBytes = 40e6;     // W; the strips beside it likewise
+
+double stage_bytes1(const Launch& L, fm_dtype dt) {  // one-level stages
+  const FmAlgDesc* g = L.alg;
+  const int slabs = L.kind == LK_S ? g->m * g->k + g->ns : L.kind == LK_T ? g->k * g->n + g->nt : g->R + g->m * g->n;
+  return (double)elem_size(dt) * L.st.nodes * L.st.rows * L.st.cols * slabs;
+}
+
+// Append one problem's S/T stages, adjacent small S and T as one launch.
+void append_pre(std::vector<Launch>& pre, std::vector<Launch>& out, fm_dtype dt) {
+  for (size_t i = 0; i < pre.size(); ++i) {
+    if (i + 1 < pre.size() && pre[i].kind == LK_S && pre[i + 1].kind == LK_T && pre[i].alg == pre[i + 1].alg &&
+        stage_bytes1(pre[i], dt) + stage_bytes1(pre[i + 1], dt) <= kSmallPairBytes) {
+      Launch L = std::move(pre[i]);
+      Launch& T = pre[++i];
+      L.kind = LK_ST;
+      L.st2 = T.st;
+      L.ops.insert(L.ops.end(), T.ops.begin(), T.ops.end());
+      out.push_back(std::move(L));
+    } else {
+      out.push_back(std::move(pre[i]));
+    }
+  }
+}
+
+// Append one problem's W stage of a level and the level's peeling products: a
+// one-level W stage adds the K remainders itself, and takes the strips into its
+// launch where both are small.
+void append_w(Launch W, std::vector<FmThinDesc> peel, std::vector<Launch>& out, fm_dtype dt) {
+  std::vector<FmThinDesc> strips;
+  if (W.kind == LK_W) {
+    for (const FmThinDesc& d : peel)
+      if (d.kind == FM_THIN_K) W.tdescs.push_back(d);
+    W.nupd = (int)W.tdescs.size();  // one per node, in node order, or none
+  }
+  for (const FmThinDesc& d : peel)
+    if (W.kind != LK_W || d.kind != FM_THIN_K) strips.push_back(d);
+  if (strips.empty()) {
+    out.push_back(std::move(W));
+    return;
+  }
+  Launch T = thin_launch(std::move(strips), dt);
+  double bytes = 0;
+  for (const FmThinDesc& d : T.tdescs) bytes += (double)elem_size(dt) * ((double)d.M * d.K + (double)d.K * d.N);
+  if (W.kind == LK_W && T.th.uniform && bytes <= kSmallWBytes && stage_bytes1(W, dt) <= kSmallWBytes) {
+    W.kind = LK_WS;
+    W.th = T.th;
+    W.tdescs.insert(W.tdescs.end(), T.tdescs.begin(), T.tdescs.end());
+    out.push_back(std::move(W));
+  } else {
+    out.push_back(std::move(W));
+    out.push_back(std::move(T));
+  }
+}
+}  // namespace
+
 fm_status assemble(Plan& P, std::vector<SubPlan>& subs, int64_t ws_elems, int persistent_grid) {
   for (SubPlan& s : subs) {
     for (const Launch& L : s.pre) {
@@ -1043,8 +1110,7 @@ fm_status assemble(Plan& P, std::vector<SubPlan>& subs, int64_t ws_elems, int pe
     for (SubPlan& s : subs) seqs.push_back(&s.pre);
     group_sequence(seqs, P.launches, P.dtype);
   } else {
-    for (SubPlan& s : subs)
-      for (Launch& L : s.pre) P.launches.push_back(std::move(L));
+    for (SubPlan& s : subs) append_pre(s.pre, P.launches, P.dtype);
   }
   std::vector<FmGemmDesc> leaves;
   for (SubPlan& s : subs) leaves.insert(leaves.end(), s.leaves.begin(), s.leaves.end());
@@ -1113,6 +1179,9 @@ fm_status assemble(Plan& P, std::vector<SubPlan>& subs, int64_t ws_elems, int pe
         seqs.push_back(&one[i]);
       }
       group_sequence(seqs, P.launches, P.dtype);
+    } else if (wl.size() == 1 && subs.size() == 1) {
+      append_w(std::move(wl[0]), std::move(peel), P.launches, P.dtype);
+      continue;
     } else {
       for (Launch& L : wl) P.launches.push_back(std::move(L));
     }
@@ -1149,8 +1218,10 @@ void Plan::pack(std::vector<char>& buf) {
       L.dev_off2 = put(L.spreps.data(), L.spreps.size() * sizeof(FmSplitPrep));
     } else if (!L.snodes.empty())
       L.dev_off = put(L.snodes.data(), L.snodes.size() * sizeof(FmStageNode));
-    else
+    else {
       L.dev_off = put(L.ops.data(), L.ops.size() * sizeof(FmOp));
+      if (!L.tdescs.empty()) L.dev_off2 = put(L.tdescs.data(), L.tdescs.size() * sizeof(FmThinDesc));
+    }
   }
   ext_off = put(ext.data(), ext.size() * sizeof(void*));
 }
@@ -1175,6 +1246,13 @@ void Plan::bind(void* dev) {
     } else {
       L.st.ops = reinterpret_cast<const FmOp*>(p);
       L.st.node = nullptr;
+      if (L.kind == LK_ST) {
+        L.st2.ops = L.st.ops + L.st.nodes;
+        L.st2.node = nullptr;
+      }
+      const FmThinDesc* t = reinterpret_cast<const FmThinDesc*>((char*)dev + L.dev_off2);
+      L.st.upd = L.nupd > 0 ? t : nullptr;
+      L.th.descs = t + L.nupd;
     }
   }
 }
@@ -1199,6 +1277,7 @@ namespace {
 struct ProfRec {
   int stage;
   hipEvent_t e0, e1;
+  int second = -1;  // the other stage of a shared launch: counted, its time is stage's
 };
 std::vector<ProfRec> g_prof_pending;
 std::vector<hipEvent_t> g_event_pool;
@@ -1227,6 +1306,7 @@ fm_status profile_read(fm_profile* out) {
     if (e != hipSuccess && st == FM_OK) st = hip_err(e, "profile event");
     g_prof_acc.ms[r.stage] += ms;
     g_prof_acc.launches[r.stage] += 1;
+    if (r.second >= 0) g_prof_acc.launches[r.second] += 1;
     g_event_pool.push_back(r.e0);
     g_event_pool.push_back(r.e1);
   }
@@ -1249,6 +1329,8 @@ fm_status Plan::run(const void* A, const void* B, void* C, void* ws, hipStream_t
   for (const Launch& L : launches) {
     hipError_t e = hipSuccess;
     ProfRec pr{L.stage, nullptr, nullptr};
+    if (L.kind == LK_ST) pr.second = FM_STAGE_T;
+    if (L.kind == LK_WS) pr.second = FM_STAGE_PEEL;
     if (g_prof_on) {
       pr.e0 = pool_event();
       pr.e1 = pool_event();
@@ -1292,6 +1374,15 @@ fm_status Plan::run(const void* A, const void* B, void* C, void* ws, hipStream_t
         e = fm_gemm_launch_bf16x3(L.cfg, g, s);
       else
         e = dtype == FM_F64 ? fm_gemm_launch_f64(L.cfg, g, s) : fm_gemm_launch_f32(L.cfg, g, s);
+    } else if (L.kind == LK_ST) {
+      FmStageArgs a = L.st, b = L.st2;
+      a.bases = b.bases = bases;
+      e = (dtype == FM_F64 ? L.alg->st_d : L.alg->st_f)(a, b, s);
+    } else if (L.kind == LK_WS) {
+      FmStageArgs a = L.st;
+      FmThinArgs t = L.th;
+      a.bases = t.bases = bases;
+      e = (dtype == FM_F64 ? L.alg->ws_d : L.alg->ws_f)(a, t, s);
     } else {
       FmStageArgs a = L.st;
       a.bases = bases;

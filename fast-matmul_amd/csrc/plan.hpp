@@ -20,8 +20,11 @@ fm_status hip_err(hipError_t e, const char* what);
 const std::string& last_error();
 void clear_error();
 
-enum LaunchKind { LK_S, LK_T, LK_W, LK_GEMM, LK_OZAKI, LK_S2, LK_T2, LK_W2, LK_SPLIT, LK_THIN, LK_NONE };
+enum LaunchKind { LK_S, LK_T, LK_W, LK_GEMM, LK_OZAKI, LK_S2, LK_T2, LK_W2, LK_SPLIT, LK_THIN, LK_ST, LK_WS, LK_NONE };
 
+// LK_THIN: peeling products.  LK_ST: the S and T stages of one level (st, st2) in
+// one launch.  LK_WS: a W stage and its level's peeled strips in one launch.
+//
 // One kernel launch.  Descriptors stay on the host until Plan::upload packs
 // them into the plan's device buffer.
 struct Launch {
@@ -29,6 +32,7 @@ struct Launch {
   int stage = 0;                   // fm_stage_kind, for profiling
   const FmAlgDesc* alg = nullptr;  // stage launches: whose combine functions
   FmStageArgs st{};
+  FmStageArgs st2{};  // LK_ST: T (its operands follow S's in ops)
   FmGemmArgs gm{};
   FmOzakiArgs oz{};
   FmSplitArgs sp{};
@@ -43,7 +47,10 @@ struct Launch {
   std::vector<FmOzakiDesc> odescs;
   std::vector<FmSplitDesc> sdescs;
   std::vector<FmSplitPrep> spreps;
+  // peeling products; W stages: first the K updates the stage adds itself
+  // (nupd, one per node), then the strips of LK_WS
   std::vector<FmThinDesc> tdescs;
+  int nupd = 0;
   size_t dev_off = 0, dev_off2 = 0;
 };
 

@@ -19,6 +19,7 @@
 #include <type_traits>
 
 #include "alg_desc.hpp"
+#include "gemm_thin_dev.hpp"
 #include "gmem.hpp"
 #include "split_bf16.hpp"
 
@@ -66,14 +67,14 @@ __device__ __forceinline__ void fm_store(fm_gptr<T> p, const FmVec<T, VEC>& r) {
 constexpr int FM_STAGE_THREADS = 256;
 
 // SIDE 0: A operand (m x k blocks, U/SX, outputs S); SIDE 1: B (k x n, V/TX, T).
+// Node q, work group bx of the node's nbx.
 template <class Cmb, typename T, int VEC, int SIDE>
-__global__ void __launch_bounds__(FM_STAGE_THREADS) fm_in_stage(FmStageArgs a) {
+__device__ __forceinline__ void fm_in_body(const FmStageArgs& a, int q, uint32_t bx, uint32_t nbx) {
   constexpr int BR = SIDE == 0 ? Cmb::m : Cmb::k;
   constexpr int BC = SIDE == 0 ? Cmb::k : Cmb::n;
   constexpr int NB = BR * BC;
   constexpr int NOUT = SIDE == 0 ? Cmb::NS : Cmb::NT;
   constexpr int NOUT_ARR = NOUT > 0 ? NOUT : 1;
-  const int q = blockIdx.y;
   const FmNodeView nv = fm_node_view(a, q, NOUT, 0);
   const FmOp op = nv.op;
   const fm_gptr<const T> src = fm_global(reinterpret_cast<const T*>(fm_base(a.bases, op.role)) + op.off);
@@ -82,8 +83,7 @@ __global__ void __launch_bounds__(FM_STAGE_THREADS) fm_in_stage(FmStageArgs a) {
   const uint32_t total = rv * (uint32_t)nv.cols;
   const int64_t ld = op.ld, rows = nv.rows, cols = nv.cols, out_ld = nv.out_ld, slab = nv.out_slab;
   const double x = nv.x;
-  for (uint32_t e = blockIdx.x * FM_STAGE_THREADS + threadIdx.x; e < total;
-       e += gridDim.x * FM_STAGE_THREADS) {
+  for (uint32_t e = bx * FM_STAGE_THREADS + threadIdx.x; e < total; e += nbx * FM_STAGE_THREADS) {
     const uint32_t j = e / rv;
     const uint32_t i = (e - j * rv) * VEC;
     FmVec<T, VEC> v[NB];
@@ -112,13 +112,36 @@ __global__ void __launch_bounds__(FM_STAGE_THREADS) fm_in_stage(FmStageArgs a) {
   }
 }
 
+template <class Cmb, typename T, int VEC, int SIDE>
+__global__ void __launch_bounds__(FM_STAGE_THREADS) fm_in_stage(FmStageArgs a) {
+  fm_in_body<Cmb, T, VEC, SIDE>(a, blockIdx.y, blockIdx.x, gridDim.x);
+}
+
+// S and T of a small problem in one launch (the first gs * a.nodes work groups
+// are S's): the two read different matrices, and a launch of its own costs
+// each about 3 us whatever it does.
+template <class Cmb, typename T>
+__global__ void __launch_bounds__(FM_STAGE_THREADS) fm_st_stage(FmStageArgs a, FmStageArgs b, uint32_t gs,
+                                                                uint32_t gt) {
+  const uint32_t w = blockIdx.x, ns = gs * (uint32_t)a.nodes;
+  if (w < ns)
+    fm_in_body<Cmb, T, 1, 0>(a, w / gs, w % gs, gs);
+  else
+    fm_in_body<Cmb, T, 1, 1>(b, (w - ns) / gt, (w - ns) % gt, gt);
+}
+
 // C_ij (+)= sum_q W[ij, q] M_q for every node; M_q of node q at
 // ws + out_off + (q * R + r) * out_slab.
-template <class Cmb, typename T, int VEC, bool BETA>
-__global__ void __launch_bounds__(FM_STAGE_THREADS) fm_w_stage(FmStageArgs a) {
+//
+// UPD: the node's K remainder (its peeled last columns of A times the peeled
+// last rows of B, linalg/linalg.hpp:214-221) is added in the same pass, in the
+// roundings of fm_thin_kernel's update, which reads and writes all of C once
+// more (grey333_23_152 two levels 4009 x 2800 x 2489 FP64: W and peeling
+// 416 -> 358 us).
+template <class Cmb, typename T, int VEC, bool BETA, bool UPD>
+__device__ __forceinline__ void fm_w_body(const FmStageArgs& a, int q, uint32_t bx, uint32_t nbx) {
   constexpr int R = Cmb::R;
   constexpr int MN = Cmb::m * Cmb::n;
-  const int q = blockIdx.y;
   const FmNodeView nv = fm_node_view(a, q, R, 0);
   const FmOp op = nv.op;
   const fm_gptr<T> c = fm_global(reinterpret_cast<T*>(fm_base(a.bases, op.role)) + op.off);
@@ -128,8 +151,15 @@ __global__ void __launch_bounds__(FM_STAGE_THREADS) fm_w_stage(FmStageArgs a) {
   const int64_t ld = op.ld, rows = nv.rows, cols = nv.cols, out_ld = nv.out_ld, slab = nv.out_slab;
   const T beta = (T)nv.beta;
   const double x = nv.x;
-  for (uint32_t e = blockIdx.x * FM_STAGE_THREADS + threadIdx.x; e < total;
-       e += gridDim.x * FM_STAGE_THREADS) {
+  constexpr int KM = Cmb::k > 1 ? Cmb::k - 1 : 1;  // largest remainder of K
+  FmThinDesc u;
+  fm_gptr<const T> ua = nullptr, ub = nullptr;
+  if constexpr (UPD) {
+    u = a.upd[q];
+    ua = fm_global(reinterpret_cast<const T*>(fm_base(a.bases, u.a.role)) + u.a.off);
+    ub = fm_global(reinterpret_cast<const T*>(fm_base(a.bases, u.b.role)) + u.b.off);
+  }
+  for (uint32_t e = bx * FM_STAGE_THREADS + threadIdx.x; e < total; e += nbx * FM_STAGE_THREADS) {
     const uint32_t j = e / rv;
     const uint32_t i = (e - j * rv) * VEC;
     FmVec<T, VEC> mv[R];
@@ -147,6 +177,36 @@ __global__ void __launch_bounds__(FM_STAGE_THREADS) fm_w_stage(FmStageArgs a) {
 #pragma unroll
       for (int t = 0; t < MN; ++t) o[t].v[l] = out[t];
     }
+    FmVec<T, VEC> up[UPD ? MN : 1];
+    if constexpr (UPD) {
+      T av[Cmb::m][KM][VEC], bv[Cmb::n][KM];
+#pragma unroll
+      for (int k = 0; k < KM; ++k) {
+        const int kk = min(k, u.K - 1);  // past the remainder: loaded, not used
+#pragma unroll
+        for (int bi = 0; bi < Cmb::m; ++bi) {
+          typedef T vt __attribute__((ext_vector_type(VEC))) __attribute__((aligned(sizeof(T))));
+          const vt x = *(fm_gptr<const vt>)(ua + (int64_t)bi * rows + i + kk * u.a.ld);
+          if constexpr (VEC == 1) {
+            av[bi][k][0] = x[0];
+          } else {
+#pragma unroll
+            for (int l = 0; l < VEC; ++l) av[bi][k][l] = x[l];
+          }
+        }
+#pragma unroll
+        for (int bj = 0; bj < Cmb::n; ++bj) bv[bj][k] = ub[kk + ((int64_t)bj * cols + j) * u.b.ld];
+      }
+#pragma unroll
+      for (int t = 0; t < MN; ++t)
+#pragma unroll
+        for (int l = 0; l < VEC; ++l) {
+          T s = T(0);
+#pragma unroll
+          for (int k = 0; k < KM; ++k) s = k < u.K ? fma(av[t / Cmb::n][k][l], bv[t % Cmb::n][k], s) : s;
+          up[t].v[l] = fm_mul((T)u.alpha, s);
+        }
+    }
 #pragma unroll
     for (int t = 0; t < MN; ++t) {
       const int bi = t / Cmb::n, bj = t % Cmb::n;
@@ -156,9 +216,45 @@ __global__ void __launch_bounds__(FM_STAGE_THREADS) fm_w_stage(FmStageArgs a) {
 #pragma unroll
         for (int l = 0; l < VEC; ++l) o[t].v[l] = fm_add(o[t].v[l], fm_mul(beta, old.v[l]));
       }
+      if constexpr (UPD) {
+#pragma unroll
+        for (int l = 0; l < VEC; ++l) o[t].v[l] = fm_add(o[t].v[l], up[t].v[l]);
+      }
       fm_store<T, VEC>(p, o[t]);
     }
   }
+}
+
+template <class Cmb, typename T, int VEC, bool BETA, bool UPD>
+__global__ void __launch_bounds__(FM_STAGE_THREADS) fm_w_stage(FmStageArgs a) {
+  fm_w_body<Cmb, T, VEC, BETA, UPD>(a, blockIdx.y, blockIdx.x, gridDim.x);
+}
+
+// W and the peeled strips of C of a small problem in one launch: the strips
+// (linalg/linalg.hpp:222-243) read only A and B and write the rows and columns
+// of C that W does not, so they need no launch after it.  The first
+// gw * a.nodes work groups are W's.
+template <class Cmb, typename T, bool BETA, bool UPD>
+__global__ void __launch_bounds__(FM_STAGE_THREADS) fm_w_strips(FmStageArgs a, FmThinArgs p, uint32_t gw) {
+  static_assert(FM_STAGE_THREADS == FM_THIN_THREADS, "one work group size");
+  constexpr int NM = Cmb::n > 1 ? Cmb::n - 1 : 1, MM = Cmb::m > 1 ? Cmb::m - 1 : 1;
+  __shared__ T red[NM * FM_THIN_THREADS];
+  const uint32_t w = blockIdx.x, nw = gw * (uint32_t)a.nodes;
+  if (w < nw) {
+    fm_w_body<Cmb, T, 1, BETA, UPD>(a, w / gw, w % gw, gw);
+    return;
+  }
+  const int t = (int)(w - nw);
+  const int kind = t >= p.t0[FM_THIN_M] ? FM_THIN_M : FM_THIN_N;
+  const FmThinDesc d = p.descs[p.d0[kind] + (t - p.t0[kind]) / p.per[kind]];
+  const int local = t - d.tile_begin, tn = local / d.tiles_m, tm = local - tn * d.tiles_m;
+  const fm_gptr<const T> A = fm_global(reinterpret_cast<const T*>(fm_base(p.bases, d.a.role)) + d.a.off);
+  const fm_gptr<const T> B = fm_global(reinterpret_cast<const T*>(fm_base(p.bases, d.b.role)) + d.b.off);
+  const fm_gptr<T> C = fm_global(reinterpret_cast<T*>(fm_base(p.bases, d.c.role)) + d.c.off);
+  if (kind == FM_THIN_N)
+    fm_thin::thin_dispatch<NM>(d.N, [&](auto v) { fm_thin::thin_n<T, decltype(v)::value>(d, tm, A, B, C, red); });
+  else
+    fm_thin::thin_dispatch<MM>(d.M, [&](auto v) { fm_thin::thin_m<T, decltype(v)::value>(d, tn, A, B, C); });
 }
 
 // Compile-time loop: f(std::integral_constant<int, I>) for I = B .. E-1.
@@ -547,25 +643,49 @@ hipError_t fm_launch_in_stage(const FmStageArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
+// f(beta, upd) as compile-time flags
+template <class F>
+void fm_w_flags(const FmStageArgs& a, F&& f) {
+  const std::true_type yes;
+  const std::false_type no;
+  if (a.beta != 0.0) {
+    if (a.upd) f(yes, yes);
+    else f(yes, no);
+  } else {
+    if (a.upd) f(no, yes);
+    else f(no, no);
+  }
+}
+
 template <class Cmb, typename T>
 hipError_t fm_launch_w_stage(const FmStageArgs& a, hipStream_t s) {
   constexpr int VMAX = sizeof(T) == 8 ? 2 : 4;
-  const bool beta = a.beta != 0.0;
-  if (a.vec == VMAX) {
-    if (beta)
-      hipLaunchKernelGGL((fm_w_stage<Cmb, T, VMAX, true>), fm_stage_grid(a, VMAX),
-                         dim3(FM_STAGE_THREADS), 0, s, a);
+  fm_w_flags(a, [&](auto beta, auto upd) {
+    constexpr bool B = decltype(beta)::value, U = decltype(upd)::value;
+    if (a.vec == VMAX)
+      hipLaunchKernelGGL((fm_w_stage<Cmb, T, VMAX, B, U>), fm_stage_grid(a, VMAX), dim3(FM_STAGE_THREADS), 0, s, a);
     else
-      hipLaunchKernelGGL((fm_w_stage<Cmb, T, VMAX, false>), fm_stage_grid(a, VMAX),
-                         dim3(FM_STAGE_THREADS), 0, s, a);
-  } else {
-    if (beta)
-      hipLaunchKernelGGL((fm_w_stage<Cmb, T, 1, true>), fm_stage_grid(a, 1),
-                         dim3(FM_STAGE_THREADS), 0, s, a);
-    else
-      hipLaunchKernelGGL((fm_w_stage<Cmb, T, 1, false>), fm_stage_grid(a, 1),
-                         dim3(FM_STAGE_THREADS), 0, s, a);
-  }
+      hipLaunchKernelGGL((fm_w_stage<Cmb, T, 1, B, U>), fm_stage_grid(a, 1), dim3(FM_STAGE_THREADS), 0, s, a);
+  });
+  return hipGetLastError();
+}
+
+template <class Cmb, typename T>
+hipError_t fm_launch_st_stage(const FmStageArgs& a, const FmStageArgs& b, hipStream_t s) {
+  const uint32_t gs = fm_stage_grid(a, 1).x, gt = fm_stage_grid(b, 1).x;
+  hipLaunchKernelGGL((fm_st_stage<Cmb, T>), dim3(gs * (uint32_t)a.nodes + gt * (uint32_t)b.nodes),
+                     dim3(FM_STAGE_THREADS), 0, s, a, b, gs, gt);
+  return hipGetLastError();
+}
+
+template <class Cmb, typename T>
+hipError_t fm_launch_w_strips(const FmStageArgs& a, const FmThinArgs& t, hipStream_t s) {
+  const uint32_t gw = fm_stage_grid(a, 1).x;
+  fm_w_flags(a, [&](auto beta, auto upd) {
+    hipLaunchKernelGGL((fm_w_strips<Cmb, T, decltype(beta)::value, decltype(upd)::value>),
+                       dim3(gw * (uint32_t)a.nodes + (uint32_t)t.total_tiles), dim3(FM_STAGE_THREADS), 0, s, a, t,
+                       gw);
+  });
   return hipGetLastError();
 }
 
@@ -682,6 +802,8 @@ constexpr FmStageLaunch fm_stage2_planes_fn() {
         GNS::Combine::a_nviews, GNS::Combine::b_nviews, GNS::Combine::a_view_slot,            \
         GNS::Combine::b_view_slot, fm_w2_fn<GNS::Combine, double>(),                          \
         fm_w2_fn<GNS::Combine, float>(), fm_stage2_planes_fn<GNS::Combine, 0>(),             \
-        fm_stage2_planes_fn<GNS::Combine, 1>()};                                             \
+        fm_stage2_planes_fn<GNS::Combine, 1>(), &fm_launch_st_stage<GNS::Combine, double>,   \
+        &fm_launch_st_stage<GNS::Combine, float>, &fm_launch_w_strips<GNS::Combine, double>, \
+        &fm_launch_w_strips<GNS::Combine, float>};                                           \
     return &d;                                                                               \
   }

@@ -223,7 +223,8 @@ const char* fm_last_error(void);
 
 /* Per-stage timing.  While enabled, every launch fm_fastmatmul/fm_gemm
  * issues is bracketed by HIP events on the caller's stream (the stream the
- * kernels run on); fm_profile_read waits for them, returns the accumulated
+ * kernels run on; a launch that S and T, or W and peeling, share is counted for
+ * both and timed as S, or W); fm_profile_read waits for them, returns the accumulated
  * device time and launch count per stage kind and resets the counters. */
 typedef enum {
   FM_STAGE_S = 0,     /* S_r = sum U A      (HBM-bound)                     */
@@ -304,7 +305,8 @@ fm_status fm_scaled_workspace_query(const char* alg, fm_dtype dtype, fm_mode mod
  * first two leaf launches' tile configuration (-1: int8-digit leaves),
  * product and tile counts. */
 typedef struct fm_plan_info {
-  int launches[5];       /* FM_STAGE_S .. FM_STAGE_PEEL (preparation counts with LEAF) */
+  int launches[5];       /* FM_STAGE_S .. FM_STAGE_PEEL (preparation counts with LEAF; a
+                            launch that two stages share counts for both) */
   double stage_bytes[5];
   int two_level_stages;
   int leaf_cfg[2];

@@ -57,6 +57,37 @@ def test_tile_edges(fm, shape, dtype):
         _check(fm, "strassen", *shape, dtype, alpha, beta, sum(shape))
 
 
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("alg,shape", [
+    ("strassen", (2056, 1027, 2052)),             # K remainder alone, 16-byte rows in the W stage
+    ("grey522_18_99", (2063, 1027, 2051)),        # every remainder, odd rows
+    ("smirnov363_40_960", (1230, 1025, 1231)),    # K remainder of 5
+])
+def test_k_remainder_in_the_w_stage_of_larger_products(fm, alg, shape, dtype):
+    """Above the size where W shares its launch with the strips."""
+    for alpha, beta in [(1.0, 0.0), (2.0, -3.0)]:
+        _check(fm, alg, *shape, dtype, alpha, beta, 5)
+
+
+def test_stages_apart_and_together_give_the_same_bits(fm):
+    """One problem's S and T, and W, K remainder and strips, share launches
+    where small; a batch of two problems runs each stage and the peeling
+    apart."""
+    rng = np.random.default_rng(11)
+    dev = lambda x: fm.col_major(torch.from_numpy(np.asfortranarray(x)).to(DEV))  # noqa: E731
+    for alg, steps, (m, k, n) in [("strassen", 2, (259, 262, 133)), ("grey424_26_206", 1, (403, 205, 303)),
+                                  ("grey333_23_152", 2, (190, 187, 185)), ("smirnov633_40_960", 1, (131, 65, 98)),
+                                  ("strassen", 1, (4099, 515, 1030))]:
+        for dt in (np.float64, np.float32):
+            A, B, C0 = (dev((rng.random(s) * 2 - 1).astype(dt)) for s in ((m, k), (k, n), (m, n)))
+            one = fm.fastmatmul(alg, A, B, C0.clone(), steps, alpha=1.5, beta=0.5)
+            probs = [{"A": A, "B": B, "C": C0.clone(), "alg": alg, "num_steps": steps, "alpha": 1.5, "beta": 0.5}
+                     for _ in range(2)]
+            fm.Batch(probs, graph=False).run()
+            torch.cuda.synchronize()
+            assert torch.equal(one, probs[0]["C"]) and torch.equal(one, probs[1]["C"]), (alg, dt)
+
+
 def test_peeling_in_a_batch_of_unequal_problems(fm):
     """Products of several shapes in one launch (found by the search, not by
     division), each equal to its own call bit for bit."""
