@@ -71,13 +71,24 @@ __global__ void __launch_bounds__(64 * WM * WN, MINW) fm_gemm_kernel(FmGemmArgs 
   constexpr int NT = 64 * WM * WN;
   constexpr int WTM = BM / WM, WTN = BN / WN;
   constexpr int TM = WTM / 16, TN = WTN / 16;
-  constexpr int BKP = BK + 1;
   // scalar (edge) load mapping
   constexpr int A_PER = BM * BK / NT, B_PER = BK * BN / NT;
   constexpr int A_KSTEP = NT / BM;  // k columns covered by one pass of the A tile
   constexpr int B_NSTEP = NT / BK;  // n columns covered by one pass of the B tile
   // 16-byte (interior) load mapping: VL consecutive elements per load
   constexpr int VL = 16 / sizeof(T);
+  // LDS strides of the spread loop.  An A fragment read takes 16 consecutive rows
+  // at 4 consecutive k: BM elements apart, these 4 runs lie on the same of the
+  // 64 banks, with 16 more on different ones (for the large tiles; the smaller
+  // would lose a resident work group to the larger array).  B columns VL longer
+  // than BK are still free of conflicts and keep 16-byte vectors aligned, so
+  // that they are stored whole: faster on the FP64 tiles 128 columns wide but
+  // for the square one, slower on the others.  8192 x 8192 x 4096, TFLOP/s
+  // before -> after: FP64 128 x 128 72.3 -> 72.9, 128 x 256 70.2 -> 71.7, 64 x 128 70.1
+  // -> 71.8; FP32 128 x 256 134.7 -> 135.9.
+  constexpr int APAD = PIPE == 3 && BM >= 128 && BN >= 128 ? 16 : 0;
+  constexpr bool BVEC = PIPE == 3 && sizeof(T) == 8 && BN >= 128 && BM != BN;
+  constexpr int BKP = BVEC ? BK + VL : BK + 1;
   constexpr bool CAN_VEC = A_PER % VL == 0 && B_PER % VL == 0 && BM % VL == 0 &&
                            BK % VL == 0 && (NT * VL) % BM == 0 && (NT * VL) % BK == 0;
   constexpr int AV_PER = CAN_VEC ? A_PER / VL : 1, BV_PER = CAN_VEC ? B_PER / VL : 1;
@@ -100,7 +111,7 @@ __global__ void __launch_bounds__(64 * WM * WN, MINW) fm_gemm_kernel(FmGemmArgs 
   // (70.8 -> 67.7 TFLOP/s), other FP64 tiles move within +-2%.
   constexpr bool GM = sizeof(T) == 4 || SPREAD;
 
-  __shared__ __align__(16) T As[2][BK][BM];
+  __shared__ __align__(16) T As[2][BK][BM + APAD];
   __shared__ __align__(16) T Bs[2][BN][BKP];
 
   // Persistent when the grid is smaller than the tile count: work group b
@@ -334,20 +345,24 @@ __global__ void __launch_bounds__(64 * WM * WN, MINW) fm_gemm_kernel(FmGemmArgs 
 #pragma unroll
       for (int i = 0; i < BV_PER; ++i)
         if (i % NS4 == q) {
-          if constexpr (TAIL) {
-            vec_t v;
+          vec_t v;
 #pragma unroll
-            for (int e = 0; e < VL; ++e) v[e] = rb[i * VL + e];
+          for (int e = 0; e < VL; ++e) v[e] = rb[i * VL + e];
+          if constexpr (TAIL) {
+            const vec_t x = v;
 #pragma unroll
             for (int e = 0; e < VL; ++e) {
-              T t = v[e];
+              T t = x[e];
 #pragma unroll
-              for (int j = e + 1; j < VL; ++j) t = tail && b_sh == j - e ? (T)v[j] : t;
-              Bs[buf][bv_col + i * BV_NSTEP][bv_k + e] = tail && bv_k + e >= kr ? T(0) : t;
+              for (int j = e + 1; j < VL; ++j) t = tail && b_sh == j - e ? (T)x[j] : t;
+              v[e] = tail && bv_k + e >= kr ? T(0) : t;
             }
+          }
+          if constexpr (BVEC) {
+            *reinterpret_cast<vec_t*>(&Bs[buf][bv_col + i * BV_NSTEP][bv_k]) = v;
           } else {
 #pragma unroll
-            for (int e = 0; e < VL; ++e) Bs[buf][bv_col + i * BV_NSTEP][bv_k + e] = rb[i * VL + e];
+            for (int e = 0; e < VL; ++e) Bs[buf][bv_col + i * BV_NSTEP][bv_k + e] = v[e];
           }
         }
     };

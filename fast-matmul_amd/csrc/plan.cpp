@@ -414,9 +414,9 @@ struct TileCand {
   double us_k, k0, lat_k;
 };
 const TileCand kF64Tiles[] = {
-    {FM_TILE_PS_128x128_O2, 0.1257, 30, 0},  {FM_TILE_PS_128x256_W8, 0.2560, 30, 0},
+    {FM_TILE_PS_128x128_O2, 0.1257, 30, 0},  {FM_TILE_PS_128x256_W8, 0.2520, 30, 0},
     {FM_TILE_PS_128x96_O2, 0.0960, 30, 0},   {FM_TILE_128x64, 0.0650, 34, 0},
-    {FM_TILE_64x128, 0.0655, 34, 0},         {FM_TILE_64x64, 0.0340, 32, 0.037},
+    {FM_TILE_64x128, 0.0645, 34, 0},         {FM_TILE_64x64, 0.0340, 32, 0.037},
     {FM_TILE_PS_32x32_K32, 0.0103, 50, 0.0129}};
 const TileCand kF32Tiles[] = {
     {FM_TILE_PS_128x256_W8, 0.1383, 44, 0}, {FM_TILE_PS_128x128_O2, 0.0695, 40, 0},
