@@ -4,7 +4,8 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <cstdio>
+#include <array>
+#include <cstdint>
 #include <cstring>
 #include <deque>
 #include <map>
@@ -36,8 +37,9 @@ namespace {
 // beta and x, so a caller that varies alpha from call to call would
 // otherwise grow it without end.  The oldest plan goes first.
 constexpr size_t kMaxPlans = 256;
-std::map<std::string, std::unique_ptr<Plan>> g_plans;
-std::deque<std::string> g_plan_order;
+typedef std::array<int64_t, 20> PlanKey;
+std::map<PlanKey, std::unique_ptr<Plan>> g_plans;
+std::deque<PlanKey> g_plan_order;
 struct Arena {
   void* p = nullptr;
   size_t bytes = 0;
@@ -47,16 +49,36 @@ struct Arena {
 // ordered by it, calls on different streams never share a workspace
 std::map<std::pair<int, hipStream_t>, Arena> g_arenas;
 
-std::string plan_key(int dev, const char* alg, int dt, int mode, int64_t m, int64_t k, int64_t n,
-                     int64_t lda, int64_t ldb, int64_t ldc, int steps, double x, double alpha,
-                     double beta, const fm_options& o) {
-  char buf[512];
-  snprintf(buf, sizeof(buf), "%d|%s|%d|%d|%d|%d|%d|%d|%zu|%d|%lld|%lld|%lld|%lld|%lld|%lld|%d|%a|%a|%a",
-           dev, alg ? alg : "<gemm>", dt, mode, mode == FM_MODE_OZAKI_INT8 ? o.ozaki_slices : 0,
-           o.stage_fusion, o.split_remainder != 0, o.dfs_levels, o.workspace_limit, o.gemm_tile,
-           (long long)m, (long long)k, (long long)n, (long long)lda, (long long)ldb,
-           (long long)ldc, steps, x, alpha, beta);
-  return buf;
+// Every argument and option a plan embeds, doubles by their bits.  (As words:
+// printed into a string, key and look-up took 1.6 us of a small call's 10 in
+// the library.)
+PlanKey plan_key(int dev, const FmAlgDesc* alg, int dt, int mode, int64_t m, int64_t k, int64_t n, int64_t lda,
+                 int64_t ldb, int64_t ldc, int steps, double x, double alpha, double beta, const fm_options& o) {
+  auto bits = [](double v) {
+    int64_t b;
+    memcpy(&b, &v, sizeof(b));
+    return b;
+  };
+  return PlanKey{dev,
+                 (int64_t)(intptr_t)alg,
+                 dt,
+                 mode,
+                 mode == FM_MODE_OZAKI_INT8 ? o.ozaki_slices : 0,
+                 o.stage_fusion,
+                 o.split_remainder != 0,
+                 o.dfs_levels,
+                 (int64_t)o.workspace_limit,
+                 o.gemm_tile,
+                 m,
+                 k,
+                 n,
+                 lda,
+                 ldb,
+                 ldc,
+                 steps,
+                 bits(x),
+                 bits(alpha),
+                 bits(beta)};
 }
 
 }  // namespace
@@ -151,14 +173,13 @@ fm_status fmplan::build_single(Plan& P, const FmAlgDesc* alg, fm_dtype dt, fm_mo
 
 namespace {
 
-fm_status get_plan(const char* alg_name, const FmAlgDesc* alg, fm_dtype dt, fm_mode mode, int m,
+fm_status get_plan(const FmAlgDesc* alg, fm_dtype dt, fm_mode mode, int m,
                    int k, int n, int64_t lda, int64_t ldb, int64_t ldc, int steps, double x,
                    double alpha, double beta, const fm_options& o, Plan** out) {
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return hip_err(e, "hipGetDevice");
-  const std::string key =
-      plan_key(dev, alg_name, dt, mode, m, k, n, lda, ldb, ldc, steps, x, alpha, beta, o);
+  const PlanKey key = plan_key(dev, alg, dt, mode, m, k, n, lda, ldb, ldc, steps, x, alpha, beta, o);
   auto it = g_plans.find(key);
   if (it != g_plans.end()) {
     *out = it->second.get();
@@ -381,7 +402,7 @@ fm_status fm_fastmatmul_ex(const char* alg_name, fm_dtype dtype, fm_mode mode, i
   std::unique_lock<std::mutex> lock(fm_api_mutex());
   const fm_options o = opts ? *opts : g_defaults;
   Plan* P = nullptr;
-  st = get_plan(alg_name, alg, dtype, mode, m, k, n, lda, ldb, ldc, num_steps, x, alpha, beta, o, &P);
+  st = get_plan(alg, dtype, mode, m, k, n, lda, ldb, ldc, num_steps, x, alpha, beta, o, &P);
   if (st != FM_OK) return st;
   void* ws = nullptr;
   const hipStream_t s = (hipStream_t)stream;
@@ -532,7 +553,7 @@ fm_status fm_fastmatmul_scaled(const char* alg_name, fm_dtype dtype, fm_mode mod
   // (beta = 0) or into a workspace temporary
   const bool temp = beta != 0.0;
   Plan* P = nullptr;
-  st = get_plan(alg_name, alg, dtype, mode, m, k, n, m, k, temp ? m : ldc, num_steps, x, 1.0, 0.0,
+  st = get_plan(alg, dtype, mode, m, k, n, m, k, temp ? m : ldc, num_steps, x, 1.0, 0.0,
                 g_defaults, &P);
   if (st != FM_OK) return st;
   const ScaledLayout lay = scaled_layout(P->ws_bytes, (size_t)elem_size(dtype), m, k, n, temp);
@@ -681,7 +702,7 @@ fm_status fm_gemm(fm_dtype dtype, fm_mode mode, int m, int k, int n, const void*
   if (k == 0) return set_err(FM_ERR_SHAPE, "k == 0");
   std::lock_guard<std::mutex> lock(fm_api_mutex());
   Plan* P = nullptr;
-  st = get_plan(nullptr, nullptr, dtype, mode, m, k, n, lda, ldb, ldc, 0, 0.0, alpha, beta, g_defaults,
+  st = get_plan(nullptr, dtype, mode, m, k, n, lda, ldb, ldc, 0, 0.0, alpha, beta, g_defaults,
                 &P);
   if (st != FM_OK) return st;
   void* ws = nullptr;

@@ -36,12 +36,12 @@ def algorithm_names():
 
 
 def _is_col_major(t: torch.Tensor) -> bool:
-    m, n = t.shape
+    (m, n), (rs, cs) = t.shape, t.stride()
     if m <= 1:  # one row: any column stride >= 1 is a valid leading dimension
-        return n <= 1 or t.stride(1) >= 1
+        return n <= 1 or cs >= 1
     if n <= 1:  # one column: rows must be contiguous
-        return t.stride(0) == 1
-    return t.stride(0) == 1 and t.stride(1) >= m
+        return rs == 1
+    return rs == 1 and cs >= m
 
 
 def _col_major(t: torch.Tensor, name: str) -> torch.Tensor:
@@ -68,12 +68,20 @@ def empty(m: int, n: int, dtype=torch.float64, device="cuda") -> torch.Tensor:
 def _ld(t: torch.Tensor) -> int:
     m, n = t.shape
     if n > 1:
-        return max(1, m, t.stride(1)) if m > 1 else max(1, t.stride(1))
+        ld = t.stride()[1]
+        return max(1, m, ld) if m > 1 else max(1, ld)
     return max(1, m)
 
 
+# The handle of the current stream without a Stream object around it (2.1 ->
+# 0.2 us a call, of the 16 us a small call's host side took).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream_handle(t: torch.Tensor):
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    if _raw_stream is not None:
+        return _raw_stream(t.get_device())
+    return torch.cuda.current_stream(t.device).cuda_stream
 
 
 def _operands(A: torch.Tensor, B: torch.Tensor, C: Optional[torch.Tensor], beta: float):
@@ -87,25 +95,26 @@ def _operands(A: torch.Tensor, B: torch.Tensor, C: Optional[torch.Tensor], beta:
     k2, n = B.shape
     if k2 != k:
         raise ValueError("inner dimensions differ: A is %d x %d, B is %d x %d" % (m, k, k2, n))
-    if A.dtype not in _DT:
-        raise TypeError("A must be float64 or float32, not %s" % A.dtype)
-    if B.dtype != A.dtype:
-        raise TypeError("B must have A's dtype %s, not %s" % (A.dtype, B.dtype))
+    dtype, device = A.dtype, A.device
+    if dtype not in _DT:
+        raise TypeError("A must be float64 or float32, not %s" % dtype)
+    if B.dtype != dtype:
+        raise TypeError("B must have A's dtype %s, not %s" % (dtype, B.dtype))
     if not A.is_cuda or not B.is_cuda:
         raise ValueError("A and B must be GPU tensors")
-    if B.device != A.device:
-        raise ValueError("A and B must be on one device (%s vs %s)" % (A.device, B.device))
+    if B.device != device:
+        raise ValueError("A and B must be on one device (%s vs %s)" % (device, B.device))
     if C is None:
         if beta != 0.0:
             raise ValueError("beta != 0 needs an input C")
-        C = empty(m, n, A.dtype, A.device)
+        C = empty(m, n, dtype, device)
     C = _col_major(C, "C")
     if tuple(C.shape) != (m, n):
         raise ValueError("C must be %d x %d, not %d x %d" % (m, n, C.shape[0], C.shape[1]))
-    if C.dtype != A.dtype:
-        raise TypeError("C must have A's dtype %s, not %s" % (A.dtype, C.dtype))
-    if not C.is_cuda or C.device != A.device:
-        raise ValueError("C must be a GPU tensor on A's device %s" % A.device)
+    if C.dtype != dtype:
+        raise TypeError("C must have A's dtype %s, not %s" % (dtype, C.dtype))
+    if C.device != device:
+        raise ValueError("C must be a GPU tensor on A's device %s" % device)
     return A, B, C, m, k, n
 
 
@@ -151,9 +160,8 @@ def fastmatmul(alg_name: str, A: torch.Tensor, B: torch.Tensor, C: Optional[torc
     A, B, C, m, k, n = _operands(A, B, C, beta)
     ws_ptr, ws_bytes = _workspace(workspace, A)
     ms = ctypes.c_float(0.0)
-    st = LIB.fm_fastmatmul_ex(alg_name.encode(), _DT[A.dtype], _lib.MODES[mode], m, k, n,
-                              ctypes.c_void_p(A.data_ptr()), _ld(A), ctypes.c_void_p(B.data_ptr()),
-                              _ld(B), ctypes.c_void_p(C.data_ptr()), _ld(C), int(num_steps),
+    st = LIB.fm_fastmatmul_ex(alg_name.encode(), _DT[A.dtype], _lib.MODES[mode], m, k, n, A.data_ptr(),
+                              _ld(A), B.data_ptr(), _ld(B), C.data_ptr(), _ld(C), int(num_steps),
                               float(x), float(alpha), float(beta), _options_ref(opts),
                               _stream_handle(A), ws_ptr, ws_bytes,
                               ctypes.byref(ms) if timed else None)
@@ -196,8 +204,7 @@ class Plan:
             raise ValueError("plan is for leading dimensions %s, not %s" % (self.lds, (_ld(A), _ld(B), _ld(C))))
         ws_ptr, ws_bytes = _workspace(workspace, A)
         ms = ctypes.c_float(0.0)
-        check(LIB.fm_plan_run(self._h, ctypes.c_void_p(A.data_ptr()), ctypes.c_void_p(B.data_ptr()),
-                              ctypes.c_void_p(C.data_ptr()), _stream_handle(A), ws_ptr, ws_bytes,
+        check(LIB.fm_plan_run(self._h, A.data_ptr(), B.data_ptr(), C.data_ptr(), _stream_handle(A), ws_ptr, ws_bytes,
                               ctypes.byref(ms) if timed else None))
         return (C, ms.value) if timed else C
 
