@@ -18,7 +18,8 @@ enum FmLeafPhase : int { FM_PHASE_PREP = 1, FM_PHASE_PRODUCT = 2, FM_PHASE_ALL =
 
 enum FmRole : int32_t { FM_ROLE_A = 0, FM_ROLE_B = 1, FM_ROLE_C = 2, FM_ROLE_WS = 3 };
 // plan-time marker of a leaf operand whose split-bf16 slice planes a stage
-// writes (FmOp::off: their byte offset in the workspace); never a kernel's role
+// writes (FmOp::off: their byte offset in the workspace, ld: their rows,
+// padding included); never a kernel's role
 constexpr int32_t FM_ROLE_PLANES = -2;
 
 // Roles 0-3 come from p[]; a batched plan numbers its problems' operands
@@ -58,7 +59,7 @@ struct FmOp {
 // ws + out_off + ((q * R + r) * R + r2) * out_slab.
 // Two-level S/T stage writing split-bf16 slice planes (FP32 data): the same
 // slab numbering, with out_off, view_off and out_slab in bytes (one slab:
-// the planes of a rows2 x cols2 operand) and out_ld unused.
+// the padded planes of a rows2 x cols2 operand) and out_ld unused.
 //
 // Grouped stage launch (the nodes of several problems, whose blocks differ
 // in shape, in one launch): `node` holds each node's operand, shape, output

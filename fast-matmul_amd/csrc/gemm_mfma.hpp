@@ -154,7 +154,9 @@ inline int fm_prep_wgs(const FmSplitPrep& p) {
 struct FmSplitDesc {
   FmOp c;
   int32_t M, N, K, Kp;
-  int32_t tiles_m, tiles_n, tile_begin, pad;
+  int32_t tiles_m, tiles_n, tile_begin;
+  int32_t a_rows, b_rows;  // rows of the A and B planes, padding included (at least the tiles')
+  int32_t pad;
   int64_t a_pl, b_pl;   // workspace byte offsets of the A and B planes
   double alpha, beta;
 };

@@ -354,7 +354,7 @@ __global__ void __launch_bounds__(64 * WM * WN) fm_split_gemm(FmSplitArgs args) 
   const fm_gptr<const char> ws = fm_global(reinterpret_cast<const char*>(args.bases.p[FM_ROLE_WS]));
   // chunk o of a slice: plane o / (4 * rows), row (o / 4) % rows, chunk o % 4;
   // consecutive K slices of a plane set are apa (bpa) rows apart
-  const int64_t apa = (int64_t)d.tiles_m * BM, bpa = (int64_t)d.tiles_n * BN;
+  const int64_t apa = d.a_rows, bpa = d.b_rows;
   const fm_gptr<const fm_u32x4> Ap = (fm_gptr<const fm_u32x4>)(ws + d.a_pl) + (int64_t)m0 * 12;
   const fm_gptr<const fm_u32x4> Bp = (fm_gptr<const fm_u32x4>)(ws + d.b_pl) + (int64_t)n0 * 12;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -527,7 +527,7 @@ __global__ void __launch_bounds__(64 * WM * WN) fm_split_gemm_bd(FmSplitArgs arg
   const int m0 = (first + rem % rows_g) * BM, n0 = (rem / rows_g) * BN;
   const int nkc = d.Kp >> 5;
   const fm_gptr<const char> ws = fm_global(reinterpret_cast<const char*>(args.bases.p[FM_ROLE_WS]));
-  const int64_t apa = (int64_t)d.tiles_m * BM, bpa = (int64_t)d.tiles_n * BN;
+  const int64_t apa = d.a_rows, bpa = d.b_rows;
   const fm_gptr<const fm_u32x4> Ap = (fm_gptr<const fm_u32x4>)(ws + d.a_pl) + (int64_t)m0 * 12;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave % WM, wn = wave / WM;

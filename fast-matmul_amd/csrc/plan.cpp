@@ -317,8 +317,12 @@ Launch split_launch(std::vector<FmGemmDesc> prods, int cfg, size_t* ws_bytes) {
   size_t off = (size_t)align_up((int64_t)*ws_bytes, 256);
   std::map<std::tuple<int, int64_t, int64_t, int, int, int>, int64_t> seen;
   int32_t prep_wgs = 0;
-  auto planes = [&](const FmOp& src, int rows, int K, int pad_to, int kcontig) {
-    if (src.role == FM_ROLE_PLANES) return src.off;  // written by the S/T stage
+  auto planes = [&](const FmOp& src, int rows, int K, int pad_to, int kcontig, int32_t* plane_rows) {
+    if (src.role == FM_ROLE_PLANES) {  // written by the S/T stage
+      *plane_rows = (int32_t)src.ld;
+      return src.off;
+    }
+    *plane_rows = (int32_t)align_up(rows, pad_to);
     const auto key = std::make_tuple(src.role, src.off, src.ld, rows, K, kcontig);
     auto it = seen.find(key);
     if (it != seen.end()) return it->second;
@@ -354,8 +358,8 @@ Launch split_launch(std::vector<FmGemmDesc> prods, int cfg, size_t* ws_bytes) {
     t += d.tiles_m * d.tiles_n;
     d.alpha = g.alpha;
     d.beta = g.beta;
-    d.a_pl = planes(g.a, g.M, g.K, bm, 0);
-    d.b_pl = planes(g.b, g.N, g.K, bn, 1);
+    d.a_pl = planes(g.a, g.M, g.K, bm, 0, &d.a_rows);
+    d.b_pl = planes(g.b, g.N, g.K, bn, 1, &d.b_rows);
     uniform = uniform && g.M == prods[0].M && g.N == prods[0].N;
     L.sdescs.push_back(d);
   }
@@ -775,21 +779,31 @@ fm_status build_subplan(fm_dtype dt, const Problem& p, int64_t ws_base, SubPlan&
     }
   }
   // Split-bf16 leaves on slice planes: the two-level S (T) stage of the last
-  // two levels writes the leaf operands' planes itself, and the preparation
+  // two levels writes the leaf operands' planes itself, padded to whole tiles of
+  // every split kernel (256 rows) and whole 32-deep slices, and the preparation
   // pass covers only leaf operands that are sub-blocks of A (B).  Taken when
-  // every split kernel's tiles divide the leaves (rows multiples of 256) and
-  // K is whole 32-deep slices, so the planes need no padding, and when the
-  // leaves' preparation grid would fit one launch (else they split on the
-  // fly, on the FP32 operands).
+  // the leaves' preparation grid would fit one launch (else they split on the
+  // fly, on the FP32 operands), for operands that need no padding, and for
+  // padded ones
+  // - of more than 128 rows: 256-row padding then takes no more workspace than
+  //   FP32 outputs with planes padded to 128;
+  // - of 2^18 elements, one wave per SIMD at 4 elements a lane: a lane forms
+  //   every output of its elements in turn, and a smaller stage is that serial
+  //   chain.
+  // Measured, separate -> stage-written: strassen two levels 600^3 51 -> 81 us,
+  // 1036^3 73 -> 94, 2048^3 211 -> 154, 3448^3 682 -> 589, 10008^3
+  // 9917 -> 8710; grey424_26_206 two levels 12000^3 23222 -> 17516.
   bool s_pl = false, t_pl = false;
   if (p.fuse_planes && dt == FM_F32 && L >= 2) {
     const Dims d = dims[L];
     double leaves = 1.0;
     for (int l = 0; l < L; ++l) leaves *= R;
     const double wgs = leaves * (double)((d.m + d.n + 126) / 64) * (double)((d.k + 127) / 128);
-    const bool ok = d.m % 256 == 0 && d.n % 256 == 0 && d.k % 32 == 0 && wgs <= 2147483647.0;
-    s_pl = ok && s2[L - 2] && alg->s2p_f != nullptr;
-    t_pl = ok && t2[L - 2] && alg->t2p_f != nullptr;
+    const bool fits = wgs <= 2147483647.0;
+    const bool whole = d.m % 256 == 0 && d.n % 256 == 0 && d.k % 32 == 0;
+    auto padded = [&](int64_t rows) { return rows > 128 && align_up(rows, 256) * align_up(d.k, 32) >= (1 << 18); };
+    s_pl = fits && (whole || padded(d.m)) && s2[L - 2] && alg->s2p_f != nullptr;
+    t_pl = fits && (whole || padded(d.n)) && t2[L - 2] && alg->t2p_f != nullptr;
   }
   const FmOp virt = op_make(-1, 0, 0);
   for (int l = 0; l < L; ++l) {
@@ -800,7 +814,8 @@ fm_status build_subplan(fm_dtype dt, const Problem& p, int64_t ws_base, SubPlan&
     // the last level's S (T) outputs and views as slice planes: bytes per
     // operand (c.m x c.k, 6 bytes an element), in FP32 workspace elements
     const bool spl = s_pl && l == L - 1, tpl = t_pl && l == L - 1;
-    const int64_t s_pb = align_up(c.m * c.k * 6, 256), t_pb = align_up(c.k * c.n * 6, 256);
+    const int64_t s_rows = align_up(c.m, 256), t_rows = align_up(c.n, 256), pk = align_up(c.k, 32);
+    const int64_t s_pb = align_up(s_rows * pk * 6, 256), t_pb = align_up(pk * t_rows * 6, 256);
     const int64_t s_step = spl ? s_pb / 4 : s_slab, t_step = tpl ? t_pb / 4 : t_slab;
     m_ld[l] = align_up(c.m, kLdAlign);
     m_slab[l] = align_up(m_ld[l] * c.n, kSlabAlign);
@@ -822,8 +837,8 @@ fm_status build_subplan(fm_dtype dt, const Problem& p, int64_t ws_base, SubPlan&
       if (s_second && nd.a.role < 0) nd.a_views = sv_off + q * alg->a_nviews * s_step;
       if (t_second && nd.b.role < 0) nd.b_views = tv_off + q * alg->b_nviews * t_step;
       // a workspace operand, or (last level, planes) the byte offset of its planes
-      auto s_op = [&](int64_t off) { return spl ? op_make(FM_ROLE_PLANES, off * 4, 0) : op_make(FM_ROLE_WS, off, s_ld); };
-      auto t_op = [&](int64_t off) { return tpl ? op_make(FM_ROLE_PLANES, off * 4, 0) : op_make(FM_ROLE_WS, off, t_ld); };
+      auto s_op = [&](int64_t off) { return spl ? op_make(FM_ROLE_PLANES, off * 4, s_rows) : op_make(FM_ROLE_WS, off, s_ld); };
+      auto t_op = [&](int64_t off) { return tpl ? op_make(FM_ROLE_PLANES, off * 4, t_rows) : op_make(FM_ROLE_WS, off, t_ld); };
       for (int r = 0; r < R; ++r) {
         Node ch;
         const int ai = alg->a_index[r], bi = alg->b_index[r];

@@ -365,11 +365,12 @@ __global__ void __launch_bounds__(FM_STAGE_THREADS) fm_in_stage2(FmStageArgs a) 
 // same order), each split by fm_split1 as the preparation pass splits a
 // stored FP32 slab, so the planes are bit-identical to preparing
 // fm_in_stage2's output.  Here out_off, view_off and out_slab are bytes (one
-// slab's planes: rows2 * cols2 * 6 bytes, no padding: the plan takes this
-// path only when the leaf operands' rows are whole tiles and their K whole
-// 32-deep slices).  A lane owns VEC consecutive k of one plane row (A side:
-// row i, columns k; B side: column j, rows k), so 32 / VEC consecutive lanes
-// write one 64-byte run of each plane.
+// slab's planes: 6 bytes an element, rows padded to 256 and K to 32 with
+// zeros; strassen two levels 3448^3 676 -> 593 us, grey424_26_206 two levels
+// 7296^3 7350 -> 5710 us against a separate preparation).  A lane owns VEC
+// consecutive k of one plane row (A side: row i, columns k; B side: column
+// j, rows k), so 32 / VEC consecutive lanes write one 64-byte run of each
+// plane.
 template <class Cmb, int SIDE>
 constexpr int fm_planes_vec() {
   constexpr int NB = SIDE == 0 ? Cmb::m * Cmb::k : Cmb::k * Cmb::n;
@@ -423,8 +424,12 @@ __global__ void __launch_bounds__(FM_STAGE_THREADS) fm_in_stage2_planes(FmStageA
   const fm_gptr<char> ws = fm_global(reinterpret_cast<char*>(a.bases.p[FM_ROLE_WS]));
   const fm_gptr<char> dst = ws + nv.out;
   const fm_gptr<char> vdst = ws + nv.view;
-  const uint32_t prow = SIDE == 0 ? (uint32_t)nv.rows2 : (uint32_t)nv.cols2;  // plane rows
-  const uint32_t nkc = (SIDE == 0 ? (uint32_t)nv.cols2 : (uint32_t)nv.rows2) / 32;
+  // the operand's rows and depth, and the planes': padded with zeros to whole
+  // tiles of every split kernel and whole 32-deep slices
+  const uint32_t rdim = SIDE == 0 ? (uint32_t)nv.rows2 : (uint32_t)nv.cols2;
+  const uint32_t kdim = SIDE == 0 ? (uint32_t)nv.cols2 : (uint32_t)nv.rows2;
+  const uint32_t prow = (rdim + 255) & ~255u;
+  const uint32_t nkc = (kdim + 31) / 32;
   const uint32_t total = prow * nkc * KQ;
   const int64_t ld = op.ld, brows = nv.rows, bcols = nv.cols, brows2 = nv.rows2,
                 bcols2 = nv.cols2, slab = nv.out_slab;
@@ -443,18 +448,32 @@ __global__ void __launch_bounds__(FM_STAGE_THREADS) fm_in_stage2_planes(FmStageA
     const uint32_t kc = rest / prow;
     const uint32_t k0 = kc * 32 + kq * VEC;
     const uint32_t i = SIDE == 0 ? r : k0, j = SIDE == 0 ? k0 : r;
+    // the work group's lanes cover RT consecutive plane rows (r0 ..) of one
+    // 32-deep slice (prow is a multiple of RT)
+    const uint32_t r0 = ((e - threadIdx.x) / KQ) % prow;
+    const bool edge = kc * 32 + 32 > kdim || r0 + RT > rdim;
     T v[NB][NB][VEC];  // v[block][sub-block][element]
     if constexpr (STAGED) {
-      // The work group's lanes cover RT consecutive plane rows (A rows
-      // r0 ..) of one 32-deep run (columns kc * 32 ..): every lane takes the
-      // same trip count (the total is a multiple of 256, plane rows a
-      // multiple of RT).  Each source's RT x 32 tile is loaded rows-first
+      // Every lane takes the same trip count (the total is a multiple of
+      // 256).  Each source's RT x 32 tile is loaded rows-first
       // (RT consecutive rows of a column per load) into LDS, then each lane
       // reads its k-first elements.  The k-first loads straight from HBM
       // fetched 32 columns' lines for 2 rows per wave instruction.
-      const uint32_t r0 = ((e - threadIdx.x) / KQ) % prow;
       const uint32_t sr = threadIdx.x % RT, sc = threadIdx.x / RT;
-      const fm_gptr<const T> ssrc = src + (r0 + sr) + (int64_t)(kc * 32 + sc) * ld;
+      // past the operand: its last row and column are loaded, zeros stored.
+      // (One lane pointer and the distances from it: a uniform pointer per
+      // source would be kept in registers over all trips, 304 against 191 of
+      // them for grey424 and one wave per SIMD less.)
+      int64_t dist[VEC];
+      bool ok[VEC];
+      const fm_gptr<const T> ssrc =
+          src + min(r0 + sr, rdim - 1) + (int64_t)min(kc * 32 + sc, kdim - 1) * ld;
+#pragma unroll
+      for (int pp = 0; pp < VEC; ++pp) {
+        const uint32_t col = kc * 32 + sc + pp * KQ;
+        dist[pp] = (int64_t)(min(col, kdim - 1) - min(kc * 32 + sc, kdim - 1)) * ld;
+        ok[pp] = r0 + sr < rdim && col < kdim;
+      }
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
         const fm_gptr<const T> bsrc = ssrc + (int64_t)(b / BC) * brows + (int64_t)(b % BC) * bcols * ld;
@@ -462,7 +481,10 @@ __global__ void __launch_bounds__(FM_STAGE_THREADS) fm_in_stage2_planes(FmStageA
         for (int sb = 0; sb < NB; ++sb) {
           const fm_gptr<const T> p = bsrc + (int64_t)(sb / BC) * brows2 + (int64_t)(sb % BC) * bcols2 * ld;
 #pragma unroll
-          for (int pp = 0; pp < VEC; ++pp) stg[(b * NB + sb) * 32 + sc + pp * KQ][sr] = p[(int64_t)pp * KQ * ld];
+          for (int pp = 0; pp < VEC; ++pp) {
+            const T t = p[dist[pp]];
+            stg[(b * NB + sb) * 32 + sc + pp * KQ][sr] = ok[pp] ? t : T(0);
+          }
         }
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -475,6 +497,32 @@ __global__ void __launch_bounds__(FM_STAGE_THREADS) fm_in_stage2_planes(FmStageA
 #pragma unroll
           for (int l = 0; l < VEC; ++l) v[b][sb][l] = stg[(b * NB + sb) * 32 + kq * VEC + l][rl];
       __syncthreads();  // the next trip overwrites the tile
+    } else if (VEC == 1 || edge) {
+      // (a lane's one element needs no path of its own; VEC elements are
+      // loaded one by one here, as vectors below)
+      int64_t dist[VEC];
+      bool ok[VEC];
+      const int64_t rr = min(r, rdim - 1), kk = min(k0, kdim - 1);
+      const fm_gptr<const T> lsrc = src + (SIDE == 0 ? rr + kk * ld : kk + rr * ld);
+#pragma unroll
+      for (int l = 0; l < VEC; ++l) {
+        dist[l] = (int64_t)(min(k0 + l, kdim - 1) - (uint32_t)kk) * estep;
+        ok[l] = r < rdim && k0 + l < kdim;
+      }
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        const fm_gptr<const T> bsrc = lsrc + (int64_t)(b / BC) * brows + (int64_t)(b % BC) * bcols * ld;
+#pragma unroll
+        for (int sb = 0; sb < NB; ++sb) {
+          const fm_gptr<const T> p = bsrc + (int64_t)(sb / BC) * brows2 + (int64_t)(sb % BC) * bcols2 * ld;
+#pragma unroll
+          for (int l = 0; l < VEC; ++l) {
+            const T t = p[dist[l]];
+            v[b][sb][l] = ok[l] ? t : T(0);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
     } else {
       const fm_gptr<const T> lsrc = src + i + (int64_t)j * ld;
 #pragma unroll
@@ -743,7 +791,8 @@ constexpr FmStageLaunch fm_stage2_fn() {
 template <class Cmb, int SIDE>
 hipError_t fm_launch_in_stage2_planes(const FmStageArgs& a, hipStream_t s) {
   constexpr int VEC = fm_planes_vec<Cmb, SIDE>();
-  const uint64_t total = (uint64_t)a.rows2 * (uint64_t)a.cols2 / VEC;
+  const uint64_t rdim = SIDE == 0 ? a.rows2 : a.cols2, kdim = SIDE == 0 ? a.cols2 : a.rows2;
+  const uint64_t total = (rdim + 255) / 256 * 256 * ((kdim + 31) / 32 * 32) / VEC;
   uint64_t gx = (total + FM_STAGE_THREADS - 1) / FM_STAGE_THREADS;
   uint64_t cap = 8192 / (uint64_t)(a.nodes > 0 ? a.nodes : 1);
   if (cap < 4) cap = 4;
