@@ -21,8 +21,9 @@ struct CostTable {
   double launch_us = 4.0;                   // one kernel launch
   double level_us[2] = {20.0, 20.0};        // one recursion level of a batched problem,
                                             // beyond its bytes and launches, per dtype
-  double tile_k_us[2] = {0.1, 0.1};         // one peeling tile's time per unit of K: a
-                                            // launch lasts at least its longest tile
+  double tile_k_us[2] = {0.1, 0.1};         // one 64 x 64 tile's time per unit of K: a
+                                            // floor under a level's peeling (a margin:
+                                            // the thin peeling kernels are faster)
   std::string source = "built-in";
 };
 

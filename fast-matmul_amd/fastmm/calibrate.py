@@ -11,7 +11,8 @@ Measures, with the library's own kernels:
   at 4096^3 over the stages' device time (the library's per-launch events);
 * the cost of one launch: a batch of one 64^3 product;
 * the time per unit of K of one 64 x 64 tile (one 64 x 4096 x 64 product):
-  a peeling launch lasts at least its longest tile, however few its flops;
+  the floor the model puts under a level's peeling, however few its flops (a
+  margin: peeling runs on thin kernels, which are faster);
 * the cost of one recursion level of a batched problem beyond its bytes and
   launches: 48 uneven problems at one level of Strassen and of <4,2,3;20>,
   measured time minus the model's estimate without that term (less the
@@ -107,7 +108,7 @@ def launch_cost():
 
 def tile_k_cost(dtype, launch_us):
     """Time per unit of K of one 64 x 64 tile (a launch of one tile, K = 4096),
-    less the launch: the floor under a peeling launch's duration."""
+    less the launch: the model's floor under a level's peeling."""
     k = 4096
     b = fastmm.Batch(_batch([(64, k, 64)], dtype, "plain"), graph=True)
     return max(0.0, (_time(b.run, 20) * 1e6 - launch_us) / k)
