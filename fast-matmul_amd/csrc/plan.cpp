@@ -413,19 +413,34 @@ namespace {
 // itself and waits for its own loads (the small tiles).  Whole-tile and ragged
 // products cost the same on these kernels (FP64 128 x 128: 8192 x 8192 x 4096
 // 71.7 TFLOP/s, 8190 x 8190 x 4090 70.0, 8191 x 8191 x 4091 69.7).
+// edge: the predicated kernel of the same tile, for launches the spread kernels
+// cannot take (M below a vector, K below a slice, columns past 32-bit offsets;
+// -1: not offered).  4096 x 4096 x 15, 7 products of 4096 x 4096 x 14 and 16384 x
+// 16384 x 8 on 64 x 64 tiles, on 128 x 128 ones: FP64 32.7, 213, 525 us and 32.3,
+// 196, 422; FP32 24.4, 144, 319 us and 20.2, 118, 310.
 struct TileCand {
   int cfg;
   double us_k, k0, lat_k;
+  int edge;
 };
-const TileCand kF64Tiles[] = {
-    {FM_TILE_PS_128x128_O2, 0.1257, 30, 0},  {FM_TILE_PS_128x256_W8, 0.2520, 30, 0},
-    {FM_TILE_PS_128x96_O2, 0.0960, 30, 0},   {FM_TILE_128x64, 0.0650, 34, 0},
-    {FM_TILE_64x128, 0.0645, 34, 0},         {FM_TILE_64x64, 0.0340, 32, 0.037},
-    {FM_TILE_PS_32x32_K32, 0.0103, 50, 0.0129}};
-const TileCand kF32Tiles[] = {
-    {FM_TILE_PS_128x256_W8, 0.1383, 44, 0}, {FM_TILE_PS_128x128_O2, 0.0695, 40, 0},
-    {FM_TILE_128x64, 0.0368, 43, 0},        {FM_TILE_64x128, 0.0368, 43, 0},
-    {FM_TILE_64x64, 0.0192, 43, 0.0227},    {FM_TILE_PS_32x32_K32, 0.0057, 60, 0.0099}};
+const TileCand kF64Tiles[] = {{FM_TILE_PS_128x128_O2, 0.1257, 30, 0, FM_TILE_128x128_O2_U1},
+                              {FM_TILE_PS_128x256_W8, 0.2520, 30, 0, -1},
+                              {FM_TILE_PS_128x96_O2, 0.0960, 30, 0, -1},
+                              {FM_TILE_128x64, 0.0650, 34, 0, -1},
+                              {FM_TILE_64x128, 0.0645, 34, 0, -1},
+                              {FM_TILE_64x64, 0.0340, 32, 0.037, FM_TILE_64x64},
+                              {FM_TILE_PS_32x32_K32, 0.0103, 50, 0.0129, -1}};
+const TileCand kF32Tiles[] = {{FM_TILE_PS_128x256_W8, 0.1383, 44, 0, -1},
+                              {FM_TILE_PS_128x128_O2, 0.0695, 40, 0, FM_TILE_128x128_W8},
+                              {FM_TILE_128x64, 0.0368, 43, 0, -1},
+                              {FM_TILE_64x128, 0.0368, 43, 0, -1},
+                              {FM_TILE_64x64, 0.0192, 43, 0.0227, FM_TILE_64x64},
+                              {FM_TILE_PS_32x32_K32, 0.0057, 60, 0.0099, -1}};
+
+const TileCand* plain_cands(fm_dtype dt, size_t* n) {
+  *n = dt == FM_F64 ? sizeof(kF64Tiles) / sizeof(kF64Tiles[0]) : sizeof(kF32Tiles) / sizeof(kF32Tiles[0]);
+  return dt == FM_F64 ? kF64Tiles : kF32Tiles;
+}
 // a launch's own cost beside its tiles
 const double kLaunchUs = 3.0;
 const double kCopyBytesPerUs = 4.9e6;
@@ -433,8 +448,7 @@ const double kCopyBytesPerUs = 4.9e6;
 // L2 (strassen one level 2048^3 FP64: 4 of 7 leaves as 256 128 x 128 tiles and
 // 3 as 64 x 64 ones 294 us, all on 64 x 64 tiles 266)
 const double kAlonePenalty = 1.15;
-// What the spread kernels cannot take (M below a vector, K below a slice,
-// columns past 32-bit offsets) runs on the 64 x 64 tile's predicated loop.
+// the predicated loop's time over the spread loop's
 const double kEdgePenalty = 1.3;
 // split-bf16: kernels on prepared slice planes (any shape: the planes are
 // padded to whole tiles), throughput per tile area and resident work groups
@@ -467,7 +481,7 @@ int64_t count_tiles(int cfg, const std::vector<FmGemmDesc>& prods) {
 // deepest tile for the end of the launch.  At least the time of the products'
 // bytes (a strip reads a whole operand again), a fifth of which is not hidden
 // behind the products of a compute-bound launch.
-double cand_us(fm_dtype dt, const TileCand& c, const std::vector<FmGemmDesc>& prods) {
+double cand_us(fm_dtype dt, const TileCand& c, const std::vector<FmGemmDesc>& prods, bool fits) {
   int bm, bn;
   fm_tile_dims(c.cfg, &bm, &bn);
   double work = 0, kmax = 0, kmin = 1e30, elems = 0;
@@ -486,8 +500,12 @@ double cand_us(fm_dtype dt, const TileCand& c, const std::vector<FmGemmDesc>& pr
                       : tiles > kCUs ? tile * (double)((tiles + kCUs - 1) / kCUs)
                                      : tile * kAlonePenalty;
   const double t = std::max(busy, std::max(c.lat_k * kmax, mem)) + 0.2 * mem;
-  const bool fits = any_tiles(dt, c.cfg, prods) || whole_tiles(dt, c.cfg, prods);
   return kLaunchUs + t * (fits ? 1.0 : kEdgePenalty);
+}
+
+// The spread kernels of configuration cfg take the products.
+bool spread_fits(fm_dtype dt, int cfg, const std::vector<FmGemmDesc>& prods) {
+  return any_tiles(dt, cfg, prods) || whole_tiles(dt, cfg, prods);
 }
 
 // Split-bf16: rounds of per_cu work groups on each CU, in relative units.
@@ -514,15 +532,13 @@ int best_tile(fm_dtype dt, fm_mode mode, const std::vector<FmGemmDesc>& prods, d
   if (mode == FM_MODE_SPLIT_BF16) {
     for (const SplitCand& c : kSplitTiles) offer(c.cfg, split_time(c, count_tiles(c.cfg, prods)), 0.999);
   } else {
-    auto fits = [&](int cfg) { return whole_tiles(dt, cfg, prods) || any_tiles(dt, cfg, prods); };
-    auto each = [&](const TileCand* c, size_t n) {
-      for (size_t i = 0; i < n; ++i)
-        if (fits(c[i].cfg) || c[i].cfg == FM_TILE_64x64) offer(c[i].cfg, cand_us(dt, c[i], prods), margin);
-    };
-    if (dt == FM_F64)
-      each(kF64Tiles, sizeof(kF64Tiles) / sizeof(kF64Tiles[0]));
-    else
-      each(kF32Tiles, sizeof(kF32Tiles) / sizeof(kF32Tiles[0]));
+    size_t n;
+    const TileCand* c = plain_cands(dt, &n);
+    for (size_t i = 0; i < n; ++i) {
+      const bool fits = spread_fits(dt, c[i].cfg, prods);
+      const int cfg = fits ? c[i].cfg : c[i].edge;
+      if (cfg >= 0) offer(cfg, cand_us(dt, c[i], prods, fits), margin);
+    }
   }
   if (t_out) *t_out = best_t;
   return best;
@@ -540,10 +556,11 @@ double list_time(fm_dtype dt, fm_mode mode, int cfg, const std::vector<FmGemmDes
       }
     return -1;
   }
-  const TileCand* c = dt == FM_F64 ? kF64Tiles : kF32Tiles;
-  const size_t n = dt == FM_F64 ? sizeof(kF64Tiles) / sizeof(kF64Tiles[0]) : sizeof(kF32Tiles) / sizeof(kF32Tiles[0]);
+  size_t n;
+  const TileCand* c = plain_cands(dt, &n);
   for (size_t i = 0; i < n; ++i)
-    if (c[i].cfg == cfg) return cand_us(dt, c[i], prods);
+    if (c[i].cfg == cfg || c[i].edge == cfg)
+      return cand_us(dt, c[i], prods, c[i].cfg == cfg && spread_fits(dt, cfg, prods));
   return -1;
 }
 
@@ -563,9 +580,8 @@ bool carve_full(const Plan& P, int cfg, std::vector<FmGemmDesc>& prods, std::vec
   if (P.tile >= 0 || P.mode != FM_MODE_PLAIN) return false;
   int64_t round;
   const double t_all = list_time(P.dtype, P.mode, cfg, prods, &round);
-  const TileCand* cands = P.dtype == FM_F64 ? kF64Tiles : kF32Tiles;
-  const size_t n = P.dtype == FM_F64 ? sizeof(kF64Tiles) / sizeof(kF64Tiles[0])
-                                     : sizeof(kF32Tiles) / sizeof(kF32Tiles[0]);
+  size_t n;
+  const TileCand* cands = plain_cands(P.dtype, &n);
   double best_t = 0.995 * t_all;
   std::vector<FmGemmDesc> core, st, best_core, best_st;
   for (size_t i = 0; i < n; ++i) {
@@ -580,10 +596,10 @@ bool carve_full(const Plan& P, int cfg, std::vector<FmGemmDesc>& prods, std::vec
       if (d.M > Mf && Nf > 0) st.push_back(gsub(d, Mf, 0, d.M - Mf, Nf));  // bottom strip
     }
     if (core.empty() || st.empty()) continue;
-    if (!whole_tiles(P.dtype, cands[i].cfg, core) && !any_tiles(P.dtype, cands[i].cfg, core)) continue;
+    if (!spread_fits(P.dtype, cands[i].cfg, core)) continue;
     double t_strips = 0;
     const int cs = best_tile(P.dtype, P.mode, st, &t_strips);
-    const double t = cand_us(P.dtype, cands[i], core) + t_strips;
+    const double t = cand_us(P.dtype, cands[i], core, true) + t_strips;
     if (t >= best_t) continue;
     best_t = t;
     best_core = core;
