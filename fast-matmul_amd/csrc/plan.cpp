@@ -201,14 +201,18 @@ bool whole_tiles(fm_dtype dt, int cfg, const std::vector<FmGemmDesc>& prods) {
 // rows and a whole K slice exist to load from, and the byte offsets of a
 // tile's columns (two slices of A, the tile's columns of B) stay within 32
 // bits.
-bool any_tiles(fm_dtype dt, int cfg, const std::vector<FmGemmDesc>& prods) {
-  if (!fm_tile_spread(cfg)) return false;
+bool any_tile(fm_dtype dt, int cfg, const FmGemmDesc& d) {
   int bm, bn;
   fm_tile_dims(cfg, &bm, &bn);
   const int64_t bk = fm_tile_bk(cfg), vl = dt == FM_F64 ? 2 : 4;
   const int64_t span = (int64_t(1) << 32) / elem_size(dt);
+  return d.M >= vl && d.K >= bk && bm + 2 * bk * d.a.ld < span && 2 * bk + bn * d.b.ld < span;
+}
+
+bool any_tiles(fm_dtype dt, int cfg, const std::vector<FmGemmDesc>& prods) {
+  if (!fm_tile_spread(cfg)) return false;
   for (const FmGemmDesc& d : prods)
-    if (d.M < vl || d.K < bk || bm + 2 * bk * d.a.ld >= span || 2 * bk + bn * d.b.ld >= span) return false;
+    if (!any_tile(dt, cfg, d)) return false;
   return true;
 }
 
@@ -569,6 +573,29 @@ FmGemmDesc gsub(const FmGemmDesc& d, int64_t i0, int64_t j0, int64_t m, int64_t 
                d.beta);
 }
 
+// One product that no spread kernel takes (a K of 8, a single row, columns past
+// 32-bit offsets) would send a whole grouped launch to the predicated kernels:
+// such products move to `odd`, a launch of their own, where that is estimated
+// faster (63 products of 512 to 2048 a side and one of 2048 x 8 x 2048: FP64 4029 ->
+// 3388 us, FP32 2244 -> 1792).  Returns the estimated time of all of them; *cfg is the tile of those
+// that stay.
+double set_apart(fm_dtype dt, std::vector<FmGemmDesc>& prods, std::vector<FmGemmDesc>& odd, int* cfg) {
+  double t_one = 0, t_fit = 0, t_odd = 0;
+  *cfg = best_tile(dt, FM_MODE_PLAIN, prods, &t_one);
+  // (the widest tile: the slice depth of all but the smallest, the longest offsets)
+  auto fits = [&](const FmGemmDesc& d) { return any_tile(dt, FM_TILE_PS_128x256_W8, d); };
+  std::vector<FmGemmDesc> in, out;
+  for (const FmGemmDesc& d : prods) (fits(d) ? in : out).push_back(d);
+  if (in.empty() || out.empty()) return t_one;
+  const int cfg_in = best_tile(dt, FM_MODE_PLAIN, in, &t_fit);
+  (void)best_tile(dt, FM_MODE_PLAIN, out, &t_odd);
+  if (t_fit + t_odd >= 0.99 * t_one) return t_one;
+  prods = std::move(in);
+  odd = std::move(out);
+  *cfg = cfg_in;
+  return t_fit + t_odd;
+}
+
 // Whole-tile carve-out: a ragged product's last tile row and column are
 // partly empty.  Cutting each product into its whole-tile core and the row and
 // column strips left over (a second launch, with the tile that fits them) is
@@ -576,19 +603,20 @@ FmGemmDesc gsub(const FmGemmDesc& d, int64_t i0, int64_t j0, int64_t m, int64_t 
 // computed by the same K-ordered MFMA sequence either way.  Returns false
 // (prods unchanged) when it does not pay or does not apply.
 bool carve_full(const Plan& P, int cfg, std::vector<FmGemmDesc>& prods, std::vector<FmGemmDesc>& strips,
-                int* cfg_core, int* cfg_strips) {
+                std::vector<FmGemmDesc>& odd, int* cfg_core, int* cfg_strips) {
   if (P.tile >= 0 || P.mode != FM_MODE_PLAIN) return false;
   int64_t round;
   const double t_all = list_time(P.dtype, P.mode, cfg, prods, &round);
   size_t n;
   const TileCand* cands = plain_cands(P.dtype, &n);
   double best_t = 0.995 * t_all;
-  std::vector<FmGemmDesc> core, st, best_core, best_st;
+  std::vector<FmGemmDesc> core, st, st_odd, best_core, best_st, best_odd;
   for (size_t i = 0; i < n; ++i) {
     int bm, bn;
     fm_tile_dims(cands[i].cfg, &bm, &bn);
     core.clear();
     st.clear();
+    st_odd.clear();
     for (const FmGemmDesc& d : prods) {
       const int64_t Mf = d.M / bm * bm, Nf = d.N / bn * bn;
       if (Mf > 0 && Nf > 0) core.push_back(gsub(d, 0, 0, Mf, Nf));
@@ -597,19 +625,21 @@ bool carve_full(const Plan& P, int cfg, std::vector<FmGemmDesc>& prods, std::vec
     }
     if (core.empty() || st.empty()) continue;
     if (!spread_fits(P.dtype, cands[i].cfg, core)) continue;
-    double t_strips = 0;
-    const int cs = best_tile(P.dtype, P.mode, st, &t_strips);
+    int cs;
+    const double t_strips = set_apart(P.dtype, st, st_odd, &cs);
     const double t = cand_us(P.dtype, cands[i], core, true) + t_strips;
     if (t >= best_t) continue;
     best_t = t;
     best_core = core;
     best_st = st;
+    best_odd = st_odd;
     *cfg_core = cands[i].cfg;
     *cfg_strips = cs;
   }
   if (best_core.empty()) return false;
   prods = std::move(best_core);
   strips = std::move(best_st);
+  odd.insert(odd.end(), best_odd.begin(), best_odd.end());
   return true;
 }
 }  // namespace
@@ -1157,6 +1187,12 @@ fm_status assemble(Plan& P, std::vector<SubPlan>& subs, int64_t ws_elems, int pe
       if (st != FM_OK) return st;
       P.launches.push_back(std::move(L));
     } else {
+      const bool several = persistent_grid == 0 && P.split_rem;  // leaf launches allowed
+      std::vector<FmGemmDesc> rest, strips, odd;
+      if (several && P.tile < 0 && P.mode == FM_MODE_PLAIN) {
+        int cfg_fit;
+        (void)set_apart(P.dtype, leaves, odd, &cfg_fit);
+      }
       const int cfg = pick_tile(P, leaves);
       if (fm_tile_planes(cfg) && P.mode != FM_MODE_SPLIT_BF16)
         return set_err(FM_ERR_INVALID_ARG, "tile config " + std::to_string(cfg) + " is for split_bf16 leaves");
@@ -1167,10 +1203,9 @@ fm_status assemble(Plan& P, std::vector<SubPlan>& subs, int64_t ws_elems, int pe
           cfg != FM_TILE_128x128_W8)
         return set_err(FM_ERR_INVALID_ARG, "tile config " + std::to_string(cfg) +
                                                " has no split_bf16 kernel");
-      std::vector<FmGemmDesc> rest, strips;
       int cfg_rest = cfg, cfg_main = cfg, cfg_strips = cfg;
-      if (persistent_grid == 0 && P.split_rem) {
-        (void)carve_full(P, cfg, leaves, strips, &cfg_main, &cfg_strips);
+      if (several) {
+        (void)carve_full(P, cfg, leaves, strips, odd, &cfg_main, &cfg_strips);
         split_remainder(P, cfg_main, leaves, rest, &cfg_rest);
       }
       auto leaf = [&](std::vector<FmGemmDesc> prods, int c) {
@@ -1189,6 +1224,10 @@ fm_status assemble(Plan& P, std::vector<SubPlan>& subs, int64_t ws_elems, int pe
       P.launches.back().sp.grid = persistent_grid;
       if (!rest.empty()) P.launches.push_back(leaf(std::move(rest), cfg_rest));
       if (!strips.empty()) P.launches.push_back(leaf(std::move(strips), cfg_strips));
+      if (!odd.empty()) {
+        const int cfg_odd = pick_tile(P, odd);
+        P.launches.push_back(leaf(std::move(odd), cfg_odd));
+      }
     }
   }
   int maxd = 0;

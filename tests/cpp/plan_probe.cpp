@@ -1,0 +1,64 @@
+// Plans of several problems, built on the host with the library's own planner
+// and printed one launch a line:
+//   plan_probe f64|f32 [problem ...]
+// problem: m,k,n[,algorithm,steps[,depth-first levels]]
+//   gemm cfg any full products tiles max_k_of_products
+//   thin products tiles | stage kind nodes k_updates
+#include <algorithm>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <string>
+#include <vector>
+
+#include "plan.hpp"
+
+using namespace fmplan;
+
+extern const FmAlgDesc* fm_find_alg(const char* name);
+
+int main(int argc, char** argv) {
+  const fm_dtype dt = strcmp(argv[1], "f64") == 0 ? FM_F64 : FM_F32;
+  Plan P;
+  P.dtype = dt;
+  std::vector<SubPlan> subs((size_t)(argc - 2));
+  int64_t ws = 0;
+  for (int i = 0; i < argc - 2; ++i) {
+    std::vector<std::string> f;
+    for (char* t = strtok(argv[i + 2], ","); t; t = strtok(nullptr, ",")) f.push_back(t);
+    Problem p;
+    p.m = p.lda = p.ldc = atoll(f[0].c_str());
+    p.k = p.ldb = atoll(f[1].c_str());
+    p.n = atoll(f[2].c_str());
+    p.role_a = 4 + 3 * i;
+    p.role_b = 5 + 3 * i;
+    p.role_c = 6 + 3 * i;
+    if (f.size() > 4) {
+      p.alg = fm_find_alg(f[3].c_str());
+      p.steps = atoi(f[4].c_str());
+      if (!p.alg) return 2;
+    }
+    if (f.size() > 5) p.dfs = atoi(f[5].c_str());
+    if (build_subplan(dt, p, ws, subs[(size_t)i]) != FM_OK) {
+      fprintf(stderr, "%s\n", last_error().c_str());
+      return 1;
+    }
+    ws += subs[(size_t)i].ws_elems;
+  }
+  if (assemble(P, subs, ws) != FM_OK) {
+    fprintf(stderr, "%s\n", last_error().c_str());
+    return 1;
+  }
+  for (const Launch& L : P.launches) {
+    if (L.kind == LK_GEMM) {
+      int k = 0;
+      for (const FmGemmDesc& d : L.gdescs) k = std::max(k, d.K);
+      printf("gemm %d %d %d %d %d %d\n", L.cfg, L.gm.any, L.gm.full, L.gm.ndesc, L.gm.total_tiles, k);
+    } else if (L.kind == LK_THIN) {
+      printf("thin %d %d\n", L.th.ndesc, L.th.total_tiles);
+    } else {
+      printf("stage %d %d %d\n", (int)L.kind, L.st.nodes, L.nupd);
+    }
+  }
+  return 0;
+}

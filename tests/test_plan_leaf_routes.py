@@ -6,11 +6,15 @@ The spread loop needs M of at least one 16-byte vector and K of at least one
 tiles (FmTileCfg 16 in FP64, 5 in FP32) where the launch has enough of them,
 64 x 64 (FmTileCfg 1) where a larger tile would be mostly empty.
 """
+import os
+import subprocess
+
 import pytest
 import torch
 
 import fastmm
 
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 EDGE = {torch.float64: 16, torch.float32: 5}
 
 
@@ -34,3 +38,73 @@ def test_single_rows_keep_the_small_predicated_tile(dtype):
     # and the spread loop takes everything else
     assert _leaf(4096, 16, 4096, dtype) not in (1, EDGE[dtype])
     assert _leaf(4, 4096, 4096, dtype) not in (EDGE[dtype],)
+
+
+# ---- several problems in one launch sequence ------------------------------------
+@pytest.fixture(scope="module")
+def probe(tmp_path_factory):
+    """run(dtype, problems): the launches of a batch's plan, as tests/cpp/plan_probe.cpp prints them."""
+    exe = str(tmp_path_factory.mktemp("plan") / "plan_probe")
+    lib = os.path.join(ROOT, "fast-matmul_amd", "fastmm")
+    subprocess.check_call(
+        ["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(ROOT, "include"),
+         "-I", os.path.join(ROOT, "fast-matmul_amd", "csrc"), "-I", "/opt/rocm/include",
+         os.path.join(ROOT, "tests", "cpp", "plan_probe.cpp"), "-o", exe, "-L", lib, "-lfastmm",
+         "-L", "/opt/rocm/lib", "-lamdhip64", "-Wl,-rpath," + lib + ":/opt/rocm/lib"])
+
+    def run(dtype, problems):
+        args = [",".join(str(v) for v in p) for p in problems]
+        out = subprocess.check_output([exe, dtype] + args, text=True)
+        return [l.split()[:1] + [int(v) for v in l.split()[1:]] for l in out.splitlines()]
+
+    return run
+
+
+def _gemms(launches):
+    """{"cfg", "any", "full", "products", "tiles", "k"} of each leaf launch."""
+    return [dict(zip(("cfg", "any", "full", "products", "tiles", "k"), l[1:])) for l in launches if l[0] == "gemm"]
+
+
+def _spread(launches):
+    return [g for g in launches if g["any"] or g["full"]]
+
+
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+@pytest.mark.parametrize("odd", [(4096, 8, 4096), (1, 2048, 2048)])
+def test_one_odd_problem_leaves_the_others_their_kernels(probe, dtype, odd):
+    # 63 large problems of ragged sizes and one that the spread loop cannot take
+    # (in FP32 one of the 63 has a bottom strip of 3 rows, less than a vector)
+    big = [(1000 + 37 * i, 1500 + 11 * (i % 7), 900 + 53 * i) for i in range(63)]
+    alone = _gemms(probe(dtype, big))
+    mixed = _gemms(probe(dtype, big[:20] + [odd] + big[20:]))
+    assert len(_spread(alone)) == 2 and _spread(mixed) == _spread(alone)
+    rest = [g for g in mixed if g not in _spread(mixed)]
+    assert len(rest) == 1 and rest[0]["products"] == (1 if dtype == "f64" else 2)
+
+
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+def test_one_row_strip_leaves_the_other_strips_their_kernels(probe, dtype):
+    # cores of whole tiles with right strips 40 columns wide, and one problem
+    # whose bottom strip is one row
+    big = [(2048, 2048, 2048 + 40)] * 200
+    alone = _gemms(probe(dtype, big + [(2048, 2048, 2048)]))
+    mixed = _gemms(probe(dtype, big + [(2049, 2048, 2048)]))
+    assert [g["products"] for g in _spread(alone)] == [201, 200]
+    for g, h in zip(_spread(mixed), _spread(alone)):
+        assert (g["cfg"], g["products"], g["tiles"]) == (h["cfg"], h["products"], h["tiles"])
+    assert len(_spread(mixed)) == 2
+    rest = [g for g in mixed if g not in _spread(mixed)]
+    assert [g["products"] for g in rest] == [1]
+
+
+def test_an_odd_problem_that_would_only_wait_stays(probe):
+    # 12 such problems: alone, the one row's chain over K would take longer than
+    # all strips do beside it, so they share its launch
+    g = _gemms(probe("f64", [(2048, 2048, 2048 + 40)] * 12 + [(2049, 2048, 2048)]))
+    assert [x["products"] for x in g] == [13, 13]
+
+
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+def test_only_odd_problems_share_one_launch(probe, dtype):
+    g = _gemms(probe(dtype, [(500, 3, 500), (1, 300, 700), (900, 15, 100)]))
+    assert len(g) == 1 and not g[0]["any"] and g[0]["products"] == 3
