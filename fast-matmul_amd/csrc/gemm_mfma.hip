@@ -62,7 +62,11 @@ constexpr int FM_TILE_GROUP = 8;
 // checks), so only the unpredicated 16-byte load path is compiled.  ANY:
 // products of any size, offset and leading dimension (M >= the vector
 // width, K >= BK, 32-bit tile spans: the launch checks) on the same
-// unconditional 16-byte loads; see the loop.
+// unconditional 16-byte loads; see the loop.  The FULL spread kernels use no
+// scratch; of the ANY ones four do: FP32 128 x 256 52 bytes a lane, FP64 128 x 128
+// 32, 128 x 64 and 64 x 128 12 each.  The first two and 64 x 128 reload 2 to 4 of
+// these registers a trip, behind its last product (rates beside the whole-tile
+// kernels': FP64 128 x 128 70 of 71.7 TFLOP/s, FP32 128 x 256 132 of 134).
 template <typename T, int BM, int BN, int BK, int WM, int WN, int MINW = 1, int UNR = BK / 4,
           int PIPE = 0, bool FULL = false, bool ANY = false>
 __global__ void __launch_bounds__(64 * WM * WN, MINW) fm_gemm_kernel(FmGemmArgs args) {
@@ -458,14 +462,17 @@ __global__ void __launch_bounds__(64 * WM * WN, MINW) fm_gemm_kernel(FmGemmArgs 
     __builtin_amdgcn_sched_barrier(0);                                                     \
     mma_step((NS4 - 1) & 1);                                                               \
   }
-    // Two slices to a trip (but for the FP64 tile 256 columns wide, which loses
-    // 0.8% to it): the LDS buffer of each is then a constant and its addresses
-    // are immediate offsets.  The vector instructions between the products are
-    // what the loop waits for (8192 x 8192 x 4096, one -> two: FP64 128 x 128
-    // 72.4 -> 73.2 TFLOP/s, 128 x 96 68.2 -> 69.9; FP32 128 x 256 134.4 -> 136.8,
-    // 128 x 64 125.2 -> 129.5; 49 products of 1250^3 FP32 on 128 x 128 tiles
-    // 110.9 -> 115.6).
-    constexpr bool PAIR = !(sizeof(T) == 8 && BN >= 256);
+    // Two slices to a trip (but for the tiles 256 columns wide): the LDS buffer of
+    // each is then a constant and its addresses are immediate offsets.  The
+    // vector instructions between the products are what the loop waits for
+    // (8192 x 8192 x 4096, one -> two: FP64 128 x 128 72.4 -> 73.2 TFLOP/s, 128 x 96
+    // 68.2 -> 69.9; FP32 128 x 64 125.2 -> 129.5; 49 products of 1250^3 FP32 on 128 x
+    // 128 tiles 110.9 -> 115.6).  The 256-column tiles have no registers left for
+    // it: FP64 loses 0.8%; FP32 (126 of the 128 that let two work groups share a
+    // CU) moves within the noise at K = 4096 and, with 52 bytes of scratch a lane
+    // for the second slice, loses 7% on shallow products (32768 x 32768 x 64 1858
+    // -> 1992 us).
+    constexpr bool PAIR = BN < 256;
     const int kb = FULL || kr == BK ? nk : max(nk - 3, 0);  // the iterations before the partial slice
     int kt = 0;
     if constexpr (PAIR) {
