@@ -8,7 +8,7 @@
 // had one work group per 64 rows walking all of K through LDS, 16 deep at a
 // time: a serial chain of loads and barriers, 0.25 us per unit of K whatever
 // the machine could stream.  Here K is spread over the lanes of a work group
-// (16 or 8 K segments in the right strip, 64 lanes in the bottom strip) with 8
+// (up to 16 or 8 K segments in the right strip, 64 lanes in the bottom strip) with 8
 // (4) loads in flight per lane, and the segments' sums meet once at the end,
 // in a fixed order that depends on the product alone.
 // Measured on MI355X (peeling per multiply, before -> after):
@@ -92,11 +92,17 @@ __global__ void __launch_bounds__(FM_THIN_THREADS) fm_thin_kernel(FmThinArgs arg
 
 }  // namespace
 
-void fm_thin_tile(int dtype_f64, int kind, int* rows, int* cols) {
-  *rows = kind == FM_THIN_K   ? FM_THIN_THREADS
-          : kind == FM_THIN_N ? (dtype_f64 ? strip_rows<double>() : strip_rows<float>())
-                              : FM_THIN_MAX;
-  *cols = kind == FM_THIN_K ? UPD_COLS : kind == FM_THIN_N ? FM_THIN_MAX : BOT_COLS * BOT_WAVES;
+void fm_thin_tile(int dtype_f64, int kind, int K, int* rows, int* cols) {
+  *rows = FM_THIN_MAX;
+  *cols = FM_THIN_MAX;
+  if (kind == FM_THIN_K) {
+    *rows = FM_THIN_THREADS;
+    *cols = UPD_COLS;
+  } else if (kind == FM_THIN_N) {
+    *rows = FM_THIN_THREADS >> strip_segs(dtype_f64 ? strip_log<double>() : strip_log<float>(), K);
+  } else {
+    *cols = BOT_WAVES * BOT_COLS * (64 >> bot_lanes(K));
+  }
 }
 
 hipError_t fm_thin_launch(int dtype_f64, const FmThinArgs& a, hipStream_t s) {

@@ -40,6 +40,6 @@ struct FmThinArgs {
   int32_t t0[3], d0[3], per[3];
 };
 
-// output tile of each kind: rows x columns of C per work group
-void fm_thin_tile(int dtype_f64, int kind, int* rows, int* cols);
+// output tile of a product of each kind and depth: rows x columns of C per work group
+void fm_thin_tile(int dtype_f64, int kind, int K, int* rows, int* cols);
 hipError_t fm_thin_launch(int dtype_f64, const FmThinArgs& a, hipStream_t s);

@@ -169,13 +169,13 @@ Launch thin_launch(std::vector<FmThinDesc> descs, fm_dtype dt) {
     for (; i < descs.size() && descs[i].kind == kind; ++i) {
       FmThinDesc& d = descs[i];
       int bm, bn;
-      fm_thin_tile(dt == FM_F64, kind, &bm, &bn);
+      fm_thin_tile(dt == FM_F64, kind, d.K, &bm, &bn);
       d.tiles_m = (d.M + bm - 1) / bm;
       d.tile_begin = t;
       const int32_t per = d.tiles_m * ((d.N + bn - 1) / bn);
       t += per;
       L.th.per[kind] = per;
-      if (d.M != descs[first].M || d.N != descs[first].N) L.th.uniform = 0;
+      if (d.M != descs[first].M || d.N != descs[first].N || d.K != descs[first].K) L.th.uniform = 0;
     }
   }
   L.th.ndesc = (int32_t)descs.size();

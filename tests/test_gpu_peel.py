@@ -58,6 +58,17 @@ def test_tile_edges(fm, shape, dtype):
 
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("k", [2, 5, 8, 9, 16, 17, 33, 64, 65, 127, 128, 129, 257])
+def test_strips_of_a_short_k(fm, k, dtype):
+    """K segments and lanes of the strips: one, as many as K fills, and all of
+    them (the limits are 8 and 4 values of K per segment and lane), with rows
+    and columns one past, and one short of, every tile that goes with them."""
+    for m, n in [(257, 1031), (1025, 513), (33, 63), (255, 129)]:
+        _check(fm, "strassen", m, k, n, dtype, -1.0, 2.0, k)
+    _check(fm, "smirnov336_40_960", 3 * 90 + 2, k + 1, 6 * 60 + 5, dtype, 1.0, 0.0, k)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
 @pytest.mark.parametrize("alg,shape", [
     ("strassen", (2056, 1027, 2052)),             # K remainder alone, 16-byte rows in the W stage
     ("grey522_18_99", (2063, 1027, 2051)),        # every remainder, odd rows

@@ -108,3 +108,26 @@ def test_an_odd_problem_that_would_only_wait_stays(probe):
 def test_only_odd_problems_share_one_launch(probe, dtype):
     g = _gemms(probe(dtype, [(500, 3, 500), (1, 300, 700), (900, 15, 100)]))
     assert len(g) == 1 and not g[0]["any"] and g[0]["products"] == 3
+
+
+# ---- peeled strips ----------------------------------------------------------------
+def _strip_tiles(launches):
+    """Work groups of the launches of peeled strips on their own."""
+    return [l[2] for l in launches if l[0] == "thin"]
+
+
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+def test_strips_of_a_short_k_take_few_work_groups(probe, dtype):
+    # two problems, so that the strips run in a launch of their own; K = 8 is one
+    # segment of 256 rows (two lanes of 512 columns)
+    for m, k, n, groups in [(1000001, 8, 4, 0), (1000000, 8, 5, 3907), (5, 8, 1000000, 1954)]:
+        t = _strip_tiles(probe(dtype, [(m, k, n, "strassen", 1), (m, k, n, "strassen", 1)]))
+        one_row = 1 if m == 1000001 else 0  # its bottom row: one work group
+        assert t == [2 * (groups or one_row)]
+
+
+def test_strips_of_long_matrices_fit_one_launch(probe):
+    # a launch holds fewer than 2^32 threads, 2^24 of these work groups
+    for p in [(1 << 28, 2, 3), ((1 << 29) + 4, 6, 3), (3, 2, 1 << 30)]:
+        t = _strip_tiles(probe("f64", [p + ("strassen", 1), (64, 64, 65, "strassen", 1)]))
+        assert t and max(t) < 1 << 24
