@@ -422,24 +422,32 @@ namespace {
 // -1: not offered).  4096 x 4096 x 15, 7 products of 4096 x 4096 x 14 and 16384 x
 // 16384 x 8 on 64 x 64 tiles, on 128 x 128 ones: FP64 32.7, 213, 525 us and 32.3,
 // 196, 422; FP32 24.4, 144, 319 us and 20.2, 118, 310.
+// deep_k: the least K in a launch of more than kManyTiles.  There the operands
+// come from HBM, and a tile of few slices costs more than the figures say: 7
+// products of 150000 x 32 x N (K = 32) on 32 x 32 and on 128 x 64 tiles, N = 8 and
+// 32, FP64 166, 213 and 123, 168 us, FP32 78, 91 and 68, 80; K = 64 FP64 209, 272 and
+// 181, 222; K = 128 300, 387 and 301, 361, and the small tile is ahead beyond.  64 x
+// 128 FP64 against 64 x 64 on 64 x K x 150000: K = 16 239 and 205 us, 32 292 and 265,
+// 64 359 and 323, 256 770 and 779.
 struct TileCand {
   int cfg;
   double us_k, k0, lat_k;
-  int edge;
+  int edge, deep_k;
 };
-const TileCand kF64Tiles[] = {{FM_TILE_PS_128x128_O2, 0.1257, 30, 0, FM_TILE_128x128_O2_U1},
-                              {FM_TILE_PS_128x256_W8, 0.2520, 30, 0, -1},
-                              {FM_TILE_PS_128x96_O2, 0.0960, 30, 0, -1},
-                              {FM_TILE_128x64, 0.0650, 34, 0, -1},
-                              {FM_TILE_64x128, 0.0645, 34, 0, -1},
-                              {FM_TILE_64x64, 0.0340, 32, 0.037, FM_TILE_64x64},
-                              {FM_TILE_PS_32x32_K32, 0.0103, 50, 0.0129, -1}};
-const TileCand kF32Tiles[] = {{FM_TILE_PS_128x256_W8, 0.1383, 44, 0, -1},
-                              {FM_TILE_PS_128x128_O2, 0.0695, 40, 0, FM_TILE_128x128_W8},
-                              {FM_TILE_128x64, 0.0368, 43, 0, -1},
-                              {FM_TILE_64x128, 0.0368, 43, 0, -1},
-                              {FM_TILE_64x64, 0.0192, 43, 0.0227, FM_TILE_64x64},
-                              {FM_TILE_PS_32x32_K32, 0.0057, 60, 0.0099, -1}};
+const TileCand kF64Tiles[] = {{FM_TILE_PS_128x128_O2, 0.1257, 30, 0, FM_TILE_128x128_O2_U1, 0},
+                              {FM_TILE_PS_128x256_W8, 0.2520, 30, 0, -1, 0},
+                              {FM_TILE_PS_128x96_O2, 0.0960, 30, 0, -1, 0},
+                              {FM_TILE_128x64, 0.0650, 34, 0, -1, 0},
+                              {FM_TILE_64x128, 0.0645, 34, 0, -1, 65},
+                              {FM_TILE_64x64, 0.0340, 32, 0.037, FM_TILE_64x64, 0},
+                              {FM_TILE_PS_32x32_K32, 0.0103, 50, 0.0129, -1, 128}};
+const TileCand kF32Tiles[] = {{FM_TILE_PS_128x256_W8, 0.1383, 44, 0, -1, 0},
+                              {FM_TILE_PS_128x128_O2, 0.0695, 40, 0, FM_TILE_128x128_W8, 0},
+                              {FM_TILE_128x64, 0.0368, 43, 0, -1, 0},
+                              {FM_TILE_64x128, 0.0368, 43, 0, -1, 0},
+                              {FM_TILE_64x64, 0.0192, 43, 0.0227, FM_TILE_64x64, 0},
+                              {FM_TILE_PS_32x32_K32, 0.0057, 60, 0.0099, -1, 128}};
+const int64_t kManyTiles = 16 * 256;  // 64 x 64 tiles: 16 per CU, the range measured
 
 const TileCand* plain_cands(fm_dtype dt, size_t* n) {
   *n = dt == FM_F64 ? sizeof(kF64Tiles) / sizeof(kF64Tiles[0]) : sizeof(kF32Tiles) / sizeof(kF32Tiles[0]);
@@ -507,6 +515,13 @@ double cand_us(fm_dtype dt, const TileCand& c, const std::vector<FmGemmDesc>& pr
   return kLaunchUs + t * (fits ? 1.0 : kEdgePenalty);
 }
 
+bool too_shallow(const TileCand& c, const std::vector<FmGemmDesc>& prods) {
+  if (c.deep_k == 0) return false;
+  int depth = 0;
+  for (const FmGemmDesc& d : prods) depth = std::max(depth, d.K);
+  return depth < c.deep_k && count_tiles(FM_TILE_64x64, prods) > kManyTiles;
+}
+
 // The spread kernels of configuration cfg take the products.
 bool spread_fits(fm_dtype dt, int cfg, const std::vector<FmGemmDesc>& prods) {
   return any_tiles(dt, cfg, prods) || whole_tiles(dt, cfg, prods);
@@ -539,6 +554,7 @@ int best_tile(fm_dtype dt, fm_mode mode, const std::vector<FmGemmDesc>& prods, d
     size_t n;
     const TileCand* c = plain_cands(dt, &n);
     for (size_t i = 0; i < n; ++i) {
+      if (too_shallow(c[i], prods)) continue;
       const bool fits = spread_fits(dt, c[i].cfg, prods);
       const int cfg = fits ? c[i].cfg : c[i].edge;
       if (cfg >= 0) offer(cfg, cand_us(dt, c[i], prods, fits), margin);
@@ -623,7 +639,7 @@ bool carve_full(const Plan& P, int cfg, std::vector<FmGemmDesc>& prods, std::vec
       if (d.N > Nf) st.push_back(gsub(d, 0, Nf, d.M, d.N - Nf));           // right strip, all rows
       if (d.M > Mf && Nf > 0) st.push_back(gsub(d, Mf, 0, d.M - Mf, Nf));  // bottom strip
     }
-    if (core.empty() || st.empty()) continue;
+    if (core.empty() || st.empty() || too_shallow(cands[i], core)) continue;
     if (!spread_fits(P.dtype, cands[i].cfg, core)) continue;
     int cs;
     const double t_strips = set_apart(P.dtype, st, st_odd, &cs);

@@ -131,3 +131,17 @@ def test_strips_of_long_matrices_fit_one_launch(probe):
     for p in [(1 << 28, 2, 3), ((1 << 29) + 4, 6, 3), (3, 2, 1 << 30)]:
         t = _strip_tiles(probe("f64", [p + ("strassen", 1), (64, 64, 65, "strassen", 1)]))
         assert t and max(t) < 1 << 24
+
+
+# ---- large launches of shallow products --------------------------------------------
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_large_shallow_launches_leave_the_smallest_tile(dtype):
+    # seven leaves of 150000 x 32 x 32: 128 x 64 tiles (FmTileCfg 2), not 32 x 32 (35)
+    assert _leaf(300000, 64, 64, dtype, 1) == 2
+    assert _leaf(300000, 64, 16, dtype, 1) == 2
+    assert _leaf(64, 64, 300000, dtype, 1) in (1, 3)
+    # deeper, or few tiles: the smallest tile still
+    assert _leaf(300000, 512, 16, dtype, 1) == 35
+    assert _leaf(64, 64, 64, dtype) == 35
+    if dtype == torch.float64:  # 64 x 64 tiles up to K = 64, 64 x 128 (3) beyond
+        assert [_leaf(128, 2 * k, 300000, dtype, 1) for k in (16, 64, 256)] == [1, 1, 3]
