@@ -48,9 +48,16 @@ __device__ __forceinline__ float mul_rn(float a, float b) { return __fmul_rn(a, 
 __device__ __forceinline__ double add_rn(double a, double b) { return __dadd_rn(a, b); }
 __device__ __forceinline__ float add_rn(float a, float b) { return __fadd_rn(a, b); }
 
+// A work group's lanes take 16 bytes of rows each.  Where a matrix has fewer rows
+// than they cover, 2^lr of them (of a wave's, in the column maxima) go along the
+// rows and the others take further columns.  With all lanes along the rows a B of
+// 7 rows kept 2 of 256 lanes busy, and every 32 columns ended in their own atomics
+// on the same 7 maxima: whole call, strassen one level, 5 x 7 x 1000000 FP32 2300 ->
+// 462 us, FP64 1800 -> 691; 64 x 64 x 100000 354 -> 120, 303 -> 196.
 constexpr int SC_THREADS = 256;
-constexpr int SC_COLS = 32;        // columns of a row-maxima tile
-constexpr int SC_WCOLS = 8;        // columns of a write tile
+constexpr int SC_COLS = 32;        // columns a lane takes in a row-maxima tile
+constexpr int SC_SHORT_COLS = 16;  // the same where lanes share the columns
+constexpr int SC_WCOLS = 8;        // columns a lane takes in a write tile
 constexpr int SC_SEGMENT = 8192;   // rows of a column-maxima segment (one wave)
 template <typename T>
 constexpr int sc_vl() {
@@ -101,65 +108,104 @@ struct MaxArgs {
   const T* pre;
   typename Bits<T>::U* out;
   int tiles_r, tiles;  // tiles along the rows, all tiles
+  int lr;              // lanes along the rows, as a power of two
 };
 
-template <typename T>
-__device__ __forceinline__ void max_tile(const MaxArgs<T>& a, int t) {
+// ALL: every lane along the rows, as constants (1000^3 FP32, whole call: 66 us, 83
+// with them read at run time).
+template <typename T, bool ALL>
+__device__ __forceinline__ void row_max_tile(const MaxArgs<T>& a, int t, T* red) {
   constexpr int VL = Rows<T>::VL;
-  const int tr = t % a.tiles_r, tc = t / a.tiles_r;
-  if (a.rowwise) {
-    const int i0 = (tr * SC_THREADS + (int)threadIdx.x) * VL;
-    if (i0 >= a.rows) return;
-    const int j0 = tc * SC_COLS, j1 = min(a.cols, j0 + SC_COLS), n = a.rows - i0;
-    T mx[VL];
+  const int tr = t % a.tiles_r, tc = t / a.tiles_r, tid = threadIdx.x;
+  // lane r of 2^lr along the rows, g of ng column groups
+  const int lr = ALL ? 8 : a.lr, ng = SC_THREADS >> lr, r = tid & ((1 << lr) - 1), g = tid >> lr;
+  const int64_t i0 = (((int64_t)tr << lr) + r) * VL, j0 = (int64_t)tc * (ALL ? SC_COLS : SC_SHORT_COLS) * ng;
+  const int n = (int)min(a.rows - i0, (int64_t)VL);
+  if (ALL && n <= 0) return;
+  const int left = (int)min(a.cols - j0, (int64_t)(ALL ? SC_COLS : SC_SHORT_COLS) * ng);  // columns of the tile
+  const int cnt = n > 0 ? (left - g + ng - 1) / ng : 0;                                // of this lane
+  const T* p = a.X + i0 + (j0 + g) * a.ld;
+  const T* pre = a.pre + j0 + g;
+  T mx[VL];
 #pragma unroll
-    for (int e = 0; e < VL; ++e) mx[e] = T(0);
+  for (int e = 0; e < VL; ++e) mx[e] = T(0);
 #pragma unroll 8
-    for (int j = j0; j < j1; ++j) {
-      Rows<T> x;
-      x.load(a.X + i0 + (int64_t)j * a.ld, n);
-      const T f = a.pre ? a.pre[j] : T(1);
+  for (int q = 0; q < cnt; ++q) {
+    Rows<T> x;
+    x.load(p + (int64_t)(q * ng) * a.ld, n);
+    const T f = a.pre ? pre[q * ng] : T(1);
 #pragma unroll
-      for (int e = 0; e < VL; ++e) mx[e] = fmax(mx[e], fabs(a.pre ? mul_rn(x.v[e], f) : x.v[e]));
-    }
+    for (int e = 0; e < VL; ++e) mx[e] = fmax(mx[e], fabs(a.pre ? mul_rn(x.v[e], f) : x.v[e]));
+  }
+  if constexpr (!ALL) {  // the column groups' maxima meet in the first group's lanes
 #pragma unroll
-    for (int e = 0; e < VL; ++e)
-      if (e < n) atomicMax(a.out + i0 + e, Bits<T>::of(mx[e]));
-  } else {
-    // one wave per column and segment of rows
-    const int j = tc * (SC_THREADS / 64) + ((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (j >= a.cols) return;
-    const int r0 = tr * SC_SEGMENT, r1 = min(a.rows, r0 + SC_SEGMENT);
-    const T* c = a.X + (int64_t)j * a.ld;
-    T mx = T(0);
+    for (int e = 0; e < VL; ++e) red[e * SC_THREADS + tid] = mx[e];
+    __syncthreads();
+    if (g > 0) return;
+    for (int q = 1; q < ng; ++q)
+#pragma unroll
+      for (int e = 0; e < VL; ++e) mx[e] = fmax(mx[e], red[e * SC_THREADS + (q << lr) + r]);
+  }
+#pragma unroll
+  for (int e = 0; e < VL; ++e)
+    if (e < n) atomicMax(a.out + i0 + e, Bits<T>::of(mx[e]));
+}
+
+template <typename T, bool ALL>
+__device__ __forceinline__ void col_max_tile(const MaxArgs<T>& a, int t) {
+  constexpr int VL = Rows<T>::VL;
+  const int tr = t % a.tiles_r, tc = t / a.tiles_r, tid = threadIdx.x;
+  // 2^lr lanes of a wave per column and segment of rows
+  const int lr = ALL ? 6 : a.lr, lane = tid & ((1 << lr) - 1);
+  const int64_t j = (int64_t)tc * (SC_THREADS >> lr) + (tid >> lr), r0 = (int64_t)tr * SC_SEGMENT;
+  if (j >= a.cols) return;
+  const int len = (int)min(a.rows - r0, (int64_t)SC_SEGMENT);
+  const T* c = a.X + r0 + j * a.ld;
+  const T* pre = a.pre + r0;
+  T mx = T(0);
 #pragma unroll 4
-    for (int i = r0 + lane * VL; i < r1; i += 64 * VL) {
-      Rows<T> x;
-      x.load(c + i, r1 - i);
-      if (a.pre) {
-        Rows<T> f;
-        f.load(a.pre + i, r1 - i);
+  for (int i = lane * VL; i < len; i += VL << lr) {
+    Rows<T> x;
+    x.load(c + i, len - i);
+    if (a.pre) {
+      Rows<T> f;
+      f.load(pre + i, len - i);
 #pragma unroll
-        for (int e = 0; e < VL; ++e) mx = fmax(mx, fabs(mul_rn(x.v[e], f.v[e])));
-      } else {
+      for (int e = 0; e < VL; ++e) mx = fmax(mx, fabs(mul_rn(x.v[e], f.v[e])));
+    } else {
 #pragma unroll
-        for (int e = 0; e < VL; ++e) mx = fmax(mx, fabs(x.v[e]));
-      }
+      for (int e = 0; e < VL; ++e) mx = fmax(mx, fabs(x.v[e]));
     }
+  }
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o));
-    if (lane == 0) atomicMax(a.out + j, Bits<T>::of(mx));
+  for (int o = (1 << lr) >> 1; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o));
+  if (lane == 0) atomicMax(a.out + j, Bits<T>::of(mx));
+}
+
+template <typename T>
+__device__ __forceinline__ void max_tile(const MaxArgs<T>& a, int t, T* red) {
+  if (a.rowwise) {
+    if (a.lr == 8)
+      row_max_tile<T, true>(a, t, red);
+    else
+      row_max_tile<T, false>(a, t, red);
+  } else {
+    if (a.lr == 6)
+      col_max_tile<T, true>(a, t);
+    else
+      col_max_tile<T, false>(a, t);
   }
 }
 
 // A and B in one launch
 template <typename T>
 __global__ void __launch_bounds__(SC_THREADS) fm_max_kernel(MaxArgs<T> a, MaxArgs<T> b) {
+  __shared__ T red[SC_THREADS * Rows<T>::VL];
   const int t = blockIdx.x;
   if (t < a.tiles)
-    max_tile(a, t);
+    max_tile(a, t, red);
   else
-    max_tile(b, t - a.tiles);
+    max_tile(b, t - a.tiles, red);
 }
 
 // Factor arithmetic follows the reference's types: the maxima are doubles
@@ -222,25 +268,36 @@ struct WriteArgs {
   int rows, cols;
   const T *rf, *cf;
   int row_first;
-  int tiles_r, tiles;
+  int tiles_r, tiles, lr;  // as in MaxArgs
 };
 
-template <typename T>
-__device__ __forceinline__ void write_tile(const WriteArgs<T>& a, int t) {
+// This lane's place in tile t of a write launch: its first row, its first column
+// and the distance to the next.
+template <typename T, bool ALL>
+__device__ __forceinline__ void write_place(int t, int tiles_r, int some, int64_t* i0, int64_t* j0, int* step) {
+  const int tr = t % tiles_r, tc = t / tiles_r, tid = threadIdx.x, lr = ALL ? 8 : some;
+  *step = SC_THREADS >> lr;
+  *i0 = (((int64_t)tr << lr) + (tid & ((1 << lr) - 1))) * Rows<T>::VL;
+  *j0 = (int64_t)tc * SC_WCOLS * *step + (tid >> lr);
+}
+
+template <typename T, bool ALL>
+__device__ __forceinline__ void write_tile_lanes(const WriteArgs<T>& a, int t) {
   constexpr int VL = Rows<T>::VL;
-  const int tr = t % a.tiles_r, tc = t / a.tiles_r;
-  const int i0 = (tr * SC_THREADS + (int)threadIdx.x) * VL;
+  int64_t i0, j0;
+  int step;
+  write_place<T, ALL>(t, a.tiles_r, a.lr, &i0, &j0, &step);
   if (i0 >= a.rows) return;
-  const int j0 = tc * SC_WCOLS, n = a.rows - i0;
+  const int n = (int)(a.rows - i0);
   Rows<T> rf;
   if (a.rf) rf.load(a.rf + i0, n);
   Rows<T> x[SC_WCOLS];
 #pragma unroll
   for (int u = 0; u < SC_WCOLS; ++u)  // columns past the end read the last one, not stored
-    x[u].load(a.X + i0 + (int64_t)min(j0 + u, a.cols - 1) * a.ldx, n);
+    x[u].load(a.X + i0 + min(j0 + u * step, (int64_t)a.cols - 1) * a.ldx, n);
 #pragma unroll
   for (int u = 0; u < SC_WCOLS; ++u) {
-    const int j = j0 + u;
+    const int64_t j = j0 + u * step;
     if (j >= a.cols) break;
     const T c = a.cf ? a.cf[j] : T(1);
 #pragma unroll
@@ -251,8 +308,16 @@ __device__ __forceinline__ void write_tile(const WriteArgs<T>& a, int t) {
       if (!a.row_first && a.rf) v = mul_rn(v, rf.v[e]);
       x[u].v[e] = v;
     }
-    x[u].store(a.Y + i0 + (int64_t)j * a.ldy, n);
+    x[u].store(a.Y + i0 + j * a.ldy, n);
   }
+}
+
+template <typename T>
+__device__ __forceinline__ void write_tile(const WriteArgs<T>& a, int t) {
+  if (a.lr == 8)
+    write_tile_lanes<T, true>(a, t);
+  else
+    write_tile_lanes<T, false>(a, t);
 }
 
 template <typename T>
@@ -265,25 +330,26 @@ __global__ void __launch_bounds__(SC_THREADS) fm_write_kernel(WriteArgs<T> a, Wr
 }
 
 // C[i, j] = alpha * ((P[i, j] * r[i]) * s[j]) + beta * C[i, j]; P may be C
-template <typename T>
+template <typename T, bool ALL>
 __global__ void __launch_bounds__(SC_THREADS) fm_post_kernel(const T* P, int64_t ldp, T* C, int64_t ldc,
                                                              int rows, int cols, const T* r, const T* s,
-                                                             T alpha, T beta, int tiles_r) {
+                                                             T alpha, T beta, int tiles_r, int lr) {
   constexpr int VL = Rows<T>::VL;
-  const int tr = (int)blockIdx.x % tiles_r, tc = (int)blockIdx.x / tiles_r;
-  const int i0 = (tr * SC_THREADS + (int)threadIdx.x) * VL;
+  int64_t i0, j0;
+  int step;
+  write_place<T, ALL>(blockIdx.x, tiles_r, lr, &i0, &j0, &step);
   if (i0 >= rows) return;
-  const int j0 = tc * SC_WCOLS, n = rows - i0;
+  const int n = (int)(rows - i0);
   Rows<T> rf, x[SC_WCOLS];
   rf.load(r + i0, n);
 #pragma unroll
-  for (int u = 0; u < SC_WCOLS; ++u) x[u].load(P + i0 + (int64_t)min(j0 + u, cols - 1) * ldp, n);
+  for (int u = 0; u < SC_WCOLS; ++u) x[u].load(P + i0 + min(j0 + u * step, (int64_t)cols - 1) * ldp, n);
 #pragma unroll
   for (int u = 0; u < SC_WCOLS; ++u) {
-    const int j = j0 + u;
+    const int64_t j = j0 + u * step;
     if (j >= cols) break;
     const T c = s[j];
-    T* out = C + i0 + (int64_t)j * ldc;
+    T* out = C + i0 + j * ldc;
     Rows<T> old;
     if (beta != T(0)) old.load(out, n);
 #pragma unroll
@@ -299,20 +365,32 @@ __global__ void __launch_bounds__(SC_THREADS) fm_post_kernel(const T* P, int64_t
 
 inline unsigned blocks_for(int n) { return (unsigned)((n + 255) / 256); }
 
+// lanes along `rows` rows, as a power of two up to max_log
+template <typename T>
+int row_lanes(int rows, int max_log) {
+  int l = 0;
+  while (l < max_log && ((int64_t)sc_vl<T>() << l) < rows) ++l;
+  return l;
+}
+
 template <typename T>
 MaxArgs<T> max_args(const T* X, int64_t ld, int rows, int cols, int rowwise, const T* pre, T* out) {
-  MaxArgs<T> a{X, ld, rows, cols, rowwise, pre, reinterpret_cast<typename Bits<T>::U*>(out), 0, 0};
-  const int tile_r = rowwise ? SC_THREADS * sc_vl<T>() : SC_SEGMENT;
-  const int tile_c = rowwise ? SC_COLS : SC_THREADS / 64;
-  a.tiles_r = (rows + tile_r - 1) / tile_r;
-  a.tiles = a.tiles_r * ((cols + tile_c - 1) / tile_c);
+  MaxArgs<T> a{X, ld, rows, cols, rowwise, pre, reinterpret_cast<typename Bits<T>::U*>(out), 0, 0, 0};
+  a.lr = row_lanes<T>(rows, rowwise ? 8 : 6);
+  const int groups = SC_THREADS >> a.lr;
+  const int64_t tile_r = rowwise ? sc_vl<T>() << a.lr : SC_SEGMENT;
+  const int64_t tile_c = rowwise ? (groups > 1 ? SC_SHORT_COLS : SC_COLS) * groups : groups;
+  a.tiles_r = (int)((rows + tile_r - 1) / tile_r);
+  a.tiles = a.tiles_r * (int)((cols + tile_c - 1) / tile_c);
   return a;
 }
 
 template <typename T>
-int write_tiles(int rows, int cols, int* tiles_r) {
-  *tiles_r = (rows + SC_THREADS * sc_vl<T>() - 1) / (SC_THREADS * sc_vl<T>());
-  return *tiles_r * ((cols + SC_WCOLS - 1) / SC_WCOLS);
+int write_tiles(int rows, int cols, int* tiles_r, int* lr) {
+  *lr = row_lanes<T>(rows, 8);
+  const int64_t tile_r = sc_vl<T>() << *lr, tile_c = SC_WCOLS * (SC_THREADS >> *lr);
+  *tiles_r = (int)((rows + tile_r - 1) / tile_r);
+  return *tiles_r * (int)((cols + tile_c - 1) / tile_c);
 }
 
 // Scaled copies of A and B, r and s.
@@ -343,10 +421,10 @@ hipError_t run_scaling(const FmScaleArgs& a, hipStream_t st) {
       hipLaunchKernelGGL(fm_inner_factors<T>, dim3(blocks_for(k)), dim3(256), 0, st, ga, gb, k);
   };
   auto write = [&](const T* ra, const T* ca, const T* rb, const T* cb) {
-    WriteArgs<T> wa{X, ldx, A, a.lda, m, k, ra, ca, outer_first, 0, 0};
-    WriteArgs<T> wb{Y, ldy, B, a.ldb, k, n, rb, cb, !outer_first, 0, 0};
-    wa.tiles = write_tiles<T>(m, k, &wa.tiles_r);
-    wb.tiles = write_tiles<T>(k, n, &wb.tiles_r);
+    WriteArgs<T> wa{X, ldx, A, a.lda, m, k, ra, ca, outer_first, 0, 0, 0};
+    WriteArgs<T> wb{Y, ldy, B, a.ldb, k, n, rb, cb, !outer_first, 0, 0, 0};
+    wa.tiles = write_tiles<T>(m, k, &wa.tiles_r, &wa.lr);
+    wb.tiles = write_tiles<T>(k, n, &wb.tiles_r, &wb.lr);
     hipLaunchKernelGGL(fm_write_kernel<T>, dim3(wa.tiles + wb.tiles), dim3(SC_THREADS), 0, st, wa, wb);
   };
   auto init = [&](int first) {
@@ -380,11 +458,12 @@ hipError_t fm_scaling_run(int dtype_f64, const FmScaleArgs& a, hipStream_t s) {
 template <typename T>
 static void post(const void* P, int64_t ldp, void* C, int64_t ldc, int rows, int cols, const void* r,
                  const void* sv, double alpha, double beta, hipStream_t s) {
-  int tiles_r;
-  const int tiles = write_tiles<T>(rows, cols, &tiles_r);
-  hipLaunchKernelGGL(fm_post_kernel<T>, dim3(tiles), dim3(SC_THREADS), 0, s, reinterpret_cast<const T*>(P), ldp,
+  int tiles_r, lr;
+  const int tiles = write_tiles<T>(rows, cols, &tiles_r, &lr);
+  auto* kernel = lr == 8 ? &fm_post_kernel<T, true> : &fm_post_kernel<T, false>;
+  hipLaunchKernelGGL(kernel, dim3(tiles), dim3(SC_THREADS), 0, s, reinterpret_cast<const T*>(P), ldp,
                      reinterpret_cast<T*>(C), ldc, rows, cols, reinterpret_cast<const T*>(r),
-                     reinterpret_cast<const T*>(sv), (T)alpha, (T)beta, tiles_r);
+                     reinterpret_cast<const T*>(sv), (T)alpha, (T)beta, tiles_r, lr);
 }
 
 hipError_t fm_scaling_post(int dtype_f64, const void* P, int64_t ldp, void* C, int64_t ldc,

@@ -40,7 +40,8 @@ def _passes(A, B, kind, steps):
 @pytest.mark.parametrize("kind,steps", [("outside_inside", 1), ("inside_outside", 2), ("inside", 1),
                                         ("outside", 2), ("outside_inside", 0)])
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
-@pytest.mark.parametrize("shape", [(1, 1, 1), (5, 33, 7), (513, 31, 65), (1027, 70, 9), (8195, 3, 33),
+@pytest.mark.parametrize("shape", [(2, 3, 4099), (4099, 3, 2), (17, 16, 1040), (255, 9, 263), (64, 65, 4097),
+                                   (3, 8193, 5), (1, 1, 1), (5, 33, 7), (513, 31, 65), (1027, 70, 9), (8195, 3, 33),
                                    (34, 8193, 1030)])
 def test_passes_bit_identical(fm, shape, dtype, kind, steps):
     m, k, n = shape
@@ -68,3 +69,18 @@ def test_passes_bit_identical(fm, shape, dtype, kind, steps):
         C = fm.fastmatmul_scaled("strassen", dev(A, pad), dev(B, pad), dev(C0, pad), 0, alpha=alpha,
                                  beta=beta, scaling=kind, scaling_steps=steps).cpu().numpy()
         assert np.array_equal(C, want), (pad, np.abs(C - want).max())
+
+
+def test_very_wide_matrices_fit_one_launch(fm):
+    """Two rows and 2^27 columns: the lanes of a work group share the columns, so
+    a pass takes 2^16 work groups (one per 8 columns would be 2^24, whose 2^32
+    threads no launch takes)."""
+    n = (1 << 27) + 8
+    B = fm.empty(2, n, torch.float32, DEV)
+    B.copy_(torch.arange(n, device=DEV, dtype=torch.float32).remainder_(251.0))
+    B[1] -= 100.0
+    A = fm.col_major(torch.tensor([[2.0, -3.0], [5.0, 7.0]], device=DEV))
+    C = fm.fastmatmul_scaled("strassen", A, B, None, 0, scaling_steps=0)
+    for i in range(2):  # whole numbers, exact in FP32
+        want = A[i, 0] * B[0] + A[i, 1] * B[1]
+        assert torch.equal(C[i], want)
