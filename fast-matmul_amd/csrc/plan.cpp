@@ -1083,7 +1083,10 @@ void group_sequence(std::vector<std::vector<Launch>*> seqs, std::vector<Launch>&
       Launch& L = (*sq)[i];
       const bool stage = L.kind == LK_S || L.kind == LK_T || L.kind == LK_W || L.kind == LK_S2 ||
                          L.kind == LK_T2 || L.kind == LK_W2;
-      if (!stage) {  // a depth-first child's leaf launch: kept as it is
+      // A depth-first child's launches come from a plan of its own: its leaves,
+      // its shared launches and its W stages that add K remainders have
+      // descriptors that group_stages does not carry, and stay as they are.
+      if (!stage || L.nupd > 0 || L.planes) {
         out.push_back(std::move(L));
         continue;
       }

@@ -3,7 +3,8 @@
 //   plan_probe f64|f32 [problem ...]
 // problem: m,k,n[,algorithm,steps[,depth-first levels]]
 //   gemm cfg any full products tiles max_k_of_products
-//   thin products tiles | stage kind nodes k_updates
+//   thin products tiles
+//   stage kind nodes k_updates peeling_products
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
@@ -57,7 +58,7 @@ int main(int argc, char** argv) {
     } else if (L.kind == LK_THIN) {
       printf("thin %d %d\n", L.th.ndesc, L.th.total_tiles);
     } else {
-      printf("stage %d %d %d\n", (int)L.kind, L.st.nodes, L.nupd);
+      printf("stage %d %d %d %d\n", (int)L.kind, L.st.nodes, L.nupd, (int)L.tdescs.size());
     }
   }
   return 0;

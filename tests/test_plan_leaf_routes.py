@@ -145,3 +145,27 @@ def test_large_shallow_launches_leave_the_smallest_tile(dtype):
     assert _leaf(64, 64, 64, dtype) == 35
     if dtype == torch.float64:  # 64 x 64 tiles up to K = 64, 64 x 128 (3) beyond
         assert [_leaf(128, 2 * k, 300000, dtype, 1) for k in (16, 64, 256)] == [1, 1, 3]
+
+
+# ---- depth-first problems of a batch -------------------------------------------------
+def _peeling_products(launches):
+    """Peeling products in launches of their own and in W stages (the K updates among them)."""
+    return sum(l[1] for l in launches if l[0] == "thin") + sum(l[4] for l in launches if l[0] == "stage")
+
+
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+@pytest.mark.parametrize("dfs", [0, 1, 2])
+def test_grouped_problems_keep_every_peeling_product(probe, dtype, dfs):
+    # remainders of every dimension at both levels; a depth-first child's W
+    # stage adds its K remainder itself, also where the same stage of another
+    # problem stands beside it
+    ps = [(2 * (2 * 130 + 1) + 1, 2 * (2 * 90 + 1) + 1, 2 * (2 * 70 + 1) + 1, "strassen", 2, dfs),
+          (2 * (2 * 60 + 1) + 1, 2 * (2 * 80 + 1) + 1, 2 * (2 * 50 + 1) + 1, "strassen", 2, dfs)]
+    alone = [_peeling_products(probe(dtype, [p])) for p in ps]
+    assert alone == [3 + 7 * 3, 3 + 7 * 3]
+    assert _peeling_products(probe(dtype, ps)) == sum(alone)
+    # K remainders alone: the W stages that add them have no strips beside them
+    ps = [(4 * m, 2 * (2 * k + 1), 4 * n, "strassen", 2, dfs) for m, k, n in [(130, 90, 70), (60, 80, 50)]]
+    alone = [_peeling_products(probe(dtype, [p])) for p in ps]
+    assert alone == [7, 7]
+    assert _peeling_products(probe(dtype, ps)) == sum(alone)
