@@ -847,11 +847,12 @@ fm_status build_subplan(fm_dtype dt, const Problem& p, int64_t ws_base, SubPlan&
   // the leaves' preparation grid would fit one launch (else they split on the
   // fly, on the FP32 operands), for operands that need no padding, and for
   // padded ones
-  // - of more than 128 rows: 256-row padding then takes no more workspace than
-  //   FP32 outputs with planes padded to 128;
+  // - of more than 128 rows and a K of one slice or more: padding then takes no
+  //   more workspace than FP32 outputs with planes padded to 128 rows (leaves of
+  //   65536 x 1 x 1 and 65536 x 2 x 1 took 6% and 4% more);
   // - of 2^18 elements, one wave per SIMD at 4 elements a lane: a lane forms
   //   every output of its elements in turn, and a smaller stage is that serial
-  //   chain.
+  //   chain; and fewer than 2^31 with the padding, as the kernel counts them.
   // Measured, separate -> stage-written: strassen two levels 600^3 51 -> 81 us,
   // 1036^3 73 -> 94, 2048^3 211 -> 154, 3448^3 682 -> 589, 10008^3
   // 9917 -> 8710; grey424_26_206 two levels 12000^3 23222 -> 17516.
@@ -863,7 +864,10 @@ fm_status build_subplan(fm_dtype dt, const Problem& p, int64_t ws_base, SubPlan&
     const double wgs = leaves * (double)((d.m + d.n + 126) / 64) * (double)((d.k + 127) / 128);
     const bool fits = wgs <= 2147483647.0;
     const bool whole = d.m % 256 == 0 && d.n % 256 == 0 && d.k % 32 == 0;
-    auto padded = [&](int64_t rows) { return rows > 128 && align_up(rows, 256) * align_up(d.k, 32) >= (1 << 18); };
+    auto padded = [&](int64_t rows) {
+      const int64_t elems = align_up(rows, 256) * align_up(d.k, 32);
+      return rows > 128 && d.k >= 32 && elems >= (1 << 18) && elems < (int64_t(1) << 31);
+    };
     s_pl = fits && (whole || padded(d.m)) && s2[L - 2] && alg->s2p_f != nullptr;
     t_pl = fits && (whole || padded(d.n)) && t2[L - 2] && alg->t2p_f != nullptr;
   }

@@ -345,7 +345,7 @@ fm_status fm_set_schedule(int dfs_levels, size_t workspace_limit, int split_rema
  * have no peeling between them, one launch forms the deeper level's S (T)
  * operands straight from the upper level's, without storing the middle
  * level.  With FM_MODE_SPLIT_BF16 leaves (FP32) whose rows are multiples of
- * 256 and K of 32, or which are large enough (padded to that, 2^18 elements
+ * 256 and K of 32, or which are large enough (K at least 32; padded to that, 2^18 elements
  * an operand), the last such stage also writes the leaf operands as bf16
  * slice planes, which the leaf kernels read, instead of FP32 blocks that a
  * preparation pass would cut into planes.  on: 1 (default), 2

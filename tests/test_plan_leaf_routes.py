@@ -169,3 +169,32 @@ def test_grouped_problems_keep_every_peeling_product(probe, dtype, dfs):
     alone = [_peeling_products(probe(dtype, [p])) for p in ps]
     assert alone == [7, 7]
     assert _peeling_products(probe(dtype, ps)) == sum(alone)
+
+
+# ---- stage-written slice planes ------------------------------------------------------
+def _split(alg, m, k, n, fusion):
+    fastmm.set_stage_fusion(fusion)
+    try:
+        return fastmm.plan_info(alg, m, k, n, 2, dtype=torch.float32, mode="split_bf16")
+    finally:
+        fastmm.set_stage_fusion(True)
+
+
+@pytest.mark.parametrize("alg,m,k,n", [("strassen", 1 << 18, 4, 4), ("strassen", 1 << 20, 8, 4),
+                                       ("grey223_11_50", 254665, 17, 387), ("grey234_20_144", 35873, 9, 49),
+                                       ("grey232_11_50", 244620, 74, 496), ("grey332_15_103", 604153, 9, 348),
+                                       ("strassen", 1 << 16, 128, 4), ("strassen", 3448, 3448, 3448)])
+def test_padded_planes_take_no_more_workspace(alg, m, k, n):
+    """Planes written by the S/T stage, padded to whole tiles and slices,
+    against planes cut from FP32 operands by the separate pass."""
+    assert _split(alg, m, k, n, 1)["workspace_bytes"] <= _split(alg, m, k, n, 2)["workspace_bytes"]
+
+
+def test_padded_planes_stay_within_32_bit_counts():
+    # leaves of 2^27 x 1: 2^32 elements with K padded to a slice; the separate pass prepares them
+    assert _split("strassen", 1 << 29, 4, 4, 1)["prep_bytes"] == _split("strassen", 1 << 29, 4, 4, 2)["prep_bytes"]
+    # leaves of 2^25 + 256 rows and 33 columns: past 2^31 with K padded to two slices
+    m = 4 * ((1 << 25) + 256)
+    assert _split("strassen", m, 4 * 33, 4, 1)["prep_bytes"] == _split("strassen", m, 4 * 33, 4, 2)["prep_bytes"]
+    # and the path itself is still taken
+    assert _split("strassen", 3448, 3448, 3448, 1)["prep_bytes"] < _split("strassen", 3448, 3448, 3448, 2)["prep_bytes"]
