@@ -26,6 +26,8 @@ namespace {
 // Update of C: one row per lane, 16 columns.
 constexpr int UPD_COLS = 16;
 
+// KT: K, or 0 for a K beyond FM_THIN_MAX, read column by column; the sums run
+// over K in the same order.
 template <typename T, int KT>
 __device__ __forceinline__ void thin_k(const FmThinDesc& d, int tm, int tn, fm_gptr<const T> A,
                                        fm_gptr<const T> B, fm_gptr<T> C) {
@@ -33,9 +35,20 @@ __device__ __forceinline__ void thin_k(const FmThinDesc& d, int tm, int tn, fm_g
   if (i >= d.M) return;
   const T alpha = (T)d.alpha, beta = (T)d.beta;
   const int64_t ldb = d.b.ld, ldc = d.c.ld;
-  T a[KT];
+  T a[KT > 0 ? KT : 1], sum[UPD_COLS];
+  if constexpr (KT > 0) {
 #pragma unroll
-  for (int q = 0; q < KT; ++q) a[q] = A[i + q * d.a.ld];
+    for (int q = 0; q < KT; ++q) a[q] = A[i + q * d.a.ld];
+  } else {
+#pragma unroll
+    for (int u = 0; u < UPD_COLS; ++u) sum[u] = T(0);
+    for (int q = 0; q < d.K; ++q) {
+      a[0] = A[i + q * d.a.ld];
+#pragma unroll
+      for (int u = 0; u < UPD_COLS; ++u)
+        sum[u] = fma(a[0], (T)B[q + (int64_t)min(j0 + u, d.N - 1) * ldb], sum[u]);
+    }
+  }
   C += i;
   // columns past N read column N - 1 again and are not stored: every load of
   // the tile is in flight at once
@@ -49,8 +62,12 @@ __device__ __forceinline__ void thin_k(const FmThinDesc& d, int tm, int tn, fm_g
     const int j = j0 + u;
     if (j >= d.N) break;
     T s = T(0);
+    if constexpr (KT > 0) {
 #pragma unroll
-    for (int q = 0; q < KT; ++q) s = fma(a[q], (T)B[q + (int64_t)j * ldb], s);
+      for (int q = 0; q < KT; ++q) s = fma(a[q], (T)B[q + (int64_t)j * ldb], s);
+    } else {
+      s = sum[u];
+    }
     T r = alpha * s;
     if (beta != T(0)) r = fma(beta, c[u], r);
     C[(int64_t)j * ldc] = r;
@@ -82,7 +99,9 @@ __global__ void __launch_bounds__(FM_THIN_THREADS) fm_thin_kernel(FmThinArgs arg
   const fm_gptr<const T> A = fm_global(reinterpret_cast<const T*>(fm_base(args.bases, d.a.role)) + d.a.off);
   const fm_gptr<const T> B = fm_global(reinterpret_cast<const T*>(fm_base(args.bases, d.b.role)) + d.b.off);
   const fm_gptr<T> C = fm_global(reinterpret_cast<T*>(fm_base(args.bases, d.c.role)) + d.c.off);
-  if (d.kind == FM_THIN_K)
+  if (d.kind == FM_THIN_K && d.K > FM_THIN_MAX)
+    thin_k<T, 0>(d, tm, tn, A, B, C);
+  else if (d.kind == FM_THIN_K)
     thin_dispatch<FM_THIN_MAX>(d.K, [&](auto v) { thin_k<T, decltype(v)::value>(d, tm, tn, A, B, C); });
   else if (d.kind == FM_THIN_N)
     thin_dispatch<FM_THIN_MAX>(d.N, [&](auto v) { thin_n<T, decltype(v)::value>(d, tm, A, B, C, red); });

@@ -1,5 +1,5 @@
 // gemm_thin.hpp -- dynamic-peeling products: one dimension is the remainder of
-// a block split (at most FM_THIN_MAX), the others are a node's full size.
+// a block split, the others are a node's full size.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -7,14 +7,18 @@
 
 #include "alg_desc.hpp"
 
-// largest remainder of a block split the kernels are built for (a split into
-// at most FM_THIN_MAX + 1 blocks)
-constexpr int FM_THIN_MAX = 7;
+// Largest thin dimension the kernels are built for: the remainder of a split into
+// FM_THIN_MAX + 1 blocks, the finest of the shipped tables.  Wider strips are
+// several products; a K beyond it is summed by a loop.  (Each further value costs
+// every FP64 strip registers: built up to 7, 182 of them, two waves a SIMD.)
+constexpr int FM_THIN_MAX = 5;
+// the largest thin dimension of a split into s blocks, as the kernels take it
+constexpr int fm_thin_limit(int s) { return s <= 1 ? 1 : s - 1 > FM_THIN_MAX ? FM_THIN_MAX : s - 1; }
 constexpr int FM_THIN_THREADS = 256;
 
 // which dimension is thin, i.e. which of the three peeling products it is
 enum FmThinKind : int32_t {
-  FM_THIN_K = 0,  // C (+)= A B with K <= FM_THIN_MAX: an update of all of C
+  FM_THIN_K = 0,  // C (+)= A B with a thin K: an update of all of C
   FM_THIN_N = 1,  // N <= FM_THIN_MAX columns: reads A once
   FM_THIN_M = 2,  // M <= FM_THIN_MAX rows: reads B once
 };

@@ -116,7 +116,9 @@ Launch stage_launch(fm_dtype dt, LaunchKind kind, const FmAlgDesc* alg, std::vec
   return L;
 }
 
-// Peeling products of one node (linalg/linalg.hpp:201-244).
+// Peeling products of one node (linalg/linalg.hpp:201-244).  Strips wider than the
+// thin kernels take (remainders of a split into more than FM_THIN_MAX + 1 blocks)
+// are several products.
 void peel_descs(const Node& nd, const Dims& D, int am, int ak, int an, double beta,
                 std::vector<FmThinDesc>& out) {
   const int64_t erA = D.m % am, ecA = D.k % ak, ecB = D.n % an;
@@ -140,12 +142,15 @@ void peel_descs(const Node& nd, const Dims& D, int am, int ak, int an, double be
     mk(FM_THIN_K, op_sub(nd.a, 0, kk), op_sub(nd.b, kk, 0), nd.c, row_dim, col_dim, ecA, 1.0);
   }
   if (ecB > 0) {
-    const int64_t s = D.n - ecB;
-    mk(FM_THIN_N, nd.a, op_sub(nd.b, 0, s), op_sub(nd.c, 0, s), D.m, ecB, D.k, beta);
+    for (int64_t s = D.n - ecB; s < D.n; s += FM_THIN_MAX)
+      mk(FM_THIN_N, nd.a, op_sub(nd.b, 0, s), op_sub(nd.c, 0, s), D.m, std::min<int64_t>(D.n - s, FM_THIN_MAX), D.k,
+         beta);
   }
   if (erA > 0) {
-    const int64_t s = D.m - erA, nc = D.n - ecB;
-    mk(FM_THIN_M, op_sub(nd.a, s, 0), nd.b, op_sub(nd.c, s, 0), erA, nc, D.k, beta);
+    const int64_t nc = D.n - ecB;
+    for (int64_t s = D.m - erA; s < D.m; s += FM_THIN_MAX)
+      mk(FM_THIN_M, op_sub(nd.a, s, 0), nd.b, op_sub(nd.c, s, 0), std::min<int64_t>(D.m - s, FM_THIN_MAX), nc, D.k,
+         beta);
   }
 }
 
@@ -800,8 +805,6 @@ fm_status build_subplan(fm_dtype dt, const Problem& p, int64_t ws_base, SubPlan&
     return FM_OK;
   }
   const FmAlgDesc* alg = p.alg;
-  if (std::max(alg->m, std::max(alg->k, alg->n)) > FM_THIN_MAX + 1)
-    return set_err(FM_ERR_UNSUPPORTED, "block split finer than the peeling kernels take");
   const int L = p.steps;
   std::vector<Dims> dims(L + 1);
   dims[0] = {p.m, p.k, p.n};
@@ -1147,17 +1150,18 @@ void append_pre(std::vector<Launch>& pre, std::vector<Launch>& out, fm_dtype dt)
 }
 
 // Append one problem's W stage of a level and the level's peeling products: a
-// one-level W stage adds the K remainders itself, and takes the strips into its
-// launch where both are small.
+// one-level W stage adds the K remainders itself (up to the K split its kernel is
+// built for), and takes the strips into its launch where both are small.
 void append_w(Launch W, std::vector<FmThinDesc> peel, std::vector<Launch>& out, fm_dtype dt) {
   std::vector<FmThinDesc> strips;
-  if (W.kind == LK_W) {
+  const bool adds = W.kind == LK_W && W.alg->k <= FM_THIN_MAX + 1;
+  if (adds) {
     for (const FmThinDesc& d : peel)
       if (d.kind == FM_THIN_K) W.tdescs.push_back(d);
     W.nupd = (int)W.tdescs.size();  // one per node, in node order, or none
   }
   for (const FmThinDesc& d : peel)
-    if (W.kind != LK_W || d.kind != FM_THIN_K) strips.push_back(d);
+    if (!adds || d.kind != FM_THIN_K) strips.push_back(d);
   if (strips.empty()) {
     out.push_back(std::move(W));
     return;
@@ -1165,7 +1169,8 @@ void append_w(Launch W, std::vector<FmThinDesc> peel, std::vector<Launch>& out, 
   Launch T = thin_launch(std::move(strips), dt);
   double bytes = 0;
   for (const FmThinDesc& d : T.tdescs) bytes += (double)elem_size(dt) * ((double)d.M * d.K + (double)d.K * d.N);
-  if (W.kind == LK_W && T.th.uniform && bytes <= kSmallWBytes && stage_bytes1(W, dt) <= kSmallWBytes) {
+  const bool k_apart = T.tdescs[0].kind == FM_THIN_K;  // it updates what W writes
+  if (W.kind == LK_W && !k_apart && T.th.uniform && bytes <= kSmallWBytes && stage_bytes1(W, dt) <= kSmallWBytes) {
     W.kind = LK_WS;
     W.th = T.th;
     W.tdescs.insert(W.tdescs.end(), T.tdescs.begin(), T.tdescs.end());

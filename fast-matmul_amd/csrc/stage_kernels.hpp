@@ -151,7 +151,7 @@ __device__ __forceinline__ void fm_w_body(const FmStageArgs& a, int q, uint32_t 
   const int64_t ld = op.ld, rows = nv.rows, cols = nv.cols, out_ld = nv.out_ld, slab = nv.out_slab;
   const T beta = (T)nv.beta;
   const double x = nv.x;
-  constexpr int KM = Cmb::k > 1 ? Cmb::k - 1 : 1;  // largest remainder of K
+  constexpr int KM = fm_thin_limit(Cmb::k);  // largest remainder of K
   FmThinDesc u;
   fm_gptr<const T> ua = nullptr, ub = nullptr;
   if constexpr (UPD) {
@@ -237,7 +237,7 @@ __global__ void __launch_bounds__(FM_STAGE_THREADS) fm_w_stage(FmStageArgs a) {
 template <class Cmb, typename T, bool BETA, bool UPD>
 __global__ void __launch_bounds__(FM_STAGE_THREADS) fm_w_strips(FmStageArgs a, FmThinArgs p, uint32_t gw) {
   static_assert(FM_STAGE_THREADS == FM_THIN_THREADS, "one work group size");
-  constexpr int NM = Cmb::n > 1 ? Cmb::n - 1 : 1, MM = Cmb::m > 1 ? Cmb::m - 1 : 1;
+  constexpr int NM = fm_thin_limit(Cmb::n), MM = fm_thin_limit(Cmb::m);
   __shared__ T red[NM * FM_THIN_THREADS];
   const uint32_t w = blockIdx.x, nw = gw * (uint32_t)a.nodes;
   if (w < nw) {

@@ -1,10 +1,12 @@
 // Plans of several problems, built on the host with the library's own planner
 // and printed one launch a line:
 //   plan_probe f64|f32 [problem ...]
-// problem: m,k,n[,algorithm,steps[,depth-first levels]]
+// problem: m,k,n[,algorithm,steps[,depth-first levels]]; the algorithm blocks:MxKxN is
+// the classical product of an M x K by K x N split (a plan only: it has no kernels)
 //   gemm cfg any full products tiles max_k_of_products
 //   thin products tiles
 //   stage kind nodes k_updates peeling_products
+//   peel kind M N K c_offset c_ld (each product of the launch above)
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
@@ -17,6 +19,32 @@
 using namespace fmplan;
 
 extern const FmAlgDesc* fm_find_alg(const char* name);
+
+namespace {
+double one(int, double) { return 1.0; }
+
+FmAlgDesc* classical(int m, int k, int n) {
+  FmAlgDesc* d = new FmAlgDesc();
+  memset(d, 0, sizeof(*d));
+  d->name = "blocks";
+  d->m = m;
+  d->k = k;
+  d->n = n;
+  d->R = m * k * n;
+  int *kind = new int[(size_t)d->R](), *a = new int[(size_t)d->R], *b = new int[(size_t)d->R];
+  for (int r = 0, i = 0; i < m; ++i)
+    for (int j = 0; j < n; ++j)
+      for (int q = 0; q < k; ++q, ++r) {
+        a[r] = i * k + q;
+        b[r] = q * n + j;
+      }
+  d->a_kind = d->b_kind = kind;
+  d->a_index = a;
+  d->b_index = b;
+  d->a_coef = d->b_coef = one;
+  return d;
+}
+}  // namespace
 
 int main(int argc, char** argv) {
   const fm_dtype dt = strcmp(argv[1], "f64") == 0 ? FM_F64 : FM_F32;
@@ -35,7 +63,11 @@ int main(int argc, char** argv) {
     p.role_b = 5 + 3 * i;
     p.role_c = 6 + 3 * i;
     if (f.size() > 4) {
-      p.alg = fm_find_alg(f[3].c_str());
+      int bm, bk, bn;
+      if (sscanf(f[3].c_str(), "blocks:%dx%dx%d", &bm, &bk, &bn) == 3)
+        p.alg = classical(bm, bk, bn);
+      else
+        p.alg = fm_find_alg(f[3].c_str());
       p.steps = atoi(f[4].c_str());
       if (!p.alg) return 2;
     }
@@ -60,6 +92,8 @@ int main(int argc, char** argv) {
     } else {
       printf("stage %d %d %d %d\n", (int)L.kind, L.st.nodes, L.nupd, (int)L.tdescs.size());
     }
+    for (const FmThinDesc& d : L.tdescs)
+      printf("peel %d %d %d %d %lld %lld\n", (int)d.kind, d.M, d.N, d.K, (long long)d.c.off, (long long)d.c.ld);
   }
   return 0;
 }

@@ -5,6 +5,9 @@ A's rows and columns inside the block split are zero except where a peeling
 product reads them, so the recursion contributes exact zeros and, on integer
 data, every element of C is an exact integer: the comparison is bit for bit,
 whatever the order of the sums."""
+import os
+import subprocess
+
 import numpy as np
 import pytest
 import torch
@@ -114,3 +117,25 @@ def test_peeling_in_a_batch_of_unequal_problems(fm):
     torch.cuda.synchronize()
     for p, s in zip(probs, single):
         assert torch.equal(p["C"], s)
+
+
+@pytest.fixture(scope="module")
+def thin_k_probe(tmp_path_factory):
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    exe = str(tmp_path_factory.mktemp("thin") / "thin_k_probe")
+    lib = os.path.join(root, "fast-matmul_amd", "fastmm")
+    subprocess.check_call(
+        ["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(root, "include"),
+         "-I", os.path.join(root, "fast-matmul_amd", "csrc"), "-I", "/opt/rocm/include",
+         os.path.join(root, "tests", "cpp", "thin_k_probe.cpp"), "-o", exe, "-L", lib, "-lfastmm",
+         "-L", "/opt/rocm/lib", "-lamdhip64", "-Wl,-rpath," + lib + ":/opt/rocm/lib"])
+    return exe
+
+
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+def test_k_update_of_a_split_finer_than_the_tables(fm, thin_k_probe, dtype):
+    """A K remainder of 5 (the last with a kernel of its own), and beyond it,
+    where the update loops over K: no shipped table splits K so finely, so
+    the kernel is called by itself."""
+    for M, N, K, beta in [(300, 37, 5, 1), (300, 37, 6, 1), (257, 16, 9, 0), (1, 1, 20, 1), (255, 33, 31, -2)]:
+        subprocess.check_call([thin_k_probe, dtype, str(M), str(N), str(K), str(beta)], timeout=60)

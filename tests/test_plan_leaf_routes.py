@@ -198,3 +198,45 @@ def test_padded_planes_stay_within_32_bit_counts():
     assert _split("strassen", m, 4 * 33, 4, 1)["prep_bytes"] == _split("strassen", m, 4 * 33, 4, 2)["prep_bytes"]
     # and the path itself is still taken
     assert _split("strassen", 3448, 3448, 3448, 1)["prep_bytes"] < _split("strassen", 3448, 3448, 3448, 2)["prep_bytes"]
+
+
+# ---- splits finer than any shipped table's -------------------------------------------
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+@pytest.mark.parametrize("split", [(9, 2, 2), (2, 9, 2), (2, 2, 9), (10, 11, 17), (2, 8, 2), (6, 6, 6), (7, 7, 7)])
+@pytest.mark.parametrize("scale", [5, 400])
+def test_remainders_of_fine_splits_are_all_peeled(probe, dtype, split, scale):
+    """The peeling products of one level cover C's strips once each, in pieces
+    the kernels take, and its core by one update of the whole K remainder."""
+    m, k, n = (s * scale + s - 1 for s in split)
+    if scale == 400 and split == (10, 11, 17):
+        m, k, n = (s * 40 + s - 1 for s in split)
+    launches = probe(dtype, [(m, k, n, "blocks:%dx%dx%d" % split, 1)])
+    cm, ck, cn = (v // s * s for v, s in zip((m, k, n), split))
+    seen = [[0] * n for _ in range(m)] if m * n < 200000 else None
+    area = updates = 0
+    at, fused = None, 0
+    for l in launches:
+        if l[0] == "stage":
+            fused = l[3]
+        if l[0] != "peel":
+            at = l
+            continue
+        kind, M, N, K, off, ld = l[1:]
+        assert ld == m
+        if kind == 0:
+            updates += 1
+            assert (M, N, K, off) == (cm, cn, k - ck, 0)
+            # added by the W stage up to a split its kernel is built for, else in a launch after it
+            assert (at[0] == "stage") == (split[1] <= 6)
+            continue
+        assert K == k and (M if kind == 2 else N) <= 5
+        i0, j0 = off % ld, off // ld
+        area += M * N
+        if seen is not None:
+            for i in range(i0, i0 + M):
+                for j in range(j0, j0 + N):
+                    seen[i][j] += 1
+    assert updates == (1 if k > ck else 0) and fused == (updates if split[1] <= 6 else 0)
+    assert area == m * n - cm * cn
+    if seen is not None:
+        assert all(seen[i][j] == (0 if i < cm and j < cn else 1) for i in range(m) for j in range(n))
