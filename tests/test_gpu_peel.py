@@ -1,10 +1,11 @@
 """Dynamic-peeling products at the edges of their kernels' tiles: every
 remainder of every block split the algorithms have, in each dimension.
 
-A's rows and columns inside the block split are zero except where a peeling
-product reads them, so the recursion contributes exact zeros and, on integer
-data, every element of C is an exact integer: the comparison is bit for bit,
-whatever the order of the sums."""
+A's (then B's) rows and columns inside the block split are zero, so the
+recursion contributes exact zeros and, on integer data, every element of C is
+an exact integer: the comparison is bit for bit, whatever the order of the
+sums.  With A's zeros the bottom strip runs over all of K, with B's the right
+strip does; the K update has all its data in both."""
 import os
 import subprocess
 
@@ -23,19 +24,18 @@ SPLITS = {"strassen": (2, 2, 2), "classical333_27_81": (3, 3, 3), "grey424_26_20
 def _check(fm, alg, m, k, n, dtype, alpha, beta, seed):
     sm, sk, sn = SPLITS[alg]
     rng = np.random.default_rng(seed)
-    A = rng.integers(-8, 9, (m, k)).astype(dtype)
-    B = rng.integers(-8, 9, (k, n)).astype(dtype)
-    C0 = rng.integers(-8, 9, (m, n)).astype(dtype)
-    A[:m - m % sm, :k - k % sk] = 0  # the core's products vanish
-    if n % sn:  # the right strip reads these columns of A: keep its product
-        want_r = alpha * (A.astype(np.float64) @ B[:, n - n % sn:].astype(np.float64))
-    want = alpha * (A.astype(np.float64) @ B.astype(np.float64)) + beta * C0.astype(np.float64)
     dev = lambda x: fm.col_major(torch.from_numpy(np.asfortranarray(x)).to(DEV))  # noqa: E731
-    C = fm.fastmatmul(alg, dev(A), dev(B), dev(C0), 1, alpha=alpha, beta=beta).double().cpu().numpy()
-    assert np.array_equal(C, want), (alg, m, k, n, np.argwhere(C != want)[:4])
-    if n % sn:
-        got = C[:, n - n % sn:] - beta * C0[:, n - n % sn:]
-        assert np.array_equal(got, want_r)
+    for zeros_in_a in (True, False):
+        A = rng.integers(-8, 9, (m, k)).astype(dtype)
+        B = rng.integers(-8, 9, (k, n)).astype(dtype)
+        C0 = rng.integers(-8, 9, (m, n)).astype(dtype)
+        if zeros_in_a:  # the core's products vanish
+            A[:m - m % sm, :k - k % sk] = 0
+        else:
+            B[:k - k % sk, :n - n % sn] = 0
+        want = alpha * (A.astype(np.float64) @ B.astype(np.float64)) + beta * C0.astype(np.float64)
+        C = fm.fastmatmul(alg, dev(A), dev(B), dev(C0), 1, alpha=alpha, beta=beta).double().cpu().numpy()
+        assert np.array_equal(C, want), (alg, m, k, n, zeros_in_a, np.argwhere(C != want)[:4])
 
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])

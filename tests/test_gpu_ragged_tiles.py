@@ -47,7 +47,19 @@ def _check(fm, m, k, n, dtype, off, pad, alpha=1.0, beta=0.0):
 @pytest.mark.parametrize("cfg", CFGS)
 def test_every_k_remainder(fm, cfg, dtype):
     fm.set_gemm_tile(cfg)
+    # (slices of 16: whole, partial and both parities of the loop's trips)
     for k in list(range(16, 34)) + [47, 63, 65, 97]:
+        _check(fm, 37, k, 29, dtype, 1, k % 3)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_every_k_remainder_of_the_32_deep_tile(fm, dtype):
+    """The 32 x 32 tile has slices of 32 and is the plan's choice only: every
+    remainder of its slice behind five and six of them, so that the loop's
+    body, both of its halves and the iterations before a partial slice all run."""
+    td = torch.float64 if dtype is np.float64 else torch.float32
+    for k in range(160, 224):
+        assert fm.plan_info("strassen", 37, k, 29, 0, dtype=td)["leaf"][0]["cfg"] == 35
         _check(fm, 37, k, 29, dtype, 1, k % 3)
 
 
