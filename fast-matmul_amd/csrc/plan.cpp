@@ -419,9 +419,10 @@ namespace {
 // measured on launches of 1 to 16 tiles per CU at K = 256 and 1024: us_k per
 // unit of K and k0 units of K for its start and end, whether the CU holds one
 // work group or several; and lat_k, the same for a tile that has its CU to
-// itself and waits for its own loads (the small tiles).  Whole-tile and ragged
-// products cost the same on these kernels (FP64 128 x 128: 8192 x 8192 x 4096
-// 71.7 TFLOP/s, 8190 x 8190 x 4090 70.0, 8191 x 8191 x 4091 69.7).
+// itself and waits for its own loads (the small tiles).  Launches of 2 to 16 tiles
+// a CU at these depths take 0.93 to 1.03 of what the figures say, on every tile.
+// Whole-tile and ragged products cost the same on these kernels (FP64 128 x 128:
+// 8192 x 8192 x 4096 71.7 TFLOP/s, 8190 x 8190 x 4090 70.0, 8191 x 8191 x 4091 69.7).
 // edge: the predicated kernel of the same tile, for launches the spread kernels
 // cannot take (M below a vector, K below a slice, columns past 32-bit offsets;
 // -1: not offered).  4096 x 4096 x 15, 7 products of 4096 x 4096 x 14 and 16384 x
@@ -463,7 +464,8 @@ const double kLaunchUs = 3.0;
 const double kCopyBytesPerUs = 4.9e6;
 // one work group to a CU: nothing covers its wait for operands that are not in
 // L2 (strassen one level 2048^3 FP64: 4 of 7 leaves as 256 128 x 128 tiles and
-// 3 as 64 x 64 ones 294 us, all on 64 x 64 tiles 266)
+// 3 as 64 x 64 ones 294 us, all on 64 x 64 tiles 266; one call's figure: with the
+// operands in L2 such a launch takes 0.86 to 1.0 of the figures without it)
 const double kAlonePenalty = 1.15;
 // the predicated loop's time over the spread loop's
 const double kEdgePenalty = 1.3;
@@ -1152,6 +1154,13 @@ void append_pre(std::vector<Launch>& pre, std::vector<Launch>& out, fm_dtype dt)
 // Append one problem's W stage of a level and the level's peeling products: a
 // one-level W stage adds the K remainders itself (up to the K split its kernel is
 // built for), and takes the strips into its launch where both are small.
+// The update saves a pass over C and costs W registers, most where K is split
+// six ways (smirnov363 FP64: one wave a SIMD, three without); it was faster with
+// every algorithm measured, K split 2 to 6 ways, remainders of 1 and the largest, beta
+// 0 and 0.5.  Whole call, one level, update apart -> in W: smirnov363 4320 x 4321 x
+// 4320 FP64 2170 -> 2110 us, FP32 1163 -> 1126, 9000 x 601 x 9000 2738 -> 2395 and 1497
+// -> 1345; strassen 9000 x 601 x 9000 FP64 2108 -> 1772; 900 x 901 x 900 FP64 54.3 ->
+// 47.1 (smirnov363), and the one loss, FP32 41.7 -> 42.3.
 void append_w(Launch W, std::vector<FmThinDesc> peel, std::vector<Launch>& out, fm_dtype dt) {
   std::vector<FmThinDesc> strips;
   const bool adds = W.kind == LK_W && W.alg->k <= FM_THIN_MAX + 1;
