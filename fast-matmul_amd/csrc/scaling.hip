@@ -22,6 +22,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "gmem.hpp"
 #include "scaling.hpp"
 
@@ -53,12 +55,13 @@ __device__ __forceinline__ float add_rn(float a, float b) { return __fadd_rn(a, 
 // rows and the others take further columns.  With all lanes along the rows a B of
 // 7 rows kept 2 of 256 lanes busy, and every 32 columns ended in their own atomics
 // on the same 7 maxima: whole call, strassen one level, 5 x 7 x 1000000 FP32 2300 ->
-// 462 us, FP64 1800 -> 691; 64 x 64 x 100000 354 -> 120, 303 -> 196.
+// 471 us, FP64 1800 -> 689; 64 x 64 x 100000 354 -> 124, 303 -> 194.
 constexpr int SC_THREADS = 256;
 constexpr int SC_COLS = 32;        // columns a lane takes in a row-maxima tile
 constexpr int SC_SHORT_COLS = 16;  // the same where lanes share the columns
 constexpr int SC_WCOLS = 8;        // columns a lane takes in a write tile
 constexpr int SC_SEGMENT = 8192;   // rows of a column-maxima segment (one wave)
+constexpr int ROW_LOG = 8, COL_LOG = 6;  // lr where all lanes go along the rows
 template <typename T>
 constexpr int sc_vl() {
   return 16 / (int)sizeof(T);
@@ -111,65 +114,48 @@ struct MaxArgs {
   int lr;              // lanes along the rows, as a power of two
 };
 
-// ALL: every lane along the rows, as constants (1000^3 FP32, whole call: 66 us, 83
-// with them read at run time).
-template <typename T, bool ALL>
-__device__ __forceinline__ void row_max_tile(const MaxArgs<T>& a, int t, T* red) {
+// All lanes along the rows: the layout a constant, uniform trip counts (1000^3
+// FP32, whole call: 66 us, 83 with the layout read at run time).
+template <typename T>
+__device__ __forceinline__ void row_max_tile(const MaxArgs<T>& a, int t) {
   constexpr int VL = Rows<T>::VL;
-  const int tr = t % a.tiles_r, tc = t / a.tiles_r, tid = threadIdx.x;
-  // lane r of 2^lr along the rows, g of ng column groups
-  const int lr = ALL ? 8 : a.lr, ng = SC_THREADS >> lr, r = tid & ((1 << lr) - 1), g = tid >> lr;
-  const int64_t i0 = (((int64_t)tr << lr) + r) * VL, j0 = (int64_t)tc * (ALL ? SC_COLS : SC_SHORT_COLS) * ng;
-  const int n = (int)min(a.rows - i0, (int64_t)VL);
-  if (ALL && n <= 0) return;
-  const int left = (int)min(a.cols - j0, (int64_t)(ALL ? SC_COLS : SC_SHORT_COLS) * ng);  // columns of the tile
-  const int cnt = n > 0 ? (left - g + ng - 1) / ng : 0;                                // of this lane
-  const T* p = a.X + i0 + (j0 + g) * a.ld;
-  const T* pre = a.pre + j0 + g;
+  const int tr = t % a.tiles_r, tc = t / a.tiles_r;
+  const int64_t i0 = ((int64_t)tr * SC_THREADS + (int)threadIdx.x) * VL;
+  if (i0 >= a.rows) return;
+  const int j0 = tc * SC_COLS, j1 = min(a.cols, j0 + SC_COLS), n = (int)(a.rows - i0);
   T mx[VL];
 #pragma unroll
   for (int e = 0; e < VL; ++e) mx[e] = T(0);
 #pragma unroll 8
-  for (int q = 0; q < cnt; ++q) {
+  for (int j = j0; j < j1; ++j) {
     Rows<T> x;
-    x.load(p + (int64_t)(q * ng) * a.ld, n);
-    const T f = a.pre ? pre[q * ng] : T(1);
+    x.load(a.X + i0 + (int64_t)j * a.ld, n);
+    const T f = a.pre ? a.pre[j] : T(1);
 #pragma unroll
     for (int e = 0; e < VL; ++e) mx[e] = fmax(mx[e], fabs(a.pre ? mul_rn(x.v[e], f) : x.v[e]));
-  }
-  if constexpr (!ALL) {  // the column groups' maxima meet in the first group's lanes
-#pragma unroll
-    for (int e = 0; e < VL; ++e) red[e * SC_THREADS + tid] = mx[e];
-    __syncthreads();
-    if (g > 0) return;
-    for (int q = 1; q < ng; ++q)
-#pragma unroll
-      for (int e = 0; e < VL; ++e) mx[e] = fmax(mx[e], red[e * SC_THREADS + (q << lr) + r]);
   }
 #pragma unroll
   for (int e = 0; e < VL; ++e)
     if (e < n) atomicMax(a.out + i0 + e, Bits<T>::of(mx[e]));
 }
 
-template <typename T, bool ALL>
+template <typename T>
 __device__ __forceinline__ void col_max_tile(const MaxArgs<T>& a, int t) {
   constexpr int VL = Rows<T>::VL;
-  const int tr = t % a.tiles_r, tc = t / a.tiles_r, tid = threadIdx.x;
-  // 2^lr lanes of a wave per column and segment of rows
-  const int lr = ALL ? 6 : a.lr, lane = tid & ((1 << lr) - 1);
-  const int64_t j = (int64_t)tc * (SC_THREADS >> lr) + (tid >> lr), r0 = (int64_t)tr * SC_SEGMENT;
+  const int tr = t % a.tiles_r, tc = t / a.tiles_r;
+  // one wave per column and segment of rows
+  const int j = tc * (SC_THREADS / 64) + ((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (j >= a.cols) return;
-  const int len = (int)min(a.rows - r0, (int64_t)SC_SEGMENT);
-  const T* c = a.X + r0 + j * a.ld;
-  const T* pre = a.pre + r0;
+  const int r0 = tr * SC_SEGMENT, len = min(a.rows - r0, SC_SEGMENT);
+  const T* c = a.X + (int64_t)j * a.ld;
   T mx = T(0);
 #pragma unroll 4
-  for (int i = lane * VL; i < len; i += VL << lr) {
+  for (int i = lane * VL; i < len; i += 64 * VL) {
     Rows<T> x;
-    x.load(c + i, len - i);
+    x.load(c + r0 + i, len - i);
     if (a.pre) {
       Rows<T> f;
-      f.load(pre + i, len - i);
+      f.load(a.pre + r0 + i, len - i);
 #pragma unroll
       for (int e = 0; e < VL; ++e) mx = fmax(mx, fabs(mul_rn(x.v[e], f.v[e])));
     } else {
@@ -178,34 +164,89 @@ __device__ __forceinline__ void col_max_tile(const MaxArgs<T>& a, int t) {
     }
   }
 #pragma unroll
-  for (int o = (1 << lr) >> 1; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o));
+  for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o));
   if (lane == 0) atomicMax(a.out + j, Bits<T>::of(mx));
 }
 
+// Short matrices.  Rows: lane r of 2^lr along the rows, g of ng column groups,
+// whose maxima meet in the first group's lanes.
 template <typename T>
+__device__ __forceinline__ void row_max_short(const MaxArgs<T>& a, int t, T* red) {
+  constexpr int VL = Rows<T>::VL;
+  const int tid = threadIdx.x, lr = a.lr, ng = SC_THREADS >> lr, r = tid & ((1 << lr) - 1), g = tid >> lr;
+  const int i0 = r * VL, n = a.rows - i0;  // one tile holds all rows
+  const int64_t j0 = (int64_t)t * SC_SHORT_COLS * ng + g;
+  T mx[VL];
+#pragma unroll
+  for (int e = 0; e < VL; ++e) mx[e] = T(0);
+  if (n > 0) {
+#pragma unroll 8
+    for (int q = 0; q < SC_SHORT_COLS; ++q) {
+      const int64_t j = j0 + q * ng;
+      if (j >= a.cols) break;
+      Rows<T> x;
+      x.load(a.X + i0 + j * a.ld, n);
+      const T f = a.pre ? a.pre[j] : T(1);
+#pragma unroll
+      for (int e = 0; e < VL; ++e) mx[e] = fmax(mx[e], fabs(a.pre ? mul_rn(x.v[e], f) : x.v[e]));
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < VL; ++e) red[e * SC_THREADS + tid] = mx[e];
+  __syncthreads();
+  if (g > 0) return;
+  for (int q = 1; q < ng; ++q)
+#pragma unroll
+    for (int e = 0; e < VL; ++e) mx[e] = fmax(mx[e], red[e * SC_THREADS + (q << lr) + r]);
+#pragma unroll
+  for (int e = 0; e < VL; ++e)
+    if (e < n) atomicMax(a.out + i0 + e, Bits<T>::of(mx[e]));
+}
+
+// Columns: 2^lr lanes of a wave per column, one vector each.
+template <typename T>
+__device__ __forceinline__ void col_max_short(const MaxArgs<T>& a, int t) {
+  constexpr int VL = Rows<T>::VL;
+  const int tid = threadIdx.x, lr = a.lr, i = (tid & ((1 << lr) - 1)) * VL;
+  const int64_t j = (int64_t)t * (SC_THREADS >> lr) + (tid >> lr);
+  if (j >= a.cols) return;
+  T mx = T(0);
+  if (i < a.rows) {
+    Rows<T> x, f;
+    x.load(a.X + i + j * a.ld, a.rows - i);
+    if (a.pre) f.load(a.pre + i, a.rows - i);
+#pragma unroll
+    for (int e = 0; e < VL; ++e) mx = fmax(mx, fabs(a.pre ? mul_rn(x.v[e], f.v[e]) : x.v[e]));
+  }
+  for (int o = (1 << lr) >> 1; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o));
+  if (i == 0) atomicMax(a.out + j, Bits<T>::of(mx));
+}
+
+template <typename T, bool SHORT>
 __device__ __forceinline__ void max_tile(const MaxArgs<T>& a, int t, T* red) {
   if (a.rowwise) {
-    if (a.lr == 8)
-      row_max_tile<T, true>(a, t, red);
+    if (!SHORT || a.lr == ROW_LOG)
+      row_max_tile(a, t);
     else
-      row_max_tile<T, false>(a, t, red);
+      row_max_short(a, t, red);
   } else {
-    if (a.lr == 6)
-      col_max_tile<T, true>(a, t);
+    if (!SHORT || a.lr == COL_LOG)
+      col_max_tile(a, t);
     else
-      col_max_tile<T, false>(a, t);
+      col_max_short(a, t);
   }
 }
 
-// A and B in one launch
-template <typename T>
+// A and B in one launch.  SHORT: A or B is short (1000^3 FP32, whole call: 65.8 us
+// without, 67.2 with those paths beside the others in one kernel).
+template <typename T, bool SHORT>
 __global__ void __launch_bounds__(SC_THREADS) fm_max_kernel(MaxArgs<T> a, MaxArgs<T> b) {
-  __shared__ T red[SC_THREADS * Rows<T>::VL];
+  __shared__ T red[SHORT ? SC_THREADS * Rows<T>::VL : 1];
   const int t = blockIdx.x;
   if (t < a.tiles)
-    max_tile(a, t, red);
+    max_tile<T, SHORT>(a, t, red);
   else
-    max_tile(b, t - a.tiles, red);
+    max_tile<T, SHORT>(b, t - a.tiles, red);
 }
 
 // Factor arithmetic follows the reference's types: the maxima are doubles
@@ -273,18 +314,21 @@ struct WriteArgs {
 
 // This lane's place in tile t of a write launch: its first row, its first column
 // and the distance to the next.
+template <bool ALL>
+using ColIdx = typename std::conditional<ALL, int, int64_t>::type;  // (tall: few columns fit)
 template <typename T, bool ALL>
-__device__ __forceinline__ void write_place(int t, int tiles_r, int some, int64_t* i0, int64_t* j0, int* step) {
-  const int tr = t % tiles_r, tc = t / tiles_r, tid = threadIdx.x, lr = ALL ? 8 : some;
-  *step = SC_THREADS >> lr;
-  *i0 = (((int64_t)tr << lr) + (tid & ((1 << lr) - 1))) * Rows<T>::VL;
-  *j0 = (int64_t)tc * SC_WCOLS * *step + (tid >> lr);
+__device__ __forceinline__ void write_place(int t, int tiles_r, int some, int64_t* i0, ColIdx<ALL>* j0, int* step) {
+  const int tr = t % tiles_r, tc = t / tiles_r, tid = threadIdx.x, lr = ALL ? ROW_LOG : some;
+  *step = ALL ? 1 : SC_THREADS >> lr;
+  *i0 = (((int64_t)tr << lr) + (ALL ? tid : tid & ((1 << lr) - 1))) * Rows<T>::VL;
+  *j0 = ALL ? tc * SC_WCOLS : (ColIdx<ALL>)tc * SC_WCOLS * *step + (tid >> lr);
 }
 
 template <typename T, bool ALL>
 __device__ __forceinline__ void write_tile_lanes(const WriteArgs<T>& a, int t) {
   constexpr int VL = Rows<T>::VL;
-  int64_t i0, j0;
+  int64_t i0;
+  ColIdx<ALL> j0;
   int step;
   write_place<T, ALL>(t, a.tiles_r, a.lr, &i0, &j0, &step);
   if (i0 >= a.rows) return;
@@ -294,10 +338,10 @@ __device__ __forceinline__ void write_tile_lanes(const WriteArgs<T>& a, int t) {
   Rows<T> x[SC_WCOLS];
 #pragma unroll
   for (int u = 0; u < SC_WCOLS; ++u)  // columns past the end read the last one, not stored
-    x[u].load(a.X + i0 + min(j0 + u * step, (int64_t)a.cols - 1) * a.ldx, n);
+    x[u].load(a.X + i0 + (int64_t)min(j0 + u * step, (ColIdx<ALL>)(a.cols - 1)) * a.ldx, n);
 #pragma unroll
   for (int u = 0; u < SC_WCOLS; ++u) {
-    const int64_t j = j0 + u * step;
+    const ColIdx<ALL> j = j0 + u * step;
     if (j >= a.cols) break;
     const T c = a.cf ? a.cf[j] : T(1);
 #pragma unroll
@@ -308,25 +352,25 @@ __device__ __forceinline__ void write_tile_lanes(const WriteArgs<T>& a, int t) {
       if (!a.row_first && a.rf) v = mul_rn(v, rf.v[e]);
       x[u].v[e] = v;
     }
-    x[u].store(a.Y + i0 + j * a.ldy, n);
+    x[u].store(a.Y + i0 + (int64_t)j * a.ldy, n);
   }
 }
 
-template <typename T>
+template <typename T, bool SHORT>
 __device__ __forceinline__ void write_tile(const WriteArgs<T>& a, int t) {
-  if (a.lr == 8)
+  if (!SHORT || a.lr == ROW_LOG)
     write_tile_lanes<T, true>(a, t);
   else
     write_tile_lanes<T, false>(a, t);
 }
 
-template <typename T>
+template <typename T, bool SHORT>
 __global__ void __launch_bounds__(SC_THREADS) fm_write_kernel(WriteArgs<T> a, WriteArgs<T> b) {
   const int t = blockIdx.x;
   if (t < a.tiles)
-    write_tile(a, t);
+    write_tile<T, SHORT>(a, t);
   else
-    write_tile(b, t - a.tiles);
+    write_tile<T, SHORT>(b, t - a.tiles);
 }
 
 // C[i, j] = alpha * ((P[i, j] * r[i]) * s[j]) + beta * C[i, j]; P may be C
@@ -335,7 +379,8 @@ __global__ void __launch_bounds__(SC_THREADS) fm_post_kernel(const T* P, int64_t
                                                              int rows, int cols, const T* r, const T* s,
                                                              T alpha, T beta, int tiles_r, int lr) {
   constexpr int VL = Rows<T>::VL;
-  int64_t i0, j0;
+  int64_t i0;
+  ColIdx<ALL> j0;
   int step;
   write_place<T, ALL>(blockIdx.x, tiles_r, lr, &i0, &j0, &step);
   if (i0 >= rows) return;
@@ -343,13 +388,13 @@ __global__ void __launch_bounds__(SC_THREADS) fm_post_kernel(const T* P, int64_t
   Rows<T> rf, x[SC_WCOLS];
   rf.load(r + i0, n);
 #pragma unroll
-  for (int u = 0; u < SC_WCOLS; ++u) x[u].load(P + i0 + min(j0 + u * step, (int64_t)cols - 1) * ldp, n);
+  for (int u = 0; u < SC_WCOLS; ++u) x[u].load(P + i0 + (int64_t)min(j0 + u * step, (ColIdx<ALL>)(cols - 1)) * ldp, n);
 #pragma unroll
   for (int u = 0; u < SC_WCOLS; ++u) {
-    const int64_t j = j0 + u * step;
+    const ColIdx<ALL> j = j0 + u * step;
     if (j >= cols) break;
     const T c = s[j];
-    T* out = C + i0 + j * ldc;
+    T* out = C + i0 + (int64_t)j * ldc;
     Rows<T> old;
     if (beta != T(0)) old.load(out, n);
 #pragma unroll
@@ -376,7 +421,7 @@ int row_lanes(int rows, int max_log) {
 template <typename T>
 MaxArgs<T> max_args(const T* X, int64_t ld, int rows, int cols, int rowwise, const T* pre, T* out) {
   MaxArgs<T> a{X, ld, rows, cols, rowwise, pre, reinterpret_cast<typename Bits<T>::U*>(out), 0, 0, 0};
-  a.lr = row_lanes<T>(rows, rowwise ? 8 : 6);
+  a.lr = row_lanes<T>(rows, rowwise ? ROW_LOG : COL_LOG);
   const int groups = SC_THREADS >> a.lr;
   const int64_t tile_r = rowwise ? sc_vl<T>() << a.lr : SC_SEGMENT;
   const int64_t tile_c = rowwise ? (groups > 1 ? SC_SHORT_COLS : SC_COLS) * groups : groups;
@@ -387,7 +432,7 @@ MaxArgs<T> max_args(const T* X, int64_t ld, int rows, int cols, int rowwise, con
 
 template <typename T>
 int write_tiles(int rows, int cols, int* tiles_r, int* lr) {
-  *lr = row_lanes<T>(rows, 8);
+  *lr = row_lanes<T>(rows, ROW_LOG);
   const int64_t tile_r = sc_vl<T>() << *lr, tile_c = SC_WCOLS * (SC_THREADS >> *lr);
   *tiles_r = (int)((rows + tile_r - 1) / tile_r);
   return *tiles_r * (int)((cols + tile_c - 1) / tile_c);
@@ -413,7 +458,9 @@ hipError_t run_scaling(const FmScaleArgs& a, hipStream_t st) {
     const T* pb = !second ? nullptr : out ? gb : fb;
     const MaxArgs<T> ma = max_args<T>(X, ldx, m, k, out, pa, out ? fa : ga);
     const MaxArgs<T> mb = max_args<T>(Y, ldy, k, n, !out, pb, out ? fb : gb);
-    hipLaunchKernelGGL(fm_max_kernel<T>, dim3(ma.tiles + mb.tiles), dim3(SC_THREADS), 0, st, ma, mb);
+    const bool whole = ma.lr == (ma.rowwise ? ROW_LOG : COL_LOG) && mb.lr == (mb.rowwise ? ROW_LOG : COL_LOG);
+    auto* kernel = whole ? &fm_max_kernel<T, false> : &fm_max_kernel<T, true>;
+    hipLaunchKernelGGL(kernel, dim3(ma.tiles + mb.tiles), dim3(SC_THREADS), 0, st, ma, mb);
     if (out)
       hipLaunchKernelGGL(fm_outer_factors<T>, dim3(blocks_for(m > n ? m : n)), dim3(256), 0, st, fa, r, m,
                          fb, s, n);
@@ -425,7 +472,8 @@ hipError_t run_scaling(const FmScaleArgs& a, hipStream_t st) {
     WriteArgs<T> wb{Y, ldy, B, a.ldb, k, n, rb, cb, !outer_first, 0, 0, 0};
     wa.tiles = write_tiles<T>(m, k, &wa.tiles_r, &wa.lr);
     wb.tiles = write_tiles<T>(k, n, &wb.tiles_r, &wb.lr);
-    hipLaunchKernelGGL(fm_write_kernel<T>, dim3(wa.tiles + wb.tiles), dim3(SC_THREADS), 0, st, wa, wb);
+    auto* kernel = wa.lr == ROW_LOG && wb.lr == ROW_LOG ? &fm_write_kernel<T, false> : &fm_write_kernel<T, true>;
+    hipLaunchKernelGGL(kernel, dim3(wa.tiles + wb.tiles), dim3(SC_THREADS), 0, st, wa, wb);
   };
   auto init = [&](int first) {
     hipLaunchKernelGGL(fm_scale_init<T>, dim3(blocks_for(longest)), dim3(256), 0, st, fa, r, m, fb, s, n, ga,
@@ -460,7 +508,7 @@ static void post(const void* P, int64_t ldp, void* C, int64_t ldc, int rows, int
                  const void* sv, double alpha, double beta, hipStream_t s) {
   int tiles_r, lr;
   const int tiles = write_tiles<T>(rows, cols, &tiles_r, &lr);
-  auto* kernel = lr == 8 ? &fm_post_kernel<T, true> : &fm_post_kernel<T, false>;
+  auto* kernel = lr == ROW_LOG ? &fm_post_kernel<T, true> : &fm_post_kernel<T, false>;
   hipLaunchKernelGGL(kernel, dim3(tiles), dim3(SC_THREADS), 0, s, reinterpret_cast<const T*>(P), ldp,
                      reinterpret_cast<T*>(C), ldc, rows, cols, reinterpret_cast<const T*>(r),
                      reinterpret_cast<const T*>(sv), (T)alpha, (T)beta, tiles_r, lr);
