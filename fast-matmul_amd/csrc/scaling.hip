@@ -16,7 +16,7 @@
 // products with the first pass's factors formed on the fly, and one last
 // pass multiplies by both factors, in order, and writes the copies.  A and B
 // share each launch.  A step reads each matrix three times and writes it
-// once, in 6 launches (it was 5 reads, 3 writes and 18 launches, and the row
+// once, in 6 launches (it was 5 reads, 3 writes and 17 launches, and the row
 // maxima ran on 256 work groups): strassen one level 4096^3 FP32, all of
 // the scaling 490 -> 136 us, the call 1435 -> 1109 us.
 #include <hip/hip_runtime.h>
